@@ -66,7 +66,8 @@ def pkda_qkv_conv_backward(x: Tensor, weight: Tensor, dq: Tensor, dk: Tensor, dv
     args = _args(x, weight, head_dim, norm_channels, eps)
     B, T, C = x.shape
     dx = torch.empty_like(x)
-    dw = torch.zeros_like(weight)
+    # an empty batch launches nothing and its dw is zero; otherwise the kernels write all of it
+    dw = torch.empty_like(weight) if B and T else torch.zeros_like(weight)
     ws = _lib.lib().pkda_qkv_conv_workspace(B, T, C // 3, weight.shape[1])
     part = torch.empty(max(ws, 1), device=x.device, dtype=torch.float32)
     args.dq, args.dk, args.dv = _ptr(dq), _ptr(dk), _ptr(dv)

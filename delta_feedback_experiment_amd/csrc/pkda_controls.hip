@@ -19,6 +19,7 @@
 // The two parameter gradients are per-block partials (each head's terms summed
 // over the block's rows in order) summed over blocks in a fixed order.
 #include "pkda_chunk_common.h"
+#include "pkda_reduce.h"
 
 namespace pkda {
 namespace {
@@ -198,8 +199,7 @@ extern "C" int pkda_controls_bwd(const pkda_controls_args* a, void* stream) {
     if (int st = launch_status("pkda_controls_bwd")) return st;
   }
   // part rows are [dA terms of H heads | ddt terms of H heads]
-  hipLaunchKernelGGL(sum_partials_tree_kernel, dim3(p.H), dim3(256), 0, s, a->part, blocks, 2 * p.H, a->dA_log_p);
-  hipLaunchKernelGGL(sum_partials_tree_kernel, dim3(p.H), dim3(256), 0, s, a->part + p.H, blocks, 2 * p.H,
-                     a->ddt_bias_p);
-  return launch_status("pkda_controls_bwd(reduce)");
+  return launch_column_sums(column_sum(a->part, blocks, 2 * p.H, p.H, a->dA_log_p),
+                            column_sum(a->part + p.H, blocks, 2 * p.H, p.H, a->ddt_bias_p), s,
+                            "pkda_controls_bwd(reduce)");
 }

@@ -25,6 +25,7 @@
 // 16-byte stores.  dw is summed per tile in registers and the tiles are
 // reduced in a fixed order by a second kernel: deterministic.
 #include "pkda_common.h"
+#include "pkda_reduce.h"
 
 namespace pkda {
 namespace {
@@ -43,7 +44,6 @@ constexpr int kConvTileFwd = 32;                 // tokens per workgroup, forwar
 constexpr int kConvTile = PKDA_CONV_TILE_BWD;    // tokens per workgroup, backward (and dw partials)
 constexpr int kGroup = PKDA_CONV_GROUP;          // token rows loaded together, forward
 constexpr int kGroupBwd = PKDA_CONV_GROUP_BWD;   // and backward
-constexpr int kDwSlices = 32;                    // first pass of the dw reduction
 
 struct ConvParams {
   const void* x;
@@ -414,33 +414,6 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_bwd_kernel(ConvParams p
     for (int w = 0; w < W; ++w) part[j * W + w] = dw[j][w];
 }
 
-// dw[c, w] = sum over tiles of dw_part[tile, c, w] in a fixed order, in two
-// passes: slice y sums tiles y, y + S, y + 2S, ... and leaves the sum in place
-// of tile y (only this thread ever reads that entry), then the S slice sums
-// are added in order.
-__global__ __launch_bounds__(256) void qkv_conv_dw_slices_kernel(ConvParams p, int W, int tiles, int S) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  const int y = blockIdx.y;
-  const int64_t CW = (int64_t)p.C * W;
-  if (e >= CW) return;
-  float s = 0.f;
-  for (int t = y; t < tiles; t += S) s += p.dw_part[t * CW + e];
-  p.dw_part[y * CW + e] = s;
-}
-
-__global__ __launch_bounds__(256) void qkv_conv_dw_kernel(ConvParams p, int W, int S) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  const int64_t CW = (int64_t)p.C * W;
-  if (e >= CW) return;
-  float s = 0.f;
-  for (int y = 0; y < S; ++y) s += p.dw_part[y * CW + e];
-  if (p.w_dtype == PKDA_BF16) {
-    static_cast<bf16_t*>(p.dw)[e] = f32_to_bf16(s);
-  } else {
-    static_cast<float*>(p.dw)[e] = s;
-  }
-}
-
 // ---------------------------------------------------------------------------
 // decode tokens: rows of one token, each continuing its slot's history.  A
 // thread owns 8 channels of kTokRows rows: it loads its weights once, and
@@ -570,12 +543,8 @@ int launch_conv(const ConvParams& p, bool backward, hipStream_t s) {
   const int tiles = p.B * p.tiles_per_row;
   hipLaunchKernelGGL((qkv_conv_bwd_kernel<T, W, G>), dim3(tiles, cblocks), dim3(kConvThreads), 0, s, p);
   if (int st = launch_status("pkda_qkv_conv_bwd")) return st;
-  const int S = min(kDwSlices, tiles);
-  const int eblocks = (p.C * W + 255) / 256;
-  hipLaunchKernelGGL(qkv_conv_dw_slices_kernel, dim3(eblocks, S), dim3(256), 0, s, p, W, tiles, S);
-  if (int st = launch_status("pkda_qkv_conv_bwd(dw slices)")) return st;
-  hipLaunchKernelGGL(qkv_conv_dw_kernel, dim3(eblocks), dim3(256), 0, s, p, W, S);
-  return launch_status("pkda_qkv_conv_bwd(dw)");
+  return launch_column_sums(column_sum(p.dw_part, tiles, p.C * W, p.C * W, p.dw, p.w_dtype), {}, s,
+                            "pkda_qkv_conv_bwd(dw)");
 }
 
 template <typename T, int G>

@@ -9,6 +9,7 @@
 #include <mutex>
 
 #include "pkda_chunk_common.h"
+#include "pkda_reduce.h"
 
 namespace pkda {
 namespace {
@@ -741,9 +742,8 @@ int gate_bwd_impl(const pkda_gate_args* a, float* dA_part, float* ddt_part, hipS
   }
   if (raw) {
     const int nH = a->heads, nHK = a->heads * a->head_dim;
-    hipLaunchKernelGGL(sum_partials_tree_kernel, dim3(nH), dim3(256), 0, s, dA_part, a->num_chunks, nH, a->dA_log);
-    hipLaunchKernelGGL(sum_partials_tree_kernel, dim3(nHK), dim3(256), 0, s, ddt_part, a->num_chunks, nHK,
-                       a->ddt_bias);
+    return launch_column_sums(column_sum(ddt_part, a->num_chunks, nHK, nHK, a->ddt_bias),
+                              column_sum(dA_part, a->num_chunks, nH, nH, a->dA_log), s, "pkda_gate_bwd(reduce)");
   }
   return launch_status("pkda_gate_bwd");
 }

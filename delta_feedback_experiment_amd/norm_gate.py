@@ -58,7 +58,8 @@ def pkda_norm_gate_backward(x: Tensor, gate: Tensor, weight: Tensor, rstd: Tenso
     gate, dy = gate.to(x.dtype).contiguous(), dy.to(x.dtype).contiguous()
     args = _args(x, gate, weight, eps)
     dx, dgate = torch.empty_like(x), torch.empty_like(x)
-    dw = torch.zeros_like(weight)
+    # no rows launch nothing and their dweight is zero; otherwise the kernels write all of it
+    dw = torch.empty_like(weight) if args.rows else torch.zeros_like(weight)
     ws = _lib.lib().pkda_norm_gate_workspace(args.rows, args.dim)
     part = torch.empty(max(ws, 1), device=x.device, dtype=torch.float32)
     args.x, args.gate, args.weight, args.rstd, args.dy = _ptr(x), _ptr(gate), _ptr(weight), _ptr(rstd), _ptr(dy)
@@ -79,9 +80,12 @@ def _setup_context(ctx, inputs, output) -> None:
     ctx.save_for_backward(x, gate, weight, rstd)
     ctx.eps = eps
     ctx.mark_non_differentiable(rstd)
+    ctx.set_materialize_grads(False)  # rstd has no gradient: fill no zeros for it
 
 
 def _backward(ctx, dy, _drstd):
+    if dy is None:
+        return None, None, None, None
     x, gate, weight, rstd = ctx.saved_tensors
     dx, dgate, dw = pkda_norm_gate_backward(x, gate, weight, rstd, dy, ctx.eps)
     return dx, dgate, dw, None

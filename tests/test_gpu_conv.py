@@ -100,3 +100,17 @@ def test_conv_screen_geometry_full_size(dev):
     errs = run_case(dev, 8, 4096, 8, 128, 4, torch.bfloat16, seed=21)
     print("  " + " ".join(f"{n}={e:.2e}" for n, e in errs.items()), flush=True)
     assert all(e < BF16_TOL for e in errs.values()), errs
+
+
+@pytest.mark.parametrize("B,T,H,d,W", [
+    (1, 1, 1, 32, 1),     # 96 columns of one partial
+    (37, 2, 1, 32, 3),    # 288 columns, 37 partials: more than the slots of a workgroup
+    (3, 65, 6, 128, 1),   # 2,304 columns, 6 partials
+    (300, 1, 8, 128, 4),  # 12,288 columns, 300 partials
+])
+def test_conv_weight_gradient_sums(dev, B, T, H, d, W):
+    """dw's partials over every width of the column sums, fewer and more of
+    them than a workgroup has slots; FP32, so the FP32 bar holds the sums."""
+    print(f"[gpu] qkv conv dw sums B={B} T={T} H={H} d={d} W={W}", flush=True)
+    errs = run_case(dev, B, T, H, d, W, torch.float32, seed=B + W)
+    assert all(e < FP32_TOL for e in errs.values()), errs

@@ -61,6 +61,17 @@ __device__ __forceinline__ float log_fast(float x) { return __builtin_amdgcn_log
 // a / b as a * (1 / b) on the hardware reciprocal (v_rcp_f32, 1 ulp).
 __device__ __forceinline__ float div_fast(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
 
+// 1 / d for d >= 1: the hardware reciprocal and one Newton step, within an ulp
+// as a division is, in five operations instead of eleven.  Infinity and NaN
+// (and d past 2^126, whose reciprocal is not a normal number) keep the
+// hardware's own result, 0 or NaN, which the step would turn into NaN.
+__device__ __forceinline__ float recip_from_one(float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float n = __builtin_fmaf(r, __builtin_fmaf(-d, r, 1.f), r);
+  return d < 0x1p126f ? n : r;
+}
+__device__ __forceinline__ float sigmoid_fast(float a) { return recip_from_one(1.f + __expf(-a)); }
+
 template <typename T> struct io;
 template <> struct io<float> {
   static constexpr int dtype = PKDA_F32;
@@ -150,6 +161,15 @@ __device__ __forceinline__ float lane_group_sum(float v) {
   if constexpr (N == 16)
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, false));  // row mirror
   return v;
+}
+
+// The same over 32 lanes: the rows of 16 summed as above, then the two rows of
+// each half wave (v_permlane16_swap leaves rows 0, 0, 2, 2 of the value in one
+// register and rows 1, 1, 3, 3 in the other).
+__device__ __forceinline__ float lane_half_sum(float v) {
+  v = lane_group_sum<16>(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
 }  // namespace pkda

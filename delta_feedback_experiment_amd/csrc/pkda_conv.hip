@@ -15,35 +15,52 @@
 // all in FP32, cast once to the output dtype; channels [0, P), [P, 2P),
 // [2P, 3P) leave as the three slabs q, k, v [B, T, P].
 //
-// Layout and threads: one thread owns 8 consecutive channels (one 16-byte
-// vector of a token row) and walks a tile of tokens with the W - 1 previous
-// rows in registers, so each row of x is read once (plus a W - 1 row halo per
-// tile) with fully coalesced 16-byte loads; the head's sum of squares is a
-// shuffle reduction over the head_dim / 8 lanes that share the head.  The
-// backward recomputes a and y for its tile plus the W - 1 rows after it (the
-// rows whose gradient reaches the tile's x), and writes dx with the same
-// 16-byte stores.  dw is summed per tile in registers and the tiles are
-// reduced in a fixed order by a second kernel: deterministic.
+// Layout and threads: one thread owns 4 consecutive channels (8 bytes of a
+// BF16 token row, 512 bytes a wave) and walks a tile of tokens with the W - 1
+// previous rows in registers, so each row of x is read once (plus a W - 1 row
+// halo per tile) with fully coalesced loads, a group of four rows ahead of the
+// one computed; whole groups run without a row test, so the windows slide by
+// renaming and not by register moves.  The head's sum of squares is a DPP
+// reduction over the head_dim / 4 lanes that share the head.  The backward
+// recomputes a and y for its tile plus the W - 1 rows after it (the rows whose
+// gradient reaches the tile's x).  dw is summed per tile in registers and the
+// tiles in a fixed order by a second kernel: deterministic.
+//
+// Bounds: HBM, with the VALU close behind (85 operations a thread and row
+// forward, 125 backward).  B8 T4096, 3 x 1,024 channels, W = 4, BF16: forward
+// 83 us for 403 MB (4.9 TB/s, the card's copy rate 5.2), backward 146 for 604
+// MB and 25 of dw partials (4.3 TB/s, 112 VGPRs, four waves a SIMD).  Eight
+// channels a thread, row tests and IEEE divisions in the sigmoids took 109
+// and 184 (227 VGPRs, two waves); eight channels in today's form 80 and 190,
+// but 15.4 us against 13.3 on 3 rows of 1,000 tokens.
 #include "pkda_common.h"
 #include "pkda_reduce.h"
+
+#include <type_traits>
 
 namespace pkda {
 namespace {
 
-constexpr int kConvThreads = 128;  // 128 x 8 = 1024 channels per workgroup
-#ifndef PKDA_CONV_TILE_BWD
-#define PKDA_CONV_TILE_BWD 64
-#endif
-#ifndef PKDA_CONV_GROUP
-#define PKDA_CONV_GROUP 4
-#endif
-#ifndef PKDA_CONV_GROUP_BWD
-#define PKDA_CONV_GROUP_BWD 4
-#endif
-constexpr int kConvTileFwd = 32;                 // tokens per workgroup, forward (swept: 16..64)
-constexpr int kConvTile = PKDA_CONV_TILE_BWD;    // tokens per workgroup, backward (and dw partials)
-constexpr int kGroup = PKDA_CONV_GROUP;          // token rows loaded together, forward
-constexpr int kGroupBwd = PKDA_CONV_GROUP_BWD;   // and backward
+constexpr int kConvThreads = 128;
+constexpr int kCh = 4;          // channels of a thread
+constexpr int kGroup = 4;       // token rows loaded together
+constexpr int kTileFwd = 32;    // longest tiles, tokens
+constexpr int kTileBwd = 64;
+constexpr int kTokRows = 1;     // decode tokens of a thread
+constexpr int kFillWaves = 4096;  // four waves on every SIMD
+
+// Tokens of a workgroup's tile: the longest of long_tile, long_tile / 2 and
+// long_tile / 4 whose waves fill the chip, else the last.  A long tile reads
+// and recomputes fewer halo rows, a short one puts more waves on a small
+// call: 3 rows of 1,000 tokens, 3,072 channels, go 13.3 us forward (tile 8)
+// against 14.0 (tile 16), 21.8 backward (tile 16) against 26.8 (tile 32);
+// 8 rows of 4,096 take the long tiles, 83 and 146 us, 1 to 4 % faster than half.
+inline int conv_tile(int B, int T, int C, int long_tile) {
+  const int64_t waves = (C + 64 * kCh - 1) / (64 * kCh);
+  int tile = long_tile;
+  while (tile > long_tile / 4 && waves * B * ((T + tile - 1) / tile) < kFillWaves) tile /= 2;
+  return tile;
+}
 
 struct ConvParams {
   const void* x;
@@ -63,83 +80,78 @@ struct ConvParams {
   void* hist_out;        // [pool, W - 1, C] or null
   int B, T, C, P, head_dim, norm_channels, x_dtype;
   float eps;
-  int tiles_per_row;
+  int tile, tiles_per_row;
 };
 
-template <typename T> struct Vec8;
-template <> struct Vec8<bf16_t> {
-  __device__ __forceinline__ static void load(const bf16_t* p, float* x) {
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+// CH elements kept as raw 16-byte pieces or one 8-byte piece (unpacked when
+// used), so a prefetched row costs a register for each two BF16 elements.
+template <typename T, int CH>
+struct RawRow {
+  static constexpr int N = CH * (int)sizeof(T) / 4;  // 32-bit words
+  static_assert(N == 2 || N % 4 == 0, "8 bytes or whole 16-byte pieces");
+  uint32_t r[N];
+  __device__ __forceinline__ void load(const T* p) {
+    if constexpr (N == 2) {
+      const uint2 v = *reinterpret_cast<const uint2*>(p);
+      r[0] = v.x; r[1] = v.y;
+    } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      x[2 * i] = __uint_as_float(w[i] << 16);
-      x[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+      for (int i = 0; i < N / 4; ++i) {
+        const uint4 v = reinterpret_cast<const uint4*>(p)[i];
+        r[4 * i] = v.x; r[4 * i + 1] = v.y; r[4 * i + 2] = v.z; r[4 * i + 3] = v.w;
+      }
     }
   }
-  __device__ __forceinline__ static void store(bf16_t* p, const float* x) {
-    uint32_t w[4];
+  __device__ __forceinline__ void store(T* p) const {
+    if constexpr (N == 2) {
+      *reinterpret_cast<uint2*>(p) = make_uint2(r[0], r[1]);
+    } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      w[i] = static_cast<uint32_t>(f32_to_bf16(x[2 * i])) | (static_cast<uint32_t>(f32_to_bf16(x[2 * i + 1])) << 16);
-    *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
-  }
-};
-template <> struct Vec8<float> {
-  __device__ __forceinline__ static void load(const float* p, float* x) {
-    const float4 a = *reinterpret_cast<const float4*>(p);
-    const float4 b = *reinterpret_cast<const float4*>(p + 4);
-    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
-    x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
-  }
-  __device__ __forceinline__ static void store(float* p, const float* x) {
-    *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]);
-    *reinterpret_cast<float4*>(p + 4) = make_float4(x[4], x[5], x[6], x[7]);
-  }
-};
-
-// Eight elements kept as raw 16-byte pieces (unpacked when used), so a
-// prefetched row costs 4 registers in BF16.
-template <typename T>
-struct Raw8 {
-  static constexpr int N = 8 * sizeof(T) / 16;
-  uint4 r[N];
-  __device__ __forceinline__ void load(const T* p) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) r[i] = reinterpret_cast<const uint4*>(p)[i];
+      for (int i = 0; i < N / 4; ++i)
+        reinterpret_cast<uint4*>(p)[i] = make_uint4(r[4 * i], r[4 * i + 1], r[4 * i + 2], r[4 * i + 3]);
+    }
   }
   __device__ __forceinline__ void unpack(float* x) const {
     if constexpr (sizeof(T) == 2) {
-      const uint32_t w[4] = {r[0].x, r[0].y, r[0].z, r[0].w};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        x[2 * i] = __uint_as_float(w[i] << 16);
-        x[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+      for (int i = 0; i < N; ++i) {
+        x[2 * i] = __uint_as_float(r[i] << 16);
+        x[2 * i + 1] = __uint_as_float(r[i] & 0xffff0000u);
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < N; ++i) {
-        x[4 * i] = __uint_as_float(r[i].x); x[4 * i + 1] = __uint_as_float(r[i].y);
-        x[4 * i + 2] = __uint_as_float(r[i].z); x[4 * i + 3] = __uint_as_float(r[i].w);
-      }
+      for (int i = 0; i < N; ++i) x[i] = __uint_as_float(r[i]);
     }
   }
+  __device__ __forceinline__ void pack(const float* x) {
+    if constexpr (sizeof(T) == 2) {
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        r[i] = static_cast<uint32_t>(f32_to_bf16(x[2 * i])) | (static_cast<uint32_t>(f32_to_bf16(x[2 * i + 1])) << 16);
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) r[i] = __float_as_uint(x[i]);
+    }
+  }
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int i = 0; i < N; ++i) r[i] = 0u;
+  }
 };
+template <typename T, int CH>
+__device__ __forceinline__ void store_row(T* p, const float* x) {
+  RawRow<T, CH> v;
+  v.pack(x);
+  v.store(p);
+}
 
 // Sum over the G lanes of one head (G a power of two, lanes aligned to G;
 // the lanes of a head are active together).
 template <int G>
 __device__ __forceinline__ float head_sum(float x) {
-  if constexpr (G <= 16) {
-    return lane_group_sum<G>(x);
-  } else {
-#pragma unroll
-    for (int off = 1; off < G; off <<= 1) x += __shfl_xor(x, off);
-    return x;
-  }
+  if constexpr (G <= 16) return lane_group_sum<G>(x);
+  else return lane_half_sum(x);
 }
-
-__device__ __forceinline__ float sigmoid_fast(float a) { return 1.f / (1.f + __expf(-a)); }
 
 // The slab (q, k or v) and the offset inside it of channel c.
 template <typename T>
@@ -158,22 +170,22 @@ __device__ __forceinline__ const T* slab_ptr(const void* q, const void* k, const
   return base + row * P;
 }
 
-// The 8 W taps of this thread's channels are contiguous: one branch on the
+// The CH W taps of this thread's channels are contiguous: one branch on the
 // dtype (uniform) around straight-line loads, so they go out together (a
 // per-element dtype test made each load wait for the one before).
-template <int W>
-__device__ __forceinline__ void load_weights(const ConvParams& p, int c0, float (&wt)[8][W]) {
+template <int CH, int W>
+__device__ __forceinline__ void load_weights(const ConvParams& p, int c0, float (&wt)[CH][W]) {
   const int64_t base = (int64_t)c0 * W;
   if (p.w_dtype == PKDA_BF16) {
     const bf16_t* w8 = static_cast<const bf16_t*>(p.weight) + base;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < CH; ++j)
 #pragma unroll
       for (int w = 0; w < W; ++w) wt[j][w] = bf16_to_f32(w8[j * W + w]);
   } else {
     const float* w8 = static_cast<const float*>(p.weight) + base;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < CH; ++j)
 #pragma unroll
       for (int w = 0; w < W; ++w) wt[j][w] = w8[j * W + w];
   }
@@ -182,23 +194,24 @@ __device__ __forceinline__ void load_weights(const ConvParams& p, int c0, float 
 // ---------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------
-template <typename T, int W, int G>
+template <typename T, int W, int D>
 __global__ __launch_bounds__(kConvThreads) void qkv_conv_fwd_kernel(ConvParams p) {
-  const int tpr = (p.T + kConvTileFwd - 1) / kConvTileFwd;
+  constexpr int CH = kCh, G = D / CH;
+  const int tpr = p.tiles_per_row;
   const int b = blockIdx.x / tpr;
-  const int t0 = (blockIdx.x - b * tpr) * kConvTileFwd;
-  const int t1 = min(t0 + kConvTileFwd, p.T);
-  const int c0 = (blockIdx.y * kConvThreads + threadIdx.x) * 8;
+  const int t0 = (blockIdx.x - b * tpr) * p.tile;
+  const int t1 = min(t0 + p.tile, p.T);
+  const int c0 = (blockIdx.y * kConvThreads + threadIdx.x) * CH;
   if (c0 >= p.C) return;  // whole heads: the lanes of one head leave together
   const bool norm = c0 < p.norm_channels;
-  float wt[8][W];
-  load_weights<W>(p, c0, wt);
+  float wt[CH][W];
+  load_weights<CH, W>(p, c0, wt);
   const T* xs = static_cast<const T*>(p.x) + (int64_t)b * p.T * p.C + c0;
-  float hist[W > 1 ? W - 1 : 1][8];  // x at t - (W - 1) .. t - 1
+  float hist[W > 1 ? W - 1 : 1][CH];  // x at t - (W - 1) .. t - 1
   {
     // the halo rows load unconditionally (row 0 stands in before the row's
     // start) and are replaced below where t < 0, so no branch holds them back
-    Raw8<T> hr[W > 1 ? W - 1 : 1];
+    RawRow<T, CH> hr[W > 1 ? W - 1 : 1];
 #pragma unroll
     for (int w = 0; w < W - 1; ++w) hr[w].load(xs + (int64_t)max(t0 - (W - 1) + w, 0) * p.C);
 #pragma unroll
@@ -208,10 +221,12 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_fwd_kernel(ConvParams p
         hr[w].unpack(hist[w]);
       } else if (p.hist_in) {  // the row's cached projections before its first token
         const int64_t sb = p.slot ? p.slot[b] : b;
-        Vec8<T>::load(static_cast<const T*>(p.hist_in) + (sb * (W - 1) + (W - 1) + t) * p.C + c0, hist[w]);
+        RawRow<T, CH> h;
+        h.load(static_cast<const T*>(p.hist_in) + (sb * (W - 1) + (W - 1) + t) * p.C + c0);
+        h.unpack(hist[w]);
       } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) hist[w][j] = 0.f;
+        for (int j = 0; j < CH; ++j) hist[w][j] = 0.f;
       }
     }
   }
@@ -219,46 +234,50 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_fwd_kernel(ConvParams p
   T* out = slab_ptr<T>(p.q, p.k, p.v, p.P, c0, (int64_t)b * p.T, off) + off;
   // tokens in groups of kGroup rows, the next group's loads in flight while
   // the current one computes
-  Raw8<T> xa[kGroup], xb[kGroup];
-  auto load_group = [&](int tg, Raw8<T> (&dst)[kGroup]) {  // rows past the tile clamp (never used)
+  using Row = RawRow<T, CH>;
+  Row xa[kGroup], xb[kGroup];
+  auto load_group = [&](int tg, Row (&dst)[kGroup]) {  // rows past the tile clamp (never used)
 #pragma unroll
     for (int i = 0; i < kGroup; ++i) dst[i].load(xs + (int64_t)min(tg + i, t1 - 1) * p.C);
   };
-  load_group(t0, xa);
-  for (int tg = t0; tg < t1; tg += kGroup) {
-    if (tg + kGroup < t1) load_group(tg + kGroup, xb);
+  auto step = [&](int t, const Row& xr) {
+    float xt[CH], y[CH];
+    xr.unpack(xt);
+    float ss = 0.f;
 #pragma unroll
-    for (int i = 0; i < kGroup; ++i) {
-      if (tg + i >= t1) break;
-      float xt[8];
-      xa[i].unpack(xt);
-      float y[8];
-      float ss = 0.f;
+    for (int j = 0; j < CH; ++j) {
+      float a = wt[j][W - 1] * xt[j];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float a = wt[j][W - 1] * xt[j];
-#pragma unroll
-        for (int w = 0; w < W - 1; ++w) a += wt[j][w] * hist[w][j];
-        y[j] = a * sigmoid_fast(a);
-        ss += y[j] * y[j];
-      }
-      if (norm) {
-        const float r = rsqrtf(head_sum<G>(ss) + p.eps);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) y[j] *= r;
-      }
-      Vec8<T>::store(out + (int64_t)(tg + i) * p.P, y);
-#pragma unroll
-      for (int w = 0; w + 1 < W - 1; ++w)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) hist[w][j] = hist[w + 1][j];
-      if (W > 1)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) hist[W > 1 ? W - 2 : 0][j] = xt[j];
+      for (int w = 0; w < W - 1; ++w) a += wt[j][w] * hist[w][j];
+      y[j] = a * sigmoid_fast(a);
+      ss += y[j] * y[j];
     }
+    if (norm) {
+      const float r = rsqrtf(head_sum<G>(ss) + p.eps);
+#pragma unroll
+      for (int j = 0; j < CH; ++j) y[j] *= r;
+    }
+    store_row<T, CH>(out + (int64_t)t * p.P, y);
+#pragma unroll
+    for (int w = 0; w + 1 < W - 1; ++w)
+#pragma unroll
+      for (int j = 0; j < CH; ++j) hist[w][j] = hist[w + 1][j];
+    if (W > 1)
+#pragma unroll
+      for (int j = 0; j < CH; ++j) hist[W > 1 ? W - 2 : 0][j] = xt[j];
+  };
+  load_group(t0, xa);
+  int tg = t0;
+  for (; tg + kGroup <= t1; tg += kGroup) {  // whole groups: no row test
+    load_group(tg + kGroup, xb);
+#pragma unroll
+    for (int i = 0; i < kGroup; ++i) step(tg + i, xa[i]);
 #pragma unroll
     for (int i = 0; i < kGroup; ++i) xa[i] = xb[i];
   }
+#pragma unroll
+  for (int i = 0; i + 1 < kGroup; ++i)  // a row's last, partial group
+    if (tg + i < t1) step(tg + i, xa[i]);
   // a row that is one tile (a decode token, a short prompt) leaves its
   // history here: hist holds its last W - 1 rows of history ++ x, and this
   // thread read its slot's old history at the start (in place is safe)
@@ -266,7 +285,7 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_fwd_kernel(ConvParams p
     if (p.hist_out && tpr == 1) {
       const int64_t sb = p.slot ? p.slot[b] : b;
 #pragma unroll
-      for (int w = 0; w < W - 1; ++w) Vec8<T>::store(static_cast<T*>(p.hist_out) + (sb * (W - 1) + w) * p.C + c0, hist[w]);
+      for (int w = 0; w < W - 1; ++w) store_row<T, CH>(static_cast<T*>(p.hist_out) + (sb * (W - 1) + w) * p.C + c0, hist[w]);
     }
   }
 }
@@ -277,35 +296,36 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_fwd_kernel(ConvParams p
 //   da = dy silu'(a),  silu'(a) = s (1 + a (1 - s)),  s = sigmoid(a)
 //   dx[t] = sum_w weight[w] da[t + W - 1 - w],  dw[w] += da[t] x[t - (W - 1) + w]
 // ---------------------------------------------------------------------------
-template <typename T, int W, int G>
+template <typename T, int W, int D>
 __global__ __launch_bounds__(kConvThreads) void qkv_conv_bwd_kernel(ConvParams p) {
+  constexpr int CH = kCh, G = D / CH;
   const int b = blockIdx.x / p.tiles_per_row;
   const int tile = blockIdx.x;
-  const int t0 = (blockIdx.x - b * p.tiles_per_row) * kConvTile;
-  const int t1 = min(t0 + kConvTile, p.T);
-  const int c0 = (blockIdx.y * kConvThreads + threadIdx.x) * 8;
+  const int t0 = (blockIdx.x - b * p.tiles_per_row) * p.tile;
+  const int t1 = min(t0 + p.tile, p.T);
+  const int c0 = (blockIdx.y * kConvThreads + threadIdx.x) * CH;
   if (c0 >= p.C) return;
   const bool norm = c0 < p.norm_channels;
-  float wt[8][W];
-  load_weights<W>(p, c0, wt);
+  float wt[CH][W];
+  load_weights<CH, W>(p, c0, wt);
   const T* xs = static_cast<const T*>(p.x) + (int64_t)b * p.T * p.C + c0;
   int off;
   const T* dn_base = slab_ptr<T>(p.dq, p.dk, p.dv, p.P, c0, (int64_t)b * p.T, off) + off;
   T* dxs = static_cast<T*>(p.dx) + (int64_t)b * p.T * p.C + c0;
 
-  float hist[W][8];   // x at t - (W - 1) .. t (hist[W - 1] = x[t] once loaded)
-  float dwin[W][8];   // da at t - (W - 1) .. t
-  float dw[8][W];
+  float hist[W][CH];   // x at t - (W - 1) .. t (hist[W - 1] = x[t] once loaded)
+  float dwin[W][CH];   // da at t - (W - 1) .. t
+  float dw[CH][W];
 #pragma unroll
   for (int w = 0; w < W; ++w)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < CH; ++j) {
       dwin[w][j] = 0.f;
       dw[j][w] = 0.f;
     }
   {
     // halo rows unconditionally (row 0 stands in before the row's start, then zeroed)
-    Raw8<T> hr[W > 1 ? W - 1 : 1];
+    RawRow<T, CH> hr[W > 1 ? W - 1 : 1];
 #pragma unroll
     for (int w = 0; w < W - 1; ++w) hr[w].load(xs + (int64_t)max(t0 - (W - 1) + w, 0) * p.C);
 #pragma unroll
@@ -313,126 +333,139 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_bwd_kernel(ConvParams p
       hr[w].unpack(hist[w]);
       if (t0 - (W - 1) + w < 0)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) hist[w][j] = 0.f;
+        for (int j = 0; j < CH; ++j) hist[w][j] = 0.f;
     }
   }
-  const int tend = t1 + W - 1;  // da of the W - 1 rows after the tile reaches its dx
-  Raw8<T> xa[kGroupBwd], xb[kGroupBwd], na[kGroupBwd], nb[kGroupBwd];
-  const int tlast = min(tend, p.T);
-  auto load_group = [&](int tg, Raw8<T> (&dx_)[kGroupBwd], Raw8<T> (&dn_)[kGroupBwd]) {
-    // rows past the last clamp (never used): no branch holds a load back
+  using Row = RawRow<T, CH>;
+  Row xa[kGroup], xb[kGroup], na[kGroup], nb[kGroup];
+  auto load_group = [&](int tg, Row (&dx_)[kGroup], Row (&dn_)[kGroup]) {
+    // rows past the row's end clamp (never used): no branch holds a load back
 #pragma unroll
-    for (int i = 0; i < kGroupBwd; ++i) {
-      const int t = min(tg + i, tlast - 1);
+    for (int i = 0; i < kGroup; ++i) {
+      const int t = min(tg + i, p.T - 1);
       dx_[i].load(xs + (int64_t)t * p.C);
       dn_[i].load(dn_base + (int64_t)t * p.P);
     }
   };
-  load_group(t0, xa, na);
-  for (int tg = t0; tg < tend; tg += kGroupBwd) {
-    if (tg + kGroupBwd < tlast) load_group(tg + kGroupBwd, xb, nb);
+  // row t: its da (zero when not LIVE, past the row's end), its share of dw
+  // when it is the tile's own, and dx of row t - (W - 1), whose da are then
+  // all known
+  auto step = [&](auto live, auto own, int t, const Row& xr, const Row& nr) {
+    float da[CH];
+    if constexpr (decltype(live)::value) {
+      xr.unpack(hist[W - 1]);
+      float dn[CH];
+      nr.unpack(dn);
+      float y[CH], slope[CH];  // silu(a) and silu'(a) = s + y (1 - s)
+      float ss = 0.f;
 #pragma unroll
-    for (int i = 0; i < kGroupBwd; ++i) {
-      const int t = tg + i;
-      if (t >= tend) break;
-      float da[8];
-      if (t < p.T) {
-        xa[i].unpack(hist[W - 1]);
-        float dn[8];
-        na[i].unpack(dn);
-        float a[8], y[8];
-        float ss = 0.f;
+      for (int j = 0; j < CH; ++j) {
+        float a = wt[j][0] * hist[0][j];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          a[j] = 0.f;
-#pragma unroll
-          for (int w = 0; w < W; ++w) a[j] += wt[j][w] * hist[w][j];
-          y[j] = a[j] * sigmoid_fast(a[j]);
-          ss += y[j] * y[j];
-        }
-        float dy[8];
-        if (norm) {
-          const float r = rsqrtf(head_sum<G>(ss) + p.eps);
-          float nd = 0.f;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) nd += y[j] * r * dn[j];
-          nd = head_sum<G>(nd);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) dy[j] = r * (dn[j] - y[j] * r * nd);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) dy[j] = dn[j];
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float s = sigmoid_fast(a[j]);
-          da[j] = dy[j] * s * (1.f + a[j] * (1.f - s));
-        }
-        if (t < t1) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int w = 0; w < W; ++w) dw[j][w] += da[j] * hist[w][j];
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) da[j] = 0.f;
+        for (int w = 1; w < W; ++w) a += wt[j][w] * hist[w][j];
+        const float sg = sigmoid_fast(a);
+        y[j] = a * sg;
+        slope[j] = sg + y[j] * (1.f - sg);
+        ss += y[j] * y[j];
       }
-      // slide the windows: dwin holds da[t - (W - 1) .. t]
+      if (norm) {
+        // dy = r (dn - n nd) with n = y r, nd = sum n dn = r sum y dn
+        const float r = rsqrtf(head_sum<G>(ss) + p.eps);
+        float yd = 0.f;
 #pragma unroll
-      for (int w = 0; w + 1 < W; ++w)
+        for (int j = 0; j < CH; ++j) yd += y[j] * dn[j];
+        const float f = r * r * (r * head_sum<G>(yd));
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          dwin[w][j] = dwin[w + 1][j];
-          hist[w][j] = hist[w + 1][j];
-        }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) dwin[W - 1][j] = da[j];
-      const int s = t - (W - 1);  // every da that reaches x[s] is known now
-      if (s >= t0) {
-        float dx[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          float acc = 0.f;
-#pragma unroll
-          for (int w = 0; w < W; ++w) acc += wt[j][w] * dwin[W - 1 - w][j];
-          dx[j] = acc;
-        }
-        Vec8<T>::store(dxs + (int64_t)s * p.C, dx);
+        for (int j = 0; j < CH; ++j) dn[j] = r * dn[j] - y[j] * f;
       }
+#pragma unroll
+      for (int j = 0; j < CH; ++j) da[j] = dn[j] * slope[j];
+      if constexpr (decltype(own)::value) {
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+#pragma unroll
+          for (int w = 0; w < W; ++w) dw[j][w] += da[j] * hist[w][j];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < CH; ++j) da[j] = 0.f;
     }
+    // slide the windows: dwin holds da[t - (W - 1) .. t]
 #pragma unroll
-    for (int i = 0; i < kGroupBwd; ++i) {
+    for (int w = 0; w + 1 < W; ++w)
+#pragma unroll
+      for (int j = 0; j < CH; ++j) {
+        dwin[w][j] = dwin[w + 1][j];
+        hist[w][j] = hist[w + 1][j];
+      }
+#pragma unroll
+    for (int j = 0; j < CH; ++j) dwin[W - 1][j] = da[j];
+    const int s = t - (W - 1);
+    if (s >= t0) {
+      float dx[CH];
+#pragma unroll
+      for (int j = 0; j < CH; ++j) {
+        float acc = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) acc += wt[j][w] * dwin[W - 1 - w][j];
+        dx[j] = acc;
+      }
+      store_row<T, CH>(dxs + (int64_t)s * p.C, dx);
+    }
+  };
+  static_assert(W - 1 <= kGroup, "the group after the tile holds its halo rows");
+  using Yes = std::true_type;
+  using No = std::false_type;
+  load_group(t0, xa, na);
+  int tg = t0;
+  for (; tg + kGroup <= t1; tg += kGroup) {  // whole groups: no row test
+    load_group(tg + kGroup, xb, nb);
+#pragma unroll
+    for (int i = 0; i < kGroup; ++i) step(Yes{}, Yes{}, tg + i, xa[i], na[i]);
+#pragma unroll
+    for (int i = 0; i < kGroup; ++i) {
       xa[i] = xb[i];
       na[i] = nb[i];
     }
   }
+  const int rem = t1 - tg;  // a row's last, partial group: its tile ends the row
+#pragma unroll
+  for (int i = 0; i + 1 < kGroup; ++i)
+    if (i < rem) step(Yes{}, Yes{}, tg + i, xa[i], na[i]);
+  // the W - 1 rows after the tile, whose da reach its dx
+#pragma unroll
+  for (int i = 0; i < W - 1; ++i) {
+    if (t1 + i < p.T) step(Yes{}, No{}, t1 + i, xa[i], na[i]);  // rem == 0: the group holds them
+    else step(No{}, No{}, t1 + i, xa[i], na[i]);
+  }
   float* part = p.dw_part + ((int64_t)tile * p.C + c0) * W;
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
+  for (int j = 0; j < CH; ++j)
 #pragma unroll
     for (int w = 0; w < W; ++w) part[j * W + w] = dw[j][w];
 }
 
 // ---------------------------------------------------------------------------
 // decode tokens: rows of one token, each continuing its slot's history.  A
-// thread owns 8 channels of kTokRows rows: it loads its weights once, and
+// thread owns 4 channels of kTokRows rows: it loads its weights once, and
 // every row's W - 1 history rows and new projection row before computing;
 // out = the normalised silu(conv), and the slot's history shifts by one row
-// in place (each thread reads its channels' rows before writing them).
+// in place (each thread reads its channels' rows before writing them).  Bound
+// by the latency of one round of loads, so a row a thread: 256 rows of 3 x
+// 4,096 channels 10.3 us, 4 of 3 x 1,024 3.2 (two rows a thread 11.3 and 4.2;
+// eight rows of eight channels, the earlier form, 16.3 and 5.5).
 // ---------------------------------------------------------------------------
-constexpr int kTokRows = 8;
-
-template <typename T, int W, int G>
+template <typename T, int W, int D>
 __global__ __launch_bounds__(kConvThreads) void qkv_conv_token_kernel(ConvParams p) {
-  const int c0 = (blockIdx.y * kConvThreads + threadIdx.x) * 8;
+  constexpr int CH = kCh, G = D / CH;
+  const int c0 = (blockIdx.y * kConvThreads + threadIdx.x) * CH;
   if (c0 >= p.C) return;
   const bool norm = c0 < p.norm_channels;
-  float wt[8][W];
-  load_weights<W>(p, c0, wt);
+  float wt[CH][W];
+  load_weights<CH, W>(p, c0, wt);
   const int b0 = blockIdx.x * kTokRows;
   const int nb = min(kTokRows, p.B - b0);
-  Raw8<T> hr[kTokRows][W - 1], xr[kTokRows];
+  RawRow<T, CH> hr[kTokRows][W - 1], xr[kTokRows];
 #pragma unroll
   for (int r = 0; r < kTokRows; ++r) {
     if (r >= nb) break;
@@ -444,8 +477,7 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_token_kernel(ConvParams
       if (p.hist_in) {
         hr[r][w].load(static_cast<const T*>(p.hist_in) + (sb * (W - 1) + w) * p.C + c0);
       } else {
-#pragma unroll
-        for (int i = 0; i < Raw8<T>::N; ++i) hr[r][w].r[i] = make_uint4(0u, 0u, 0u, 0u);
+        hr[r][w].zero();
       }
     }
   }
@@ -454,14 +486,14 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_token_kernel(ConvParams
     if (r >= nb) break;
     const int b = b0 + r;
     const int64_t sb = p.slot ? p.slot[b] : b;
-    float xt[8], hist[W - 1][8];
+    float xt[CH], hist[W - 1][CH];
     xr[r].unpack(xt);
 #pragma unroll
     for (int w = 0; w < W - 1; ++w) hr[r][w].unpack(hist[w]);
-    float y[8];
+    float y[CH];
     float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < CH; ++j) {
       float a = wt[j][W - 1] * xt[j];
 #pragma unroll
       for (int w = 0; w < W - 1; ++w) a += wt[j][w] * hist[w][j];
@@ -471,16 +503,16 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_token_kernel(ConvParams
     if (norm) {
       const float rn = rsqrtf(head_sum<G>(ss) + p.eps);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) y[j] *= rn;
+      for (int j = 0; j < CH; ++j) y[j] *= rn;
     }
     int off;
     T* out = slab_ptr<T>(p.q, p.k, p.v, p.P, c0, (int64_t)b, off) + off;
-    Vec8<T>::store(out, y);
+    store_row<T, CH>(out, y);
     if (p.hist_out) {
       T* ho = static_cast<T*>(p.hist_out) + sb * (W - 1) * p.C + c0;
 #pragma unroll
-      for (int w = 0; w + 1 < W - 1; ++w) Vec8<T>::store(ho + (int64_t)w * p.C, hist[w + 1]);
-      Vec8<T>::store(ho + (int64_t)(W - 2) * p.C, xt);
+      for (int w = 0; w + 1 < W - 1; ++w) store_row<T, CH>(ho + (int64_t)w * p.C, hist[w + 1]);
+      store_row<T, CH>(ho + (int64_t)(W - 2) * p.C, xt);
     }
   }
 }
@@ -494,76 +526,76 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_token_kernel(ConvParams
 // ---------------------------------------------------------------------------
 template <typename T, int W>
 __global__ __launch_bounds__(kConvThreads) void qkv_conv_history_kernel(ConvParams p) {
+  constexpr int CH = kCh;
   const int b = blockIdx.x;
-  const int c0 = (blockIdx.y * kConvThreads + threadIdx.x) * 8;
+  const int c0 = (blockIdx.y * kConvThreads + threadIdx.x) * CH;
   if (c0 >= p.C) return;
   const int64_t sb = p.slot ? p.slot[b] : b;
   const T* xs = static_cast<const T*>(p.x) + (int64_t)b * p.T * p.C + c0;
-  float rows[W - 1][8];
+  RawRow<T, CH> rows[W - 1];
 #pragma unroll
   for (int j = 0; j < W - 1; ++j) {
     const int t = p.T - (W - 1) + j;  // position relative to the row's first token
     if (t >= 0) {
-      Vec8<T>::load(xs + (int64_t)t * p.C, rows[j]);
+      rows[j].load(xs + (int64_t)t * p.C);
     } else if (p.hist_in) {
-      Vec8<T>::load(static_cast<const T*>(p.hist_in) + (sb * (W - 1) + (W - 1) + t) * p.C + c0, rows[j]);
+      rows[j].load(static_cast<const T*>(p.hist_in) + (sb * (W - 1) + (W - 1) + t) * p.C + c0);
     } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) rows[j][e] = 0.f;
+      rows[j].zero();
     }
   }
 #pragma unroll
-  for (int j = 0; j < W - 1; ++j) Vec8<T>::store(static_cast<T*>(p.hist_out) + (sb * (W - 1) + j) * p.C + c0, rows[j]);
+  for (int j = 0; j < W - 1; ++j) rows[j].store(static_cast<T*>(p.hist_out) + (sb * (W - 1) + j) * p.C + c0);
 }
 
-template <typename T, int W, int G>
+template <typename T, int W, int D>
 int launch_conv(const ConvParams& p, bool backward, hipStream_t s) {
-  const int cblocks = (p.C + 8 * kConvThreads - 1) / (8 * kConvThreads);
+  constexpr int CB = kConvThreads * kCh;  // channels of a workgroup
+  const int cblocks = (p.C + CB - 1) / CB;
+  const dim3 grid(p.B * p.tiles_per_row, cblocks);
   if (!backward) {
     if constexpr (W > 1) {
       if (p.T == 1 && (p.hist_in || p.hist_out)) {  // decode tokens
-        hipLaunchKernelGGL((qkv_conv_token_kernel<T, W, G>), dim3((p.B + kTokRows - 1) / kTokRows, cblocks),
+        hipLaunchKernelGGL((qkv_conv_token_kernel<T, W, D>), dim3((p.B + kTokRows - 1) / kTokRows, cblocks),
                            dim3(kConvThreads), 0, s, p);
         return launch_status("pkda_qkv_conv_fwd(token)");
       }
     }
     if (p.T > 0) {
-      const int tiles = p.B * ((p.T + kConvTileFwd - 1) / kConvTileFwd);
-      hipLaunchKernelGGL((qkv_conv_fwd_kernel<T, W, G>), dim3(tiles, cblocks), dim3(kConvThreads), 0, s, p);
+      hipLaunchKernelGGL((qkv_conv_fwd_kernel<T, W, D>), grid, dim3(kConvThreads), 0, s, p);
       if (int st = launch_status("pkda_qkv_conv_fwd")) return st;
     }
     if constexpr (W > 1) {
-      if (p.hist_out && (p.T == 0 || p.T > kConvTileFwd)) {  // else the forward kernel wrote it
+      if (p.hist_out && p.tiles_per_row != 1) {  // else the forward kernel wrote it
         hipLaunchKernelGGL((qkv_conv_history_kernel<T, W>), dim3(p.B, cblocks), dim3(kConvThreads), 0, s, p);
         return launch_status("pkda_qkv_conv_fwd(history)");
       }
     }
     return 0;
   }
-  const int tiles = p.B * p.tiles_per_row;
-  hipLaunchKernelGGL((qkv_conv_bwd_kernel<T, W, G>), dim3(tiles, cblocks), dim3(kConvThreads), 0, s, p);
+  hipLaunchKernelGGL((qkv_conv_bwd_kernel<T, W, D>), grid, dim3(kConvThreads), 0, s, p);
   if (int st = launch_status("pkda_qkv_conv_bwd")) return st;
-  return launch_column_sums(column_sum(p.dw_part, tiles, p.C * W, p.C * W, p.dw, p.w_dtype), {}, s,
+  return launch_column_sums(column_sum(p.dw_part, p.B * p.tiles_per_row, p.C * W, p.C * W, p.dw, p.w_dtype), {}, s,
                             "pkda_qkv_conv_bwd(dw)");
 }
 
-template <typename T, int G>
+template <typename T, int D>
 int dispatch_w(const ConvParams& p, int W, bool backward, hipStream_t s) {
   switch (W) {
-    case 1: return launch_conv<T, 1, G>(p, backward, s);
-    case 2: return launch_conv<T, 2, G>(p, backward, s);
-    case 3: return launch_conv<T, 3, G>(p, backward, s);
-    case 4: return launch_conv<T, 4, G>(p, backward, s);
+    case 1: return launch_conv<T, 1, D>(p, backward, s);
+    case 2: return launch_conv<T, 2, D>(p, backward, s);
+    case 3: return launch_conv<T, 3, D>(p, backward, s);
+    case 4: return launch_conv<T, 4, D>(p, backward, s);
     default: set_error("conv_size %d not built (1..4)", W); return PKDA_EUNSUPPORTED;
   }
 }
 
 template <typename T>
 int dispatch(const ConvParams& p, int W, bool backward, hipStream_t s) {
-  switch (p.head_dim / 8) {
-    case 4: return dispatch_w<T, 4>(p, W, backward, s);
-    case 8: return dispatch_w<T, 8>(p, W, backward, s);
-    case 16: return dispatch_w<T, 16>(p, W, backward, s);
+  switch (p.head_dim) {
+    case 32: return dispatch_w<T, 32>(p, W, backward, s);
+    case 64: return dispatch_w<T, 64>(p, W, backward, s);
+    case 128: return dispatch_w<T, 128>(p, W, backward, s);
     default: set_error("head_dim %d not built (32, 64, 128)", p.head_dim); return PKDA_EUNSUPPORTED;
   }
 }
@@ -590,7 +622,8 @@ int conv_call(const pkda_qkv_conv_args* a, void* stream, bool backward) {
   p.norm_channels = a->norm_channels;
   p.x_dtype = a->dtype;
   p.eps = a->eps;
-  p.tiles_per_row = (a->seqlen + kConvTile - 1) / kConvTile;
+  p.tile = backward ? conv_tile(p.B, p.T, p.C, kTileBwd) : conv_tile(p.B, p.T, p.C, kTileFwd);
+  p.tiles_per_row = (a->seqlen + p.tile - 1) / p.tile;
   p.x = a->x;
   p.weight = a->weight;
   p.w_dtype = a->w_dtype;
@@ -623,7 +656,8 @@ int conv_call(const pkda_qkv_conv_args* a, void* stream, bool backward) {
 }  // namespace pkda
 
 extern "C" int64_t pkda_qkv_conv_workspace(int32_t batch, int32_t seqlen, int32_t width, int32_t conv_size) {
-  const int64_t tiles = (int64_t)batch * ((seqlen + pkda::kConvTile - 1) / pkda::kConvTile);
+  const int tile = pkda::conv_tile(batch, seqlen, 3 * width, pkda::kTileBwd);
+  const int64_t tiles = (int64_t)batch * ((seqlen + tile - 1) / tile);
   return tiles * 3 * (int64_t)width * conv_size;
 }
 

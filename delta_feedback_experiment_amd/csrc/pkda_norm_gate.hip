@@ -93,8 +93,6 @@ __device__ __forceinline__ float row_sum(float x) {
   }
 }
 
-__device__ __forceinline__ float sigm(float a) { return 1.f / (1.f + __expf(-a)); }
-
 // ---------------------------------------------------------------------------
 template <typename T, int D>
 __global__ __launch_bounds__(kNgThreads) void norm_gate_fwd_kernel(NgParams p) {
@@ -118,7 +116,7 @@ __global__ __launch_bounds__(kNgThreads) void norm_gate_fwd_kernel(NgParams p) {
     const float rs = rsqrtf(row_sum<L>(ss) / D + p.eps);
     float y[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) y[j] = x[j] * rs * w[j] * sigm(g[j]);
+    for (int j = 0; j < 8; ++j) y[j] = x[j] * rs * w[j] * sigmoid_fast(g[j]);
     V8<T>::store(ys + r * D + c0, y);
     if (lane_in_row == 0) p.rstd[r] = rs;
   }
@@ -153,7 +151,7 @@ __global__ __launch_bounds__(kNgThreads) void norm_gate_bwd_kernel(NgParams p) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       n[j] = x[j] * rs;
-      const float s = sigm(g[j]);
+      const float s = sigmoid_fast(g[j]);
       dg[j] = dy[j] * n[j] * w[j] * s * (1.f - s);
       const float dys_ = dy[j] * s;
       dw[j] += dys_ * n[j];

@@ -114,3 +114,45 @@ def test_conv_weight_gradient_sums(dev, B, T, H, d, W):
     print(f"[gpu] qkv conv dw sums B={B} T={T} H={H} d={d} W={W}", flush=True)
     errs = run_case(dev, B, T, H, d, W, torch.float32, seed=B + W)
     assert all(e < FP32_TOL for e in errs.values()), errs
+
+
+@pytest.mark.parametrize("B,T,H,d", [
+    (22, 1001, 8, 128),  # tiles of 32 and 64 tokens, a last tile of 9 and 41
+    (11, 1003, 8, 128),  # 32 and 32
+    (6, 998, 8, 128),    # 16 and 16: groups of four and a pair
+    (3, 33, 2, 64),      # 8 and 16: a last tile of one token
+])
+def test_conv_tiles_match_oracle(dev, B, T, H, d):
+    """Every tile length the sizes choose, forward and backward, with a last
+    tile and a last group that are not whole; FP32 at the FP32 bar (the dw
+    sums of both sides are FP32 over B T tokens)."""
+    from delta_feedback_experiment_amd import pkda_qkv_conv
+
+    print(f"[gpu] qkv conv tiles B={B} T={T} H={H} d={d}", flush=True)
+    x, w, do = (t.to(dev) if torch.is_tensor(t) else [g.to(dev) for g in t]
+                for t in make(B, T, H, d, 4, torch.float32, seed=T))
+    leaves = [x.requires_grad_(), w.requires_grad_()]
+    ref = co.qkv_conv_reference(*leaves, d, 2 * H * d, EPS)
+    out = pkda_qkv_conv(*leaves, d, 2 * H * d, EPS)
+    grads = zip(torch.autograd.grad(out, leaves, do), torch.autograd.grad(ref, leaves, do))
+    for name, (a, b) in zip(("q", "k", "v", "dx", "dw"), list(zip(out, ref)) + list(grads)):
+        assert rel_l2(a, b) < FP32_TOL, name
+
+
+def test_conv_keeps_infinities_and_nan(dev):
+    """The sigmoid's reciprocal keeps a division's results at the ends: silu
+    of a large negative input is zero, of infinities and NaN what torch's
+    a / (1 + e^-a) gives."""
+    from delta_feedback_experiment_amd import pkda_norm_gate, pkda_qkv_conv
+
+    print("[gpu] sigmoid ends", flush=True)
+    vals = torch.tensor([0.0, -80.0, -88.9, -200.0, 200.0, 3e38, -3e38, float("inf"), float("-inf"), float("nan")],
+                        device=dev)
+    x = torch.zeros(1, 1, 3 * 32, device=dev)
+    x[0, 0, 64:64 + len(vals)] = vals  # the V slab: no norm
+    v = pkda_qkv_conv(x, torch.ones(96, 1, device=dev), 32, 64, EPS)[2][0, 0, :len(vals)]
+    torch.testing.assert_close(v, vals / (1 + torch.exp(-vals)), rtol=1e-5, atol=1e-30, equal_nan=True)
+    gate = torch.zeros(1, 64, device=dev)
+    gate[0, :len(vals)] = vals
+    y = pkda_norm_gate(torch.ones(1, 64, device=dev), gate, torch.ones(64, device=dev), 0.0)[0]
+    torch.testing.assert_close(y, torch.sigmoid(gate), rtol=1e-5, atol=1e-30, equal_nan=True)

@@ -1,0 +1,109 @@
+"""Registration of this package's operators with PyTorch's dispatcher.
+
+Each operator is a schema with a device kernel, a fake implementation and,
+where it has one, an autograd formula -- what ``torch.library.custom_op``
+registers, written straight onto the dispatcher keys.  A single call of a
+decode step or a small block is mostly host time: ``custom_op``'s generic
+layers (argument trees flattened and rebuilt around the autograd function,
+schema defaults filled in, alias and disabled-kernel checks around the
+kernel) took about half of the 33 us of each operator of a decode token, and
+more for the training operator, whose outputs hold a list.
+
+The dispatcher's own order is kept: autograd, then tracing modes and
+functionalization, then the device kernel, so fake tensors, ``torch.compile``,
+saved-tensor hooks and the refusal of CPU tensors work as for any operator.
+"""
+
+from __future__ import annotations
+
+import torch
+from torch import Tensor, _C
+from torch.autograd.function import once_differentiable
+
+_LIBRARY = torch.library.Library("pkda_mi355x", "FRAGMENT")
+
+
+def device_op(schema: str):
+    """Decorator: register ``fn`` as the device kernel of ``schema`` (``name(args)
+    -> returns``) and return the operator.  Arguments the schema marks as
+    written have their version counters raised after the kernel's launches."""
+
+    def register(fn):
+        name = schema.split("(", 1)[0]
+        _LIBRARY.define(schema, tags=(torch.Tag.pt2_compliant_tag,))
+        op = getattr(torch.ops.pkda_mi355x, name).default
+        written = [i for i, a in enumerate(op._schema.arguments) if a.alias_info is not None and a.alias_info.is_write]
+
+        def mutating(*args):
+            out = fn(*args)
+            for i in written:
+                t = args[i]
+                if t is not None and not t.is_inference():
+                    torch.autograd.graph.increment_version(t)
+            return out
+
+        _LIBRARY.impl(name, mutating if written else fn, "CUDA")
+        _autograd(op, name, None, None)
+        return op
+
+    return register
+
+
+def register_fake(op, fn) -> None:
+    torch.library.register_fake(op.name(), fn, lib=_LIBRARY)
+
+
+def register_autograd(op, backward, setup_context) -> None:
+    """Give ``op`` a backward formula, ``backward(ctx, *output_grads)`` and
+    ``setup_context(ctx, inputs, output)`` as ``torch.library.register_autograd``
+    takes them (a list output's gradients come one by one, after the others)."""
+    _FORMULAS[op] = (setup_context, backward)
+
+
+_FORMULAS: dict = {}
+
+
+def _autograd(op, name: str, setup_context, backward) -> None:
+    def flat(out):
+        if isinstance(out, (tuple, list)) and out and isinstance(out[-1], list):
+            return (*out[:-1], *out[-1])
+        return out
+
+    class Operator(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, keyset, *args):
+            with _C._AutoDispatchBelowAutograd():
+                out = op.redispatch(keyset & _C._after_autograd_keyset, *args)
+            if op in _FORMULAS:
+                _FORMULAS[op][0](ctx, args, out)
+            return flat(out)
+
+        @staticmethod
+        @once_differentiable
+        def backward(ctx, *grads):
+            if op not in _FORMULAS:
+                raise RuntimeError(f"Trying to backward through {op} but no autograd formula was registered.")
+            return (None, *_FORMULAS[op][1](ctx, *grads))
+
+    Operator.__name__ = f"BackwardFor_pkda_mi355x_{name}"
+    returns = op._schema.returns
+    listed = len(returns) > 1 and isinstance(returns[-1].type, _C.ListType)
+
+    def kernel(keyset, *args):
+        if _C.is_grad_enabled() and _C._any_requires_grad(*args):
+            out = Operator.apply(keyset, *args)
+            return (*out[:len(returns) - 1], list(out[len(returns) - 1:])) if listed else out
+        with _C._AutoDispatchBelowAutograd():
+            return op.redispatch(keyset & _C._after_autograd_keyset, *args)
+
+    _LIBRARY.impl(name, kernel, "Autograd", with_keyset=True)
+
+
+def call(op, *args):
+    """``op(*args)``, past the autograd key when nothing asks for gradients:
+    the same dispatch below it, without the round trip through the autograd
+    kernel above.  (Dynamo traces the plain call.)"""
+    if torch.compiler.is_compiling() or (_C.is_grad_enabled() and _C._any_requires_grad(*args)):
+        return op(*args)
+    with _C._AutoDispatchBelowAutograd():
+        return op(*args)

@@ -19,7 +19,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from .pkda import _dtype_code, _f32, _ptr, _stream
+from .pkda import _dtype_code, _f32, _on, _ptr, _stream
 
 CHUNK_SIZE = 64
 
@@ -56,7 +56,7 @@ class ChunkPlan:
             raise ValueError("cu_seqlens needs at least one element")
         bound = -(-T // CHUNK_SIZE) + N
         table = torch.empty(4 * bound + 3 * N + 3, device=q.device, dtype=torch.int32)
-        with torch.cuda.device(q.device):
+        with _on(q.device):
             status = _lib.lib().pkda_chunk_table(
                 _ptr(cu), N, T, bound, _ptr(table), _stream(q.device)
             )
@@ -541,7 +541,7 @@ def chunk_pkda(
     if initial_state is not None and tuple(initial_state.shape) != (N, q.shape[2], D, D):
         raise ValueError(f"initial_state must be {(N, q.shape[2], D, D)}")
     opts = (use_gate_in_kernel, float(scale), output_final_state, float(x), float(eps), lean)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         o, S_T, A_T = _ChunkPKDA.apply(q, k, v, g, beta, g_atk, beta_atk, A_log, dt_bias, log_atk_scale,
                                       initial_state, initial_A_state, cu_seqlens, decay_up, opts)
     if not output_final_state:

@@ -27,8 +27,8 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
-from . import _lib
-from .pkda import _dtype_code, _f32, _ptr, _stream
+from . import _lib, _registry
+from .pkda import _dtype_code, _f32, _on, _ptr, _stream
 
 
 def _rows(packed: Tensor, width: int) -> tuple[Tensor, int, int]:
@@ -55,7 +55,8 @@ def _args(packed: Tensor, A_log_p: Tensor, dt_bias_p: Tensor, rank: int, heads: 
     return args, flat, A32, dt32, gate_width
 
 
-@torch.library.custom_op("pkda_mi355x::pkda_controls_act", mutates_args=(), device_types="cuda")
+@_registry.device_op("pkda_controls_act(Tensor packed, Tensor A_log_p, Tensor dt_bias_p, int rank, int heads) "
+                     "-> (Tensor, Tensor, Tensor)")
 def pkda_controls_act(packed: Tensor, A_log_p: Tensor, dt_bias_p: Tensor, rank: int,
                       heads: int) -> tuple[Tensor, Tensor, Tensor]:
     """``(beta, precond_decay, precond_beta)`` ``[..., H]`` of the packed controls."""
@@ -65,19 +66,21 @@ def pkda_controls_act(packed: Tensor, A_log_p: Tensor, dt_bias_p: Tensor, rank: 
     pbeta = torch.empty_like(beta)
     pdecay = torch.empty(*lead, heads, device=packed.device, dtype=torch.float32)
     args.beta, args.precond_decay, args.precond_beta = _ptr(beta), _ptr(pdecay), _ptr(pbeta)
-    with torch.cuda.device(packed.device):
+    with _on(packed.device):
         _lib.call("pkda_controls_fwd", args, _stream(packed.device))
     return beta, pdecay, pbeta
 
 
-@pkda_controls_act.register_fake
 def _pkda_controls_act_fake(packed, A_log_p, dt_bias_p, rank, heads):
     lead = packed.shape[:-1]
     beta = packed.new_empty(*lead, heads)
     return beta, packed.new_empty(*lead, heads, dtype=torch.float32), packed.new_empty(*lead, heads)
 
 
-@torch.library.custom_op("pkda_mi355x::pkda_controls_backward", mutates_args=(), device_types="cuda")
+@_registry.device_op(
+    "pkda_controls_backward(Tensor packed, Tensor A_log_p, Tensor dt_bias_p, Tensor? d_decay_hidden, Tensor? dbeta, "
+    "Tensor? dprecond_decay, Tensor? dprecond_beta, Tensor? d_gate_hidden, int rank, int heads) "
+    "-> (Tensor, Tensor, Tensor)")
 def pkda_controls_backward(packed: Tensor, A_log_p: Tensor, dt_bias_p: Tensor, d_decay_hidden: Tensor | None,
                            dbeta: Tensor | None, dprecond_decay: Tensor | None, dprecond_beta: Tensor | None,
                            d_gate_hidden: Tensor | None, rank: int, heads: int) -> tuple[Tensor, Tensor, Tensor]:
@@ -103,15 +106,18 @@ def pkda_controls_backward(packed: Tensor, A_log_p: Tensor, dt_bias_p: Tensor, d
     args.d_decay_hidden, args.dbeta, args.dprecond_decay = _ptr(dh), _ptr(db), _ptr(dpd)
     args.dprecond_beta, args.d_gate_hidden = _ptr(dpb), _ptr(dg)
     args.dpacked, args.part, args.dA_log_p, args.ddt_bias_p = _ptr(dpacked), _ptr(part), _ptr(dA), _ptr(ddt)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("pkda_controls_bwd", args, _stream(dev))
     return dpacked, dA.to(A_log_p.dtype), ddt.to(dt_bias_p.dtype)
 
 
-@pkda_controls_backward.register_fake
 def _pkda_controls_backward_fake(packed, A_log_p, dt_bias_p, d_decay_hidden, dbeta, dprecond_decay, dprecond_beta,
                                  d_gate_hidden, rank, heads):
     return packed.new_empty(packed.shape), torch.empty_like(A_log_p), torch.empty_like(dt_bias_p)
+
+
+_registry.register_fake(pkda_controls_act, _pkda_controls_act_fake)
+_registry.register_fake(pkda_controls_backward, _pkda_controls_backward_fake)
 
 
 class _Controls(torch.autograd.Function):
@@ -119,7 +125,7 @@ class _Controls(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, packed, A_log_p, dt_bias_p, rank, heads):
-        beta, pdecay, pbeta = pkda_controls_act(packed, A_log_p, dt_bias_p, rank, heads)
+        beta, pdecay, pbeta = _registry.call(pkda_controls_act, packed, A_log_p, dt_bias_p, rank, heads)
         ctx.save_for_backward(packed, A_log_p, dt_bias_p)
         ctx.geometry = (rank, heads)
         return packed[..., :rank], beta, pdecay, pbeta, packed[..., rank + 3 * heads:]

@@ -16,8 +16,8 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
-from . import _lib
-from .pkda import _dtype_code, _ptr, _stream
+from . import _lib, _registry
+from .pkda import _dtype_code, _on, _ptr, _stream
 
 
 def _args(x: Tensor, weight: Tensor, head_dim: int, norm_channels: int, eps: float) -> _lib.QkvConvArgs:
@@ -34,7 +34,8 @@ def _args(x: Tensor, weight: Tensor, head_dim: int, norm_channels: int, eps: flo
     )
 
 
-@torch.library.custom_op("pkda_mi355x::pkda_qkv_conv", mutates_args=(), device_types="cuda")
+@_registry.device_op("pkda_qkv_conv(Tensor x, Tensor weight, int head_dim, int norm_channels, float eps) "
+                     "-> (Tensor, Tensor, Tensor)")
 def pkda_qkv_conv(x: Tensor, weight: Tensor, head_dim: int, norm_channels: int,
                   eps: float) -> tuple[Tensor, Tensor, Tensor]:
     """One SiLU short convolution over concatenated Q/K/V with the per-head L2
@@ -45,18 +46,18 @@ def pkda_qkv_conv(x: Tensor, weight: Tensor, head_dim: int, norm_channels: int,
     B, T, C = x.shape
     q, k, v = (torch.empty(B, T, C // 3, device=x.device, dtype=x.dtype) for _ in range(3))
     args.q, args.k, args.v = _ptr(q), _ptr(k), _ptr(v)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.call("pkda_qkv_conv_fwd", args, _stream(x.device))
     return q, k, v
 
 
-@pkda_qkv_conv.register_fake
 def _pkda_qkv_conv_fake(x, weight, head_dim, norm_channels, eps):
     B, T, C = x.shape
     return tuple(x.new_empty(B, T, C // 3) for _ in range(3))
 
 
-@torch.library.custom_op("pkda_mi355x::pkda_qkv_conv_backward", mutates_args=(), device_types="cuda")
+@_registry.device_op("pkda_qkv_conv_backward(Tensor x, Tensor weight, Tensor dq, Tensor dk, Tensor dv, int head_dim, "
+                     "int norm_channels, float eps) -> (Tensor, Tensor)")
 def pkda_qkv_conv_backward(x: Tensor, weight: Tensor, dq: Tensor, dk: Tensor, dv: Tensor, head_dim: int,
                            norm_channels: int, eps: float) -> tuple[Tensor, Tensor]:
     """``(dx, dw)`` of :func:`pkda_qkv_conv` (fla_ops.py:181-215).  ``dw`` is a
@@ -72,12 +73,11 @@ def pkda_qkv_conv_backward(x: Tensor, weight: Tensor, dq: Tensor, dk: Tensor, dv
     part = torch.empty(max(ws, 1), device=x.device, dtype=torch.float32)
     args.dq, args.dk, args.dv = _ptr(dq), _ptr(dk), _ptr(dv)
     args.dx, args.dw, args.dw_part = _ptr(dx), _ptr(dw), _ptr(part)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.call("pkda_qkv_conv_bwd", args, _stream(x.device))
     return dx, dw
 
 
-@pkda_qkv_conv_backward.register_fake
 def _pkda_qkv_conv_backward_fake(x, weight, dq, dk, dv, head_dim, norm_channels, eps):
     return torch.empty_like(x), torch.empty_like(weight)
 
@@ -95,4 +95,6 @@ def _backward(ctx, dq, dk, dv):
     return dx, dw, None, None, None
 
 
-pkda_qkv_conv.register_autograd(_backward, setup_context=_setup_context)
+_registry.register_fake(pkda_qkv_conv, _pkda_qkv_conv_fake)
+_registry.register_fake(pkda_qkv_conv_backward, _pkda_qkv_conv_backward_fake)
+_registry.register_autograd(pkda_qkv_conv, _backward, _setup_context)

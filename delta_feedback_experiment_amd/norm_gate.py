@@ -14,8 +14,8 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
-from . import _lib
-from .pkda import _dtype_code, _ptr, _stream
+from . import _lib, _registry
+from .pkda import _dtype_code, _on, _ptr, _stream
 
 
 def _args(x: Tensor, gate: Tensor, weight: Tensor, eps: float) -> _lib.NormGateArgs:
@@ -28,7 +28,7 @@ def _args(x: Tensor, gate: Tensor, weight: Tensor, eps: float) -> _lib.NormGateA
                              rows=x.numel() // max(x.shape[-1], 1), eps=float(eps))
 
 
-@torch.library.custom_op("pkda_mi355x::pkda_norm_gate", mutates_args=(), device_types="cuda")
+@_registry.device_op("pkda_norm_gate(Tensor x, Tensor gate, Tensor weight, float eps) -> (Tensor, Tensor)")
 def pkda_norm_gate(x: Tensor, gate: Tensor, weight: Tensor, eps: float) -> tuple[Tensor, Tensor]:
     """Fused RMSNorm with a sigmoid output gate; ``rstd`` feeds the backward
     (fla_ops.py:572-593)."""
@@ -37,18 +37,18 @@ def pkda_norm_gate(x: Tensor, gate: Tensor, weight: Tensor, eps: float) -> tuple
     y = torch.empty_like(x)
     rstd = torch.empty(args.rows, device=x.device, dtype=torch.float32)
     args.x, args.gate, args.weight, args.y, args.rstd = _ptr(x), _ptr(gate), _ptr(weight), _ptr(y), _ptr(rstd)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.call("pkda_norm_gate_fwd", args, _stream(x.device))
     return y, rstd
 
 
-@pkda_norm_gate.register_fake
 def _pkda_norm_gate_fake(x, gate, weight, eps):
     rows = x.numel() // x.shape[-1]
     return torch.empty_like(x), torch.empty((rows,), device=x.device, dtype=torch.float32)
 
 
-@torch.library.custom_op("pkda_mi355x::pkda_norm_gate_backward", mutates_args=(), device_types="cuda")
+@_registry.device_op("pkda_norm_gate_backward(Tensor x, Tensor gate, Tensor weight, Tensor rstd, Tensor dy, float eps) "
+                     "-> (Tensor, Tensor, Tensor)")
 def pkda_norm_gate_backward(x: Tensor, gate: Tensor, weight: Tensor, rstd: Tensor, dy: Tensor,
                             eps: float) -> tuple[Tensor, Tensor, Tensor]:
     """``(dx, dgate, dweight)`` (fla_ops.py:610-637); ``dweight`` is a
@@ -64,12 +64,11 @@ def pkda_norm_gate_backward(x: Tensor, gate: Tensor, weight: Tensor, rstd: Tenso
     part = torch.empty(max(ws, 1), device=x.device, dtype=torch.float32)
     args.x, args.gate, args.weight, args.rstd, args.dy = _ptr(x), _ptr(gate), _ptr(weight), _ptr(rstd), _ptr(dy)
     args.dx, args.dgate, args.dw, args.dw_part = _ptr(dx), _ptr(dgate), _ptr(dw), _ptr(part)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.call("pkda_norm_gate_bwd", args, _stream(x.device))
     return dx, dgate.to(gate_dtype), dw
 
 
-@pkda_norm_gate_backward.register_fake
 def _pkda_norm_gate_backward_fake(x, gate, weight, rstd, dy, eps):
     return torch.empty_like(x), torch.empty_like(gate), torch.empty_like(weight)
 
@@ -91,4 +90,6 @@ def _backward(ctx, dy, _drstd):
     return dx, dgate, dw, None
 
 
-pkda_norm_gate.register_autograd(_backward, setup_context=_setup_context)
+_registry.register_fake(pkda_norm_gate, _pkda_norm_gate_fake)
+_registry.register_fake(pkda_norm_gate_backward, _pkda_norm_gate_backward_fake)
+_registry.register_autograd(pkda_norm_gate, _backward, _setup_context)

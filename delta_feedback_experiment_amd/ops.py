@@ -18,13 +18,15 @@ reference's backward always does (``fla_ops.py:423-432``).
 
 from __future__ import annotations
 
+from contextlib import nullcontext
+
 import torch
 from torch import Tensor
 
-from . import _lib
+from . import _lib, _registry
 from .chunk import (CHUNK_SIZE, ChunkPlan, chunk_backward, chunk_forward, gate_backward, gate_forward,
                     wants_gcum_lo)
-from .pkda import _f32
+from .pkda import _f32, _on
 from . import precond as pre
 
 SAVED_ALWAYS = ("k_write", "a_chunk")
@@ -115,6 +117,14 @@ def _check_inputs(q, k, v, g, g_atk, beta_atk, beta, A_log, dt_bias, log_atk_sca
 _GATE_STREAMS: dict[int, torch.cuda.Stream] = {}
 
 
+OVERLAP_ELEMENTS = 3 << 24
+"""Elements of q from which the gate runs on its second stream.  The fork and
+the join cost the host 200 us a forward and backward, which a small call
+waits for, and the two kernels share the memory's bandwidth once they are
+large: 2 M elements (1,000 tokens of 16 heads) 700 us a step overlapped, 480
+in order; 8 M 720 and 480; 34 M 1,318 and 1,300; 67 M 2,315 and 2,333."""
+
+
 def _gate_stream(dev: torch.device) -> torch.cuda.Stream:
     """A second stream per device (default priority) for the per-channel
     gate, which neither reads nor writes anything of the preconditioner's:
@@ -127,6 +137,41 @@ def _gate_stream(dev: torch.device) -> torch.cuda.Stream:
     return s
 
 
+def _autocast(dtype: torch.dtype | None):
+    if dtype is None and not torch.is_autocast_enabled("cuda"):
+        return nullcontext()  # the state asked for
+    return torch.autocast("cuda", enabled=dtype is not None, dtype=dtype or torch.bfloat16)
+
+
+class _beside:
+    """Launches inside the ``with`` go to the gate's stream when ``like`` is
+    large enough for that to pay, else stay on the current one;
+    :meth:`join` lets the current stream wait for them and marks their
+    results, allocated over there, as used by it."""
+
+    def __init__(self, like: Tensor):
+        self.cur = self.side = None
+        if like.numel() >= OVERLAP_ELEMENTS:
+            self.cur, self.side = torch.cuda.current_stream(like.device), _gate_stream(like.device)
+
+    def __enter__(self) -> "_beside":
+        if self.side is not None:
+            self.side.wait_stream(self.cur)
+            self.switch = torch.cuda.stream(self.side)
+            self.switch.__enter__()
+        return self
+
+    def __exit__(self, *exc) -> None:
+        if self.side is not None:
+            self.switch.__exit__(*exc)
+
+    def join(self, *results: Tensor) -> None:
+        if self.side is not None:
+            self.cur.wait_stream(self.side)
+            for t in results:
+                t.record_stream(self.cur)
+
+
 def _forward(q, k, v, g, g_atk, beta_atk, beta, A_log, dt_bias, log_atk_scale, scale, squash_x, squash_eps,
              save_all: bool):
     plan = ChunkPlan.make(q, None)
@@ -136,16 +181,12 @@ def _forward(q, k, v, g, g_atk, beta_atk, beta, A_log, dt_bias, log_atk_scale, s
         gf = gf.float()
     A32, dt32 = _f32(A_log), _f32(dt_bias)
     gcum_lo = _gcum_lo(plan, qf)
-    # the gate on its own stream beside the preconditioner (both read only
-    # the inputs); gcum is allocated there and recorded as used by this one
-    cur, side = torch.cuda.current_stream(q.device), _gate_stream(q.device)
-    side.wait_stream(cur)
-    with torch.cuda.stream(side):
+    # the gate beside the preconditioner (both read only the inputs)
+    with _beside(qf) as own:
         gcum = gate_forward(plan, gf, _lib.GATE_RAW_CHANNEL, A32, dt32, gcum_lo=gcum_lo)
     pstate = pre.precond_forward(plan, kf, g_atk, beta_atk, log_atk_scale, squash_x, squash_eps, None,
                                  want_kw32=True)
-    cur.wait_stream(side)
-    gcum.record_stream(cur)
+    own.join(gcum)
     beta32 = _f32(beta).reshape(plan.num_tokens, plan.heads)
     o, _, fs = chunk_forward(plan, qf, kf, pstate.kw, vf, gcum, beta32, scale, None, False, save_states=save_all,
                              gcum_lo=gcum_lo)
@@ -159,7 +200,10 @@ def _gcum_lo(plan: ChunkPlan, qf: Tensor) -> Tensor | None:
     return torch.empty(plan.num_tokens, plan.heads, plan.head_dim, device=qf.device, dtype=torch.float32)
 
 
-@torch.library.custom_op("pkda_mi355x::pkda_recurrence", mutates_args=(), device_types="cuda")
+@_registry.device_op(
+    "pkda_recurrence(Tensor q, Tensor k, Tensor v, Tensor g, Tensor g_atk, Tensor beta_atk, Tensor beta, Tensor A_log, "
+    "Tensor dt_bias, Tensor log_atk_scale, float scale, float squash_x, float squash_eps, bool lean) "
+    "-> (Tensor, Tensor[])")
 def pkda_recurrence(
     q: Tensor, k: Tensor, v: Tensor, g: Tensor, g_atk: Tensor, beta_atk: Tensor, beta: Tensor,
     A_log: Tensor, dt_bias: Tensor, log_atk_scale: Tensor,
@@ -172,7 +216,7 @@ def pkda_recurrence(
     computed on the device.  ``o`` is in ``q.dtype``.
     """
     _check_inputs(q, k, v, g, g_atk, beta_atk, beta, A_log, dt_bias, log_atk_scale)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         (plan, qf, kf, vf, gf, A32, dt32, gcum, gcum_lo, pstate, beta32, o, fs) = _forward(
             q, k, v, g, g_atk, beta_atk, beta, A_log, dt_bias, log_atk_scale, scale, squash_x, squash_eps,
             save_all=not lean)
@@ -185,7 +229,6 @@ def pkda_recurrence(
     return o.reshape(*q.shape[:3], v.shape[-1]).to(q.dtype), saved
 
 
-@pkda_recurrence.register_fake
 def _pkda_recurrence_fake(q, k, v, g, g_atk, beta_atk, beta, A_log, dt_bias, log_atk_scale,
                           scale, squash_x, squash_eps, lean):
     out = torch.empty((*q.shape[:3], v.shape[-1]), device=q.device, dtype=q.dtype)
@@ -193,7 +236,10 @@ def _pkda_recurrence_fake(q, k, v, g, g_atk, beta_atk, beta, A_log, dt_bias, log
     return out, saved
 
 
-@torch.library.custom_op("pkda_mi355x::pkda_recurrence_backward", mutates_args=(), device_types="cuda")
+@_registry.device_op(
+    "pkda_recurrence_backward(Tensor q, Tensor k, Tensor v, Tensor g, Tensor g_atk, Tensor beta_atk, Tensor beta, "
+    "Tensor A_log, Tensor dt_bias, Tensor log_atk_scale, Tensor[] saved, Tensor do, float scale, float squash_x, "
+    "float squash_eps, ScalarType? autocast_dtype, bool lean) -> Tensor[]")
 def pkda_recurrence_backward(
     q: Tensor, k: Tensor, v: Tensor, g: Tensor, g_atk: Tensor, beta_atk: Tensor, beta: Tensor,
     A_log: Tensor, dt_bias: Tensor, log_atk_scale: Tensor, saved: list[Tensor], do: Tensor,
@@ -209,8 +255,7 @@ def pkda_recurrence_backward(
     gradients do not depend on it."""
     from .chunk import FwdSaved
 
-    with torch.cuda.device(q.device), torch.autocast(
-            "cuda", enabled=autocast_dtype is not None, dtype=autocast_dtype or torch.bfloat16):
+    with _on(q.device), _autocast(autocast_dtype):
         plan = ChunkPlan.make(q, None)
         flat = lambda t: t.contiguous().reshape(plan.num_tokens, plan.heads, *t.shape[3:])  # noqa: E731
         qf, kf, vf, gf = flat(q), flat(k), flat(v), flat(g)
@@ -237,17 +282,13 @@ def pkda_recurrence_backward(
         pstate = pre.PrecondState(kw, a_chunk, None, None)
         dk = torch.empty_like(kf)  # the preconditioner's scan writes the final dk in k's dtype
         # the gate's backward (dgcum only) beside the preconditioner's (dk, dkw)
-        cur, side = torch.cuda.current_stream(q.device), _gate_stream(q.device)
-        side.wait_stream(cur)
-        with torch.cuda.stream(side):
+        with _beside(qf) as own:
             dg, dA_log, ddt_bias = gate_backward(plan, gf, _lib.GATE_RAW_CHANNEL, A32, dt32, gr.dgcum,
                                                  dg_dtype=gf.dtype)
         dg_atk, dbeta_atk, dcenter, _ = pre.precond_backward(
             plan, kf, g_atk, beta_atk, log_atk_scale, squash_x, squash_eps, pstate, gr.dkw, gr.dk, None, False,
             dk_final=dk)
-        cur.wait_stream(side)
-        for t in (dg, dA_log, ddt_bias):
-            t.record_stream(cur)
+        own.join(dg, dA_log, ddt_bias)
     shape = tuple(q.shape)
     lead = shape[:3]
     return [
@@ -259,7 +300,6 @@ def pkda_recurrence_backward(
     ]
 
 
-@pkda_recurrence_backward.register_fake
 def _pkda_recurrence_backward_fake(q, k, v, g, g_atk, beta_atk, beta, A_log, dt_bias, log_atk_scale, saved, do,
                                    scale, squash_x, squash_eps, autocast_dtype, lean):
     return [torch.empty_like(t) for t in (q, k, v, g, g_atk, beta_atk, beta, A_log, dt_bias, log_atk_scale)]
@@ -277,7 +317,7 @@ def _setup_context(ctx, inputs, output) -> None:
     ctx.set_materialize_grads(False)
 
 
-def _backward(ctx, do, _dsaved):
+def _backward(ctx, do, *_dsaved):
     if do is None:
         return (None,) * 14
     tensors = ctx.saved_tensors
@@ -287,4 +327,6 @@ def _backward(ctx, do, _dsaved):
     return (*grads, None, None, None, None)
 
 
-pkda_recurrence.register_autograd(_backward, setup_context=_setup_context)
+_registry.register_fake(pkda_recurrence, _pkda_recurrence_fake)
+_registry.register_fake(pkda_recurrence_backward, _pkda_recurrence_backward_fake)
+_registry.register_autograd(pkda_recurrence, _backward, _setup_context)

@@ -17,12 +17,12 @@ no CPU fallback.
 
 from __future__ import annotations
 
-import ctypes
+from contextlib import nullcontext
 
 import torch
 from torch import Tensor
 
-from . import _lib
+from . import _lib, _registry
 
 
 def _ptr(t: Tensor | None) -> int | None:
@@ -52,11 +52,22 @@ def _require_cuda(*tensors: Tensor | None) -> torch.device:
 
 
 def _f32(t: Tensor | None) -> Tensor | None:
-    return None if t is None else t.detach().to(torch.float32).contiguous()
+    if t is None:
+        return None
+    t = t.detach()
+    return t if t.dtype == torch.float32 and t.is_contiguous() else t.to(torch.float32).contiguous()
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+def _on(device: torch.device):
+    """A context with ``device`` current: nothing to do when it is already."""
+    if device.index is None or device.index == torch.cuda.current_device():
+        return nullcontext()
+    return torch.cuda.device(device)
 
 
 def gate_form(g: Tensor, lead_shape: tuple[int, ...], K: int, use_gate_in_kernel: bool,
@@ -273,13 +284,15 @@ def pkda_decode_step_(
     o = out if out is not None else torch.empty_like(v)
     if o.shape != v.shape or o.dtype != v.dtype or not o.is_contiguous():
         raise ValueError(f"out must be a contiguous {v.dtype} {tuple(v.shape)} tensor")
-    decode_step_op(q, k, v, g, beta, state_pool, slot_idx, a_pool, g_atk, beta_atk, log_atk_scale, A_log, dt_bias,
-                   bool(use_gate_in_kernel), float(scale), float(x), float(eps), o)
+    _registry.call(decode_step_op, q, k, v, g, beta, state_pool, slot_idx, a_pool, g_atk, beta_atk, log_atk_scale,
+                   A_log, dt_bias, bool(use_gate_in_kernel), float(scale), float(x), float(eps), o)
     return o
 
 
-@torch.library.custom_op("pkda_mi355x::decode_step_", mutates_args=("state_pool", "a_pool", "o"),
-                         device_types="cuda")
+@_registry.device_op(
+    "decode_step_(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor(a!) state_pool, Tensor? slot_idx, "
+    "Tensor(b!)? a_pool, Tensor? g_atk, Tensor? beta_atk, Tensor? log_atk_scale, Tensor? A_log, Tensor? dt_bias, "
+    "bool use_gate_in_kernel, float scale, float x, float eps, Tensor(c!) o) -> ()")
 def decode_step_op(
     q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, state_pool: Tensor, slot_idx: Tensor | None,
     a_pool: Tensor | None, g_atk: Tensor | None, beta_atk: Tensor | None, log_atk_scale: Tensor | None,
@@ -306,11 +319,8 @@ def decode_step_op(
         state_pool=_ptr(state_pool), a_pool=_ptr(a_pool), pool_size=state_pool.shape[0],
         slot_idx=_ptr(idx), o=_ptr(o),
     )
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("pkda_decode_step", args, _stream(device))
 
 
-@decode_step_op.register_fake
-def _decode_step_fake(q, k, v, g, beta, state_pool, slot_idx, a_pool, g_atk, beta_atk, log_atk_scale, A_log,
-                      dt_bias, use_gate_in_kernel, scale, x, eps, o) -> None:
-    return None
+_registry.register_fake(decode_step_op, lambda *args: None)

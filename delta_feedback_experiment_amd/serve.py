@@ -33,9 +33,9 @@ from dataclasses import dataclass
 import torch
 from torch import Tensor
 
-from . import _lib
+from . import _lib, _registry
 from .chunk import ChunkPlan, _flat, chunk_forward, gate_forward, validate_cu_seqlens, wants_gcum_lo
-from .pkda import (_check_common, _dtype_code, _f32, _ptr, _require_cuda, _require_device, _stream,
+from .pkda import (_check_common, _dtype_code, _f32, _on, _ptr, _require_cuda, _require_device, _stream,
                    check_slot_indices, gate_form)
 
 
@@ -132,12 +132,17 @@ def pkda_prefill_(
     if scale is None:
         scale = D ** -0.5
     o = torch.empty_like(v)
-    prefill_op(q, k, v, g, beta, state_pool, slot_idx, a_pool, bool(continue_state), cu_seqlens, g_atk, beta_atk,
-               log_atk_scale, A_log, dt_bias, bool(use_gate_in_kernel), float(scale), float(x), float(eps), o)
+    _registry.call(prefill_op, q, k, v, g, beta, state_pool, slot_idx, a_pool, bool(continue_state), cu_seqlens,
+                   g_atk, beta_atk, log_atk_scale, A_log, dt_bias, bool(use_gate_in_kernel), float(scale), float(x),
+                   float(eps), o)
     return o
 
 
-@torch.library.custom_op("pkda_mi355x::prefill_", mutates_args=("state_pool", "a_pool", "o"), device_types="cuda")
+@_registry.device_op(
+    "prefill_(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor(a!) state_pool, Tensor slot_idx, "
+    "Tensor(b!)? a_pool, bool continue_state, Tensor? cu_seqlens, Tensor? g_atk, Tensor? beta_atk, "
+    "Tensor? log_atk_scale, Tensor? A_log, Tensor? dt_bias, bool use_gate_in_kernel, float scale, float x, float eps, "
+    "Tensor(c!) o) -> ()")
 def prefill_op(
     q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, state_pool: Tensor, slot_idx: Tensor,
     a_pool: Tensor | None, continue_state: bool, cu_seqlens: Tensor | None, g_atk: Tensor | None,
@@ -152,7 +157,7 @@ def prefill_op(
     idx = slot_idx.contiguous()
     from . import precond as pre
 
-    with torch.no_grad(), torch.cuda.device(device):
+    with torch.no_grad(), _on(device):
         plan = ChunkPlan.make(q, cu_seqlens)
         kind, g_used = gate_form(g, q.shape[:-1], D, use_gate_in_kernel, A_log, dt_bias)
         g_used = g_used.contiguous()
@@ -175,10 +180,7 @@ def prefill_op(
                       slot_idx=idx, final_state=state_pool, out=_flat(o, plan), gcum_lo=gcum_lo)
 
 
-@prefill_op.register_fake
-def _prefill_fake(q, k, v, g, beta, state_pool, slot_idx, a_pool, continue_state, cu_seqlens, g_atk, beta_atk,
-                  log_atk_scale, A_log, dt_bias, use_gate_in_kernel, scale, x, eps, o) -> None:
-    return None
+_registry.register_fake(prefill_op, lambda *args: None)
 
 
 def pkda_qkv_conv_cached_(
@@ -219,11 +221,13 @@ def pkda_qkv_conv_cached_(
         _slots(slot_idx, B, P, check_slots)
     elif B > P:
         raise ValueError("more rows than pool slots")
-    return qkv_conv_cached_op(x, weight, int(head_dim), int(norm_channels), float(eps), conv_pool, slot_idx,
-                              bool(continue_state))
+    return _registry.call(qkv_conv_cached_op, x, weight, int(head_dim), int(norm_channels), float(eps), conv_pool,
+                          slot_idx, bool(continue_state))
 
 
-@torch.library.custom_op("pkda_mi355x::qkv_conv_cached_", mutates_args=("conv_pool",), device_types="cuda")
+@_registry.device_op(
+    "qkv_conv_cached_(Tensor x, Tensor weight, int head_dim, int norm_channels, float eps, Tensor(a!) conv_pool, "
+    "Tensor? slot_idx, bool continue_state) -> (Tensor, Tensor, Tensor)")
 def qkv_conv_cached_op(
     x: Tensor, weight: Tensor, head_dim: int, norm_channels: int, eps: float, conv_pool: Tensor,
     slot_idx: Tensor | None, continue_state: bool,
@@ -245,12 +249,14 @@ def qkv_conv_cached_op(
         slot_idx=_ptr(idx), history_in=_ptr(conv_pool) if continue_state else None,
         history_out=_ptr(conv_pool), pool_size=P,
     )
-    with torch.no_grad(), torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.call("pkda_qkv_conv_fwd", args, _stream(x.device))
     return q, k, v
 
 
-@qkv_conv_cached_op.register_fake
 def _qkv_conv_cached_fake(x, weight, head_dim, norm_channels, eps, conv_pool, slot_idx, continue_state):
     B, T, Cx = x.shape
     return tuple(x.new_empty(B, T, Cx // 3) for _ in range(3))
+
+
+_registry.register_fake(qkv_conv_cached_op, _qkv_conv_cached_fake)

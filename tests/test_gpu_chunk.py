@@ -749,3 +749,29 @@ def test_production_key_gradient_handoff(dev):
     for n, (x, y, z) in res.items():
         assert x < BF16_TOL and y < BF16_TOL, (n, x, y)
         assert z < 1e-2, (n, z)
+
+
+@pytest.mark.parametrize("lean", [False, True])
+def test_pkda_recurrence_overlap_same_bits(dev, lean, monkeypatch):
+    """The gate on its second stream (large calls) and on the caller's (small
+    ones): the same output and gradients bit for bit, and the overlapped form
+    captured and replayed as the graph test above does for the other."""
+    from delta_feedback_experiment_amd import ops
+
+    print(f"[gpu] pkda_recurrence overlap lean={lean}", flush=True)
+    (q, k, v, g_raw, beta, A_log, dt_bias, g_atk, beta_atk, center) = _production_inputs(
+        2, 100, 2, 64, torch.bfloat16, 17)
+    leaves = [x.to(dev).clone().requires_grad_()
+              for x in (q, k, v, g_raw, g_atk, beta_atk, beta, A_log, dt_bias, center)]
+    do = torch.randn(2, 100, 2, 64, generator=torch.Generator().manual_seed(6)).to(dev, torch.bfloat16)
+
+    def step():
+        o, _ = ops.pkda_recurrence(*leaves, 0.125, 1.5, 1e-6, lean)
+        return [o.detach()] + list(torch.autograd.grad(o, leaves, do))
+
+    monkeypatch.setattr(ops, "OVERLAP_ELEMENTS", 1 << 60)
+    in_order = [t.clone() for t in step()]
+    monkeypatch.setattr(ops, "OVERLAP_ELEMENTS", 0)
+    for a, b in zip(step(), in_order):
+        assert torch.equal(a, b)
+    test_pkda_recurrence_graph_replays_match_eager(dev, lean)

@@ -1,0 +1,72 @@
+"""The operators' registration: what a backward through an operator without a
+formula, a second derivative and a CPU tensor raise, and the version counters
+of what an operator writes."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from delta_feedback_experiment_amd import _registry, pkda_norm_gate, pkda_qkv_conv
+from delta_feedback_experiment_amd.serve import qkv_conv_cached_op
+
+
+def _meta(*shape, grad=False):
+    return torch.empty(*shape, device="meta", requires_grad=grad)
+
+
+def test_backward_without_a_formula_raises():
+    args = (_meta(2, 3, 96, grad=True), _meta(96, 4), 32, 64, 1e-6, _meta(4, 3, 96), None, True)
+    for call in (qkv_conv_cached_op, lambda *a: _registry.call(qkv_conv_cached_op, *a)):
+        q, _, _ = call(*args)
+        assert q.requires_grad
+        with pytest.raises(RuntimeError, match="no autograd formula"):
+            q.sum().backward()
+
+
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_second_derivative_raises(create_graph):
+    x, gate, w = _meta(5, 64, grad=True), _meta(5, 64, grad=True), _meta(64, grad=True)
+    y, rstd = pkda_norm_gate(x, gate, w, 1e-6)
+    assert not rstd.requires_grad
+    dx, dgate, dw = torch.autograd.grad(y, (x, gate, w), torch.empty_like(y), create_graph=create_graph)
+    assert dx.shape == x.shape and dw.shape == w.shape
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(dx, x, torch.empty_like(dx))
+
+
+def test_saved_tensor_hooks_see_the_inputs():
+    packed = []
+    x, w = _meta(2, 5, 96, grad=True), _meta(96, 4, grad=True)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(tuple(t.shape)) or t, lambda t: t):
+        q, k, v = pkda_qkv_conv(x, w, 32, 64, 1e-6)
+    assert packed == [(2, 5, 96), (96, 4)]
+    torch.autograd.grad((q, k, v), (x, w), [torch.empty_like(t) for t in (q, k, v)])
+
+
+def test_cpu_tensors_are_refused():
+    x = torch.zeros(5, 64)
+    with pytest.raises(NotImplementedError, match="CPU"):
+        pkda_norm_gate(x, x, torch.ones(64), 1e-6)
+
+
+@pytest.mark.gpu
+def test_written_tensors_change_version():
+    from delta_feedback_experiment_amd import pkda_decode_step_, pkda_qkv_conv_cached_
+
+    print("[gpu] version counters of the pools", flush=True)
+    dev = torch.device("cuda:0")
+    pool, a_pool, conv = (torch.zeros(*s, device=dev) for s in ((3, 1, 64, 64), (3, 1, 64), (3, 3, 192)))
+    q, g, idx = torch.ones(2, 1, 64, device=dev), torch.zeros(2, 1, device=dev), torch.tensor([2, 0], device=dev).int()
+    before = [t._version for t in (pool, a_pool, conv)]
+    for grad in (False, True):  # with gradients asked for, through the operator's autograd kernel
+        pkda_decode_step_(q.clone().requires_grad_(grad), q, q, g, g, pool, idx, a_pool=a_pool, g_atk=g, beta_atk=g,
+                          log_atk_scale=torch.zeros(1, device=dev))
+        pkda_qkv_conv_cached_(torch.ones(2, 1, 192, device=dev, requires_grad=grad), torch.ones(192, 4, device=dev),
+                              64, 128, 1e-6, conv, idx)
+        after = [t._version for t in (pool, a_pool, conv)]
+        assert all(b > a for a, b in zip(before, after)), (before, after)
+        before = after
+    with torch.inference_mode():
+        pkda_decode_step_(q, q, q, g, g, pool.clone(), idx)
+    torch.cuda.synchronize()

@@ -2123,6 +2123,348 @@ __global__ __launch_bounds__(64 * (BV / 16 + kRrLoadersBwd)) void chunk_state_bw
   }
 }
 
+// The same pass with the chunk's outputs on waves of their own, as the
+// forward's chunk_state_fwd_split_kernel: BV / 16 chain waves keep dS and do the
+// chain dS -> KW dS -> dU -> Z -> dS; they leave the entering dS as B operands
+// and Z in FP32, lane for lane, in LDS, and BV / 16 output waves store the
+// checkpoint in the same step and form the dBv / dv rows in the next one.  Q^T
+// (s e^G dO), which waits for nothing of the chain, is added to the decayed dS
+// while Z forms.
+template <int D, int BV>
+struct RrSplitBwdLayout : RrBwdLayout<D, BV, true> {
+  using Base = RrBwdLayout<D, BV, true>;
+  static constexpr int NC = BV / 16;
+  static constexpr int SB = NC * (D / 32) * 1024;  // entering dS as B operands, one 16-byte piece a lane
+  static constexpr int ZB = NC * 4 * 1024;         // Z's accumulators
+  static constexpr int off_SB = 2 * Base::BUF;
+  static constexpr int off_ZB = off_SB + 2 * SB;
+  static constexpr int off_Out = off_ZB + 2 * ZB;
+  static constexpr int bytes = off_Out + 2 * Base::OUT;
+  static_assert(bytes <= 160 * 1024, "LDS of one compute unit");
+};
+
+template <int D, int BV, bool PACK, bool DEFER>
+__global__ __launch_bounds__(64 * (2 * (BV / 16) + kSplitLoaders))
+__attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_state_bwd_split_kernel(BwdParams p) {
+  using L = RrSplitBwdLayout<D, BV>;
+  using T = bf16_t;
+  constexpr int NC = BV / 16;
+  constexpr int NKT = D / 16;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const DocSlot ds = doc_slot(p.geom, p.H, D / BV);
+  const int n = ds.n, h = ds.h, v0 = ds.z * BV;
+  const int H = p.H;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int64_t gs = (int64_t)H * D;
+  int first, count, dstart, dlen;
+  doc_chunks(p.geom, n, first, count, dstart, dlen);
+  const int q4 = 4 * (lane >> 4), il = lane & 15;
+  auto sb_slot = [&](int w, int s, int kk) {
+    return reinterpret_cast<uint4*>(smem + L::off_SB + (s & 1) * L::SB + (w * (NKT / 2) + kk) * 1024) + lane;
+  };
+  auto z_slot = [&](int w, int s, int rb) {
+    return reinterpret_cast<f32x4*>(smem + L::off_ZB + (s & 1) * L::ZB + (w * 4 + rb) * 1024) + lane;
+  };
+
+  // Visits s = 0, 1, ... take chunks jc = count - 1 - s; steps 0 .. count + 1, a
+  // barrier before each: the chain takes visit s in step s, its rows reach the
+  // output stage by the end of step s + 1 and global memory in step s + 2.
+  if (wave >= 2 * NC) {
+    constexpr int NGT = 128;        // threads of one loader group
+    const int ltid = tid - 64 * 2 * NC;
+    const int lgroup = ltid / NGT;  // takes visits s with s % 2 == lgroup
+    const int lt = ltid % NGT;
+    RegTile<NGT, C, D, T> rQ, rKW;
+    std::conditional_t<PACK, TriRegTile<NGT>, RegTile<NGT, C, C, T>> rA, rT;
+    RegTile<NGT, C, BV, T> rdO;
+    float rg = 0.f, rb = 0.f;
+    if constexpr (PACK) {  // the stages' blocks above the diagonal: zero once
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        zero_upper_blocks<2 * NGT>(ltid, reinterpret_cast<T*>(smem + b * L::BUF + L::off_A), L::LDC);
+        zero_upper_blocks<2 * NGT>(ltid, reinterpret_cast<T*>(smem + b * L::BUF + L::off_T), L::LDC);
+      }
+    }
+    auto load = [&](int s) {
+      const int jc = count - 1 - s;
+      const int cstart = dstart + jc * C;
+      const int clen = min(C, dlen - jc * C);
+      const int64_t row0 = (int64_t)cstart * H + h;
+      rQ.load_as(lt, static_cast<const T*>(p.q) + row0 * D, gs, clen);
+      rKW.load_as(lt, static_cast<const T*>(p.kw) + row0 * D, gs, clen);
+      if constexpr (PACK) {
+        const int64_t tri0 = ((int64_t)(first + jc) * H + h) * kTriElems;
+        rA.load_as(lt, static_cast<const T*>(p.aqk) + tri0);
+        rT.load_as(lt, static_cast<const T*>(p.akk) + tri0);
+      } else {
+        rA.load_as(lt, static_cast<const T*>(p.aqk) + row0 * C, (int64_t)H * C, clen);
+        rT.load_as(lt, static_cast<const T*>(p.akk) + row0 * C, (int64_t)H * C, clen);
+      }
+      rdO.load_as(lt, static_cast<const T*>(p.dO) + row0 * D + v0, gs, clen);
+      if (lt < C) {
+        const int64_t gi = (int64_t)(cstart + min(lt, clen - 1)) * H + h;
+        rg = p.gcum[gi];
+        rb = lt < clen ? p.beta[gi] : 0.f;
+      }
+    };
+    auto stash = [&](int b) {
+      char* buf = smem + b * L::BUF;
+      rQ.store_as(lt, reinterpret_cast<T*>(buf + L::off_Q), L::LD);
+      rKW.store_as(lt, reinterpret_cast<T*>(buf + L::off_KW), L::LD);
+      rA.store_as(lt, reinterpret_cast<T*>(buf + L::off_A), L::LDC);
+      rT.store_as(lt, reinterpret_cast<T*>(buf + L::off_T), L::LDC);
+      rdO.store_as(lt, reinterpret_cast<T*>(buf + L::off_dO), L::LDV);
+      if (lt < C) {
+        reinterpret_cast<float*>(buf + L::off_G)[lt] = rg;
+        reinterpret_cast<float*>(buf + L::off_B)[lt] = rb;
+      }
+    };
+    // visit s's dBv / dv rows from the output stage to global memory
+    auto flush = [&](int s) {
+      constexpr int SEG = BV / 8;  // 16-byte pieces of a row
+      static_assert(C * SEG % NGT == 0, "whole passes over the stage");
+      const T* so = reinterpret_cast<const T*>(smem + L::off_Out + (s & 1) * L::OUT);
+      const int jc = count - 1 - s;
+      const int clen = min(C, dlen - jc * C);
+      const int64_t row0 = (int64_t)(dstart + jc * C) * H + h;
+#pragma unroll
+      for (int it = 0; it < C * SEG / NGT; ++it) {
+        const int i = lt + it * NGT;
+        const int r = i / SEG, sg = i % SEG;
+        if (r < clen) {
+          const uint4 x = *reinterpret_cast<const uint4*>(so + r * L::LDV + 8 * sg);
+          store16_nt(static_cast<T*>(p.dv_handoff ? p.dv : p.du) + (row0 + (int64_t)r * H) * D + v0 + 8 * sg, x);
+        }
+      }
+    };
+    if (lgroup < count) load(lgroup);
+    if (lgroup == 0 && count > 0) {
+      stash(0);
+      if (!DEFER && count > 2) load(2);
+    }
+    for (int s = 0; s < count + 2; ++s) {
+      __syncthreads();
+      if (((s + 1) & 1) == lgroup) {
+        if (s + 1 < count) {
+          stash((s + 1) & 1);
+          if (!DEFER && s + 3 < count) load(s + 3);
+        }
+      } else {
+        if (DEFER && s + 2 < count) load(s + 2);
+        if (s >= 2) flush(s - 2);
+      }
+    }
+    return;
+  }
+
+  if (wave >= NC) {  // output waves
+    const int w = wave - NC;  // the chain wave whose columns these are
+    const int col0 = v0 + 16 * w;
+    float bl = 0.f, b4[4][4];  // beta of row `lane` and of this lane's accumulator rows
+    for (int s = 0; s < count + 2; ++s) {
+      __syncthreads();
+      if (s >= 1 && s <= count) {
+        // visit s - 1: the per-chunk kernel needs dU only through dBv = T^T dU =
+        // -Z: hand it that, or (dv_handoff) dv = beta dBv with dBv itself for
+        // the rows whose beta is too small to divide by
+        f32x4 hz[4];
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) hz[rb] = -*z_slot(w, s - 1, rb);
+        if (p.dv_handoff) {
+          // one test per chunk (lane r looks at row r; the ballot is uniform)
+          const int jc = count - s;
+          const int clen = min(C, dlen - jc * C);
+          if (__builtin_expect(__ballot(lane < clen && !(fabsf(bl) >= 1e-20f)) != 0, 0)) {
+            T* du_out = static_cast<T*>(p.du) + ((int64_t)(dstart + jc * C) * H + h) * D + col0;
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const int r = 16 * rb + q4 + j;
+                if (r < clen && !(fabsf(b4[rb][j]) >= 1e-20f)) du_out[(int64_t)r * gs + il] = to_e<T>(hz[rb][j]);
+              }
+          }
+#pragma unroll
+          for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) hz[rb][j] *= b4[rb][j];
+        }
+        T* so = reinterpret_cast<T*>(smem + L::off_Out + ((s - 1) & 1) * L::OUT) + 16 * w;
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) store_acc_global<T, true>(so, L::LDV, hz[rb], 16 * rb, 0, C, lane);
+      }
+      if (s < count) {  // visit s: the checkpoint; its beta, whose stage the next step takes
+        const float* sB = reinterpret_cast<const float*>(smem + (s & 1) * L::BUF + L::off_B);
+        T* hb = static_cast<T*>(p.dh) + ((int64_t)(first + count - 1 - s) * H + h) * D * D;
+#pragma unroll
+        for (int kk = 0; kk < NKT / 2; ++kk) {
+          const uint4 x = *sb_slot(w, s, kk);
+          store_packed_tile_nt(hb + tile_offset(D, 2 * kk, col0 / 16), x.x, x.y, lane);
+          store_packed_tile_nt(hb + tile_offset(D, 2 * kk + 1, col0 / 16), x.z, x.w, lane);
+        }
+        bl = sB[lane];
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) lds4(sB + 16 * rb + q4, b4[rb]);
+      }
+    }
+    return;
+  }
+
+  const int col0 = v0 + 16 * wave;
+  f32x4 dS[NKT];
+  s16x8_t dSB[NKT / 2];  // dS as B operands
+#pragma unroll
+  for (int rt = 0; rt < NKT; ++rt)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      dS[rt][j] = p.dht ? p.dht[(((int64_t)n * H + h) * D + 16 * rt + q4 + j) * D + col0 + il] : 0.f;
+  const float scale = p.scale;
+  auto publish = [&](int s) {  // dS entering visit s
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk) {
+      dSB[kk] = pack_acc_pair(dS[2 * kk], dS[2 * kk + 1]);
+      *sb_slot(wave, s, kk) = __builtin_bit_cast(uint4, dSB[kk]);
+    }
+  };
+  publish(0);
+  for (int s = 0; s < count; ++s) {
+    __syncthreads();
+    const char* buf = smem + (s & 1) * L::BUF;
+    const T* sQ = reinterpret_cast<const T*>(buf + L::off_Q);
+    const T* sK = reinterpret_cast<const T*>(buf + L::off_KW);
+    const T* sA = reinterpret_cast<const T*>(buf + L::off_A);
+    const T* sT = reinterpret_cast<const T*>(buf + L::off_T);
+    const T* sdO = reinterpret_cast<const T*>(buf + L::off_dO);
+    const float* sG = reinterpret_cast<const float*>(buf + L::off_G);
+    const float* sB = reinterpret_cast<const float*>(buf + L::off_B);
+    // the LDS reads ahead of what waits for them (as in the forward's chain)
+    s16x8_t ak[NKT / 2][4];
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) ak[kk][rb] = lds_a_perm(sK + 16 * rb * L::LD, L::LD, 32 * kk, lane);
+    // dO of this wave's columns as B operands over the tokens; Aqk^T's row
+    // block rb needs k steps kt >= rb / 2, and so T^T's
+    const s16x8_t dOB[2] = {lds_kmajor_perm(sdO + 16 * wave, L::LDV, 0, lane),
+                            lds_kmajor_perm(sdO + 16 * wave, L::LDV, 32, lane)};
+    s16x8_t aa[6];
+    aa[0] = lds_kmajor_perm(sA + 0, L::LDC, 0, lane);
+    aa[1] = lds_kmajor_perm(sA + 0, L::LDC, 32, lane);
+    aa[2] = lds_kmajor_perm(sA + 16, L::LDC, 0, lane);
+    aa[3] = lds_kmajor_perm(sA + 16, L::LDC, 32, lane);
+    aa[4] = lds_kmajor_perm(sA + 32, L::LDC, 32, lane);
+    aa[5] = lds_kmajor_perm(sA + 48, L::LDC, 32, lane);
+    float gg[4][4], bb[4][4];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) {
+      lds4(sG + 16 * rb + q4, gg[rb]);
+      lds4(sB + 16 * rb + q4, bb[rb]);
+    }
+    const float gC = sG[C - 1];
+    __builtin_amdgcn_sched_barrier(0);
+    // KW dS and Aqk^T dO
+    f32x4 KS[4], dU[4];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) KS[rb] = dU[rb] = zero4();
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) mfma_bf16(KS[rb], ak[kk][rb], dSB[kk]);
+    mfma_bf16(dU[0], aa[0], dOB[0]);
+    mfma_bf16(dU[1], aa[2], dOB[0]);
+    mfma_bf16(dU[0], aa[1], dOB[1]);
+    mfma_bf16(dU[1], aa[3], dOB[1]);
+    mfma_bf16(dU[2], aa[4], dOB[1]);
+    mfma_bf16(dU[3], aa[5], dOB[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    s16x8_t at[6];
+    at[0] = lds_kmajor_perm(sT + 0, L::LDC, 0, lane);
+    at[1] = lds_kmajor_perm(sT + 0, L::LDC, 32, lane);
+    at[2] = lds_kmajor_perm(sT + 16, L::LDC, 0, lane);
+    at[3] = lds_kmajor_perm(sT + 16, L::LDC, 32, lane);
+    at[4] = lds_kmajor_perm(sT + 32, L::LDC, 32, lane);
+    at[5] = lds_kmajor_perm(sT + 48, L::LDC, 32, lane);
+    s16x8_t kq[2][NKT];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) kq[kt][rt] = lds_kmajor_perm(sQ + 16 * rt, L::LD, 32 * kt, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    // dU = Aqk^T dO + diag(e^{G_C - G}) KW dS
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dU[rb][j] += exp_fast(gC - gg[rb][j]) * KS[rb][j];
+    // Z = T^T (-dU)
+    const s16x8_t dUnB[2] = {pack_acc_pair(-dU[0], -dU[1]), pack_acc_pair(-dU[2], -dU[3])};
+    f32x4 Z[4];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) Z[rb] = zero4();
+    mfma_bf16(Z[0], at[0], dUnB[0]);
+    mfma_bf16(Z[1], at[2], dUnB[0]);
+    mfma_bf16(Z[0], at[1], dUnB[1]);
+    mfma_bf16(Z[1], at[3], dUnB[1]);
+    mfma_bf16(Z[2], at[4], dUnB[1]);
+    mfma_bf16(Z[3], at[5], dUnB[1]);
+    // dS <- e^{G_C} dS + Q^T (s e^G dO) + K^T diag(beta e^G) Z
+    s16x8_t dOgB[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      float f[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] = scale * exp_fast(gg[2 * kt + (e < 4 ? 0 : 1)][e & 3]);
+      dOgB[kt] = scale_frag(dOB[kt], f);
+    }
+    const float decay = exp_fast(gC);
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt) dS[rt] = dS[rt] * decay;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], kq[kt][rt], dOgB[kt]);
+    s16x8_t km[2][NKT];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) km[kt][rt] = lds_kmajor_perm(sK + 16 * rt, L::LD, 32 * kt, lane);
+    s16x8_t ZB[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      float fa[4], fb[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        fa[j] = bb[2 * kt][j] * exp_fast(gg[2 * kt][j]);
+        fb[j] = bb[2 * kt + 1][j] * exp_fast(gg[2 * kt + 1][j]);
+      }
+      ZB[kt] = pack_acc_pair_scaled(Z[2 * kt], fa, Z[2 * kt + 1], fb);
+    }
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) *z_slot(wave, s, rb) = Z[rb];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], km[kt][rt], ZB[kt]);
+    publish(s + 1);
+  }
+  __syncthreads();
+  __syncthreads();
+  if (p.dh0) {
+    float* db = p.dh0 + ((int64_t)n * H + h) * D * D + col0;
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt) store_acc_global<float>(db, D, dS[rt], 16 * rt, 0, D, lane);
+  }
+}
+
+template <int D, bool PACK>
+int launch_state_bwd_split(const BwdParams& p, hipStream_t s) {
+  auto kern = state_pass_workgroups(p.geom, p.H, D / 32) <= kDeferHead ? chunk_state_bwd_split_kernel<D, 32, PACK, true>
+                                                                       : chunk_state_bwd_split_kernel<D, 32, PACK, false>;
+  constexpr int bytes = RrSplitBwdLayout<D, 32>::bytes;
+  if (int st = set_smem(kern, bytes)) return st;
+  hipLaunchKernelGGL(kern, doc_grid(p.geom.num_seqs, p.H, D / 32), dim3(64 * (4 + kSplitLoaders)), bytes, s, p);
+  return launch_status("pkda_chunk_bwd(state)");
+}
+
 template <int D, int BV, bool ALIAS, bool PACK = false>
 int launch_state_bwd_rr_as(const BwdParams& p, hipStream_t s) {
   auto kern = chunk_state_bwd_rr_kernel<D, BV, ALIAS, PACK>;
@@ -2139,10 +2481,9 @@ int launch_state_bwd_rr(const BwdParams& p, hipStream_t s) {
   const int N = p.geom.num_seqs;
   if (N <= 0) return 0;
   const bool narrow = (int64_t)N * p.H * (D / 64) < 256;
-  if (p.tri_packed) {  // kw = k (checked at the entry point)
-    return narrow ? launch_state_bwd_rr_as<D, 32, true, true>(p, s) : launch_state_bwd_rr_as<D, 64, true, true>(p, s);
-  }
-  if (narrow) return p.kw_is_k ? launch_state_bwd_rr_as<D, 32, true>(p, s) : launch_state_bwd_rr_as<D, 32, false>(p, s);
+  if (p.tri_packed)  // kw = k (checked at the entry point)
+    return narrow ? launch_state_bwd_split<D, true>(p, s) : launch_state_bwd_rr_as<D, 64, true, true>(p, s);
+  if (narrow) return p.kw_is_k ? launch_state_bwd_split<D, false>(p, s) : launch_state_bwd_rr_as<D, 32, false>(p, s);
   return p.kw_is_k ? launch_state_bwd_rr_as<D, 64, true>(p, s) : launch_state_bwd_rr_as<D, 64, false>(p, s);
 }
 
@@ -2368,13 +2709,217 @@ __global__ __launch_bounds__(64 * (BV / 16 + kRrLoadersBwd)) void chunk_state_bw
   }
 }
 
+// The per-channel form with its outputs on waves of their own
+// (chunk_state_bwd_split_kernel's division, for the same calls).  The stage
+// leaves no room for an output stage: the output waves store the dU rows.
 template <int D, int BV>
-int launch_state_bwd_rr_pc_as(const BwdParams& p, hipStream_t s) {
-  auto kern = chunk_state_bwd_rr_pc_kernel<D, BV>;
-  constexpr int bytes = RrPcBwdLayout<D, BV>::bytes;
-  if (int st = set_smem(kern, bytes)) return st;
-  hipLaunchKernelGGL(kern, doc_grid(p.geom.num_seqs, p.H, D / BV), dim3(64 * (BV / 16 + kRrLoadersBwd)), bytes, s, p);
-  return launch_status("pkda_chunk_bwd(state)");
+struct RrPcSplitBwdLayout : RrPcBwdLayout<D, BV> {
+  using Base = RrPcBwdLayout<D, BV>;
+  static constexpr int NC = BV / 16;
+  static constexpr int SB = NC * (D / 32) * 1024;
+  static constexpr int UB = NC * 2 * 1024;  // dU as B operands (negated)
+  static constexpr int off_SB = 2 * Base::BUF;
+  static constexpr int off_UB = off_SB + 2 * SB;
+  static constexpr int bytes = off_UB + 2 * UB;
+  static_assert(bytes <= 160 * 1024, "LDS of one compute unit");
+};
+
+template <int D, int BV>
+__global__ __launch_bounds__(64 * (2 * (BV / 16) + kSplitLoaders))
+__attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_state_bwd_split_pc_kernel(BwdParams p) {
+  using L = RrPcSplitBwdLayout<D, BV>;
+  using T = bf16_t;
+  constexpr int NC = BV / 16;
+  constexpr int NKT = D / 16;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const DocSlot ds = doc_slot(p.geom, p.H, D / BV);
+  const int n = ds.n, h = ds.h, v0 = ds.z * BV;
+  const int H = p.H;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int64_t gs = (int64_t)H * D;
+  int first, count, dstart, dlen;
+  doc_chunks(p.geom, n, first, count, dstart, dlen);
+  const int q4 = 4 * (lane >> 4), il = lane & 15;
+  auto sb_slot = [&](int w, int s, int kk) {
+    return reinterpret_cast<uint4*>(smem + L::off_SB + (s & 1) * L::SB + (w * (NKT / 2) + kk) * 1024) + lane;
+  };
+  auto ub_slot = [&](int w, int s, int kt) {
+    return reinterpret_cast<uint4*>(smem + L::off_UB + (s & 1) * L::UB + (w * 2 + kt) * 1024) + lane;
+  };
+
+  // visits s take chunks jc = count - 1 - s; steps 0 .. count, a barrier before
+  // each: the chain takes visit s in step s, its rows leave in step s + 1
+  if (wave >= 2 * NC) {
+    constexpr int NGT = 128;        // threads of one loader group
+    static_assert(D <= NGT, "one loader thread per gate channel");
+    const int ltid = tid - 64 * 2 * NC;
+    const int lgroup = ltid / NGT;  // takes visits s with s % 2 == lgroup
+    const int lt = ltid % NGT;
+    RegTile<NGT, C, D, T> rQ, rK, rW;
+    RegTile<NGT, C, C, T> rA;
+    RegTile<NGT, C, BV, T> rdO;
+    float re = 0.f;
+    auto load = [&](int s) {
+      const int jc = count - 1 - s;
+      const int cstart = dstart + jc * C;
+      const int clen = min(C, dlen - jc * C);
+      const int64_t row0 = (int64_t)cstart * H + h;
+      rQ.load_as(lt, static_cast<const T*>(p.qg) + row0 * D, gs, clen);
+      rK.load_as(lt, static_cast<const T*>(p.kg) + row0 * D, gs, clen);
+      rW.load_as(lt, static_cast<const T*>(p.w) + row0 * D, gs, clen);
+      rA.load_as(lt, static_cast<const T*>(p.aqk) + row0 * C, (int64_t)H * C, clen);
+      rdO.load_as(lt, static_cast<const T*>(p.dO) + row0 * D + v0, gs, clen);
+      if (lt < D) re = p.gcum[((int64_t)(cstart + clen - 1) * H + h) * D + lt];
+    };
+    auto stash = [&](int b) {
+      char* buf = smem + b * L::BUF;
+      rQ.store_as(lt, reinterpret_cast<T*>(buf + L::off_Q), L::LD);
+      rK.store_as(lt, reinterpret_cast<T*>(buf + L::off_KG), L::LD);
+      rW.store_as(lt, reinterpret_cast<T*>(buf + L::off_W), L::LD);
+      rA.store_as(lt, reinterpret_cast<T*>(buf + L::off_A), L::LDC);
+      rdO.store_as(lt, reinterpret_cast<T*>(buf + L::off_dO), L::LDV);
+      if (lt < D) reinterpret_cast<float*>(buf + L::off_E)[lt] = exp_fast(re);
+    };
+    if (lgroup < count) load(lgroup);
+    if (lgroup == 0 && count > 0) {
+      stash(0);
+    }
+    for (int s = 0; s <= count; ++s) {  // the loads deferred (pkda_chunk_common.h)
+      __syncthreads();
+      if (((s + 1) & 1) == lgroup) {
+        if (s + 1 < count) stash((s + 1) & 1);
+      } else if (s + 2 < count) {
+        load(s + 2);
+      }
+    }
+    return;
+  }
+
+  if (wave >= NC) {  // output waves
+    const int w = wave - NC;  // the chain wave whose columns these are
+    const int col0 = v0 + 16 * w;
+    for (int s = 0; s <= count; ++s) {
+      __syncthreads();
+      if (s >= 1) {  // visit s - 1: the dU rows (the operand holds -dU: flip the signs back)
+        const int jc = count - s;
+        const int clen = min(C, dlen - jc * C);
+        T* du_out = static_cast<T*>(p.du) + ((int64_t)(dstart + jc * C) * H + h) * D + col0;
+        constexpr uint32_t kSigns = 0x80008000u;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+          const uint4 u = *ub_slot(w, s - 1, kt);
+          store_packed_rows(du_out, gs, u.x ^ kSigns, u.y ^ kSigns, 32 * kt, 0, clen, lane);
+          store_packed_rows(du_out, gs, u.z ^ kSigns, u.w ^ kSigns, 32 * kt + 16, 0, clen, lane);
+        }
+      }
+      if (s < count) {  // visit s: the checkpoint
+        T* hb = static_cast<T*>(p.dh) + ((int64_t)(first + count - 1 - s) * H + h) * D * D;
+#pragma unroll
+        for (int kk = 0; kk < NKT / 2; ++kk) {
+          const uint4 x = *sb_slot(w, s, kk);
+          store_packed_tile_nt(hb + tile_offset(D, 2 * kk, col0 / 16), x.x, x.y, lane);
+          store_packed_tile_nt(hb + tile_offset(D, 2 * kk + 1, col0 / 16), x.z, x.w, lane);
+        }
+      }
+    }
+    return;
+  }
+
+  const int col0 = v0 + 16 * wave;
+  f32x4 dS[NKT];
+  s16x8_t dSB[NKT / 2];  // dS as B operands
+#pragma unroll
+  for (int rt = 0; rt < NKT; ++rt)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      dS[rt][j] = p.dht ? p.dht[(((int64_t)n * H + h) * D + 16 * rt + q4 + j) * D + col0 + il] : 0.f;
+  auto publish = [&](int s) {  // dS entering visit s
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk) {
+      dSB[kk] = pack_acc_pair(dS[2 * kk], dS[2 * kk + 1]);
+      *sb_slot(wave, s, kk) = __builtin_bit_cast(uint4, dSB[kk]);
+    }
+  };
+  publish(0);
+  for (int s = 0; s < count; ++s) {
+    __syncthreads();
+    const char* buf = smem + (s & 1) * L::BUF;
+    const T* sQ = reinterpret_cast<const T*>(buf + L::off_Q);
+    const T* sK = reinterpret_cast<const T*>(buf + L::off_KG);
+    const T* sW = reinterpret_cast<const T*>(buf + L::off_W);
+    const T* sA = reinterpret_cast<const T*>(buf + L::off_A);
+    const T* sdO = reinterpret_cast<const T*>(buf + L::off_dO);
+    const float* sE = reinterpret_cast<const float*>(buf + L::off_E);
+    // the LDS reads ahead of what waits for them (as in the forward's chain)
+    s16x8_t ak[NKT / 2][4];
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) ak[kk][rb] = lds_a_perm(sK + 16 * rb * L::LD, L::LD, 32 * kk, lane);
+    // dO of this wave's columns as B operands over the tokens
+    const s16x8_t dOB[2] = {lds_kmajor_perm(sdO + 16 * wave, L::LDV, 0, lane),
+                            lds_kmajor_perm(sdO + 16 * wave, L::LDV, 32, lane)};
+    s16x8_t aa[6];  // Aqk^T row block rb needs k steps kt >= rb / 2
+    aa[0] = lds_kmajor_perm(sA + 0, L::LDC, 0, lane);
+    aa[1] = lds_kmajor_perm(sA + 0, L::LDC, 32, lane);
+    aa[2] = lds_kmajor_perm(sA + 16, L::LDC, 0, lane);
+    aa[3] = lds_kmajor_perm(sA + 16, L::LDC, 32, lane);
+    aa[4] = lds_kmajor_perm(sA + 32, L::LDC, 32, lane);
+    aa[5] = lds_kmajor_perm(sA + 48, L::LDC, 32, lane);
+    float ee[NKT][4];
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt) lds4(sE + 16 * rt + q4, ee[rt]);
+    __builtin_amdgcn_sched_barrier(0);
+    // dU = kg dS + Aqk^T dO
+    f32x4 dU[4];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) dU[rb] = zero4();
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) mfma_bf16(dU[rb], ak[kk][rb], dSB[kk]);
+    mfma_bf16(dU[0], aa[0], dOB[0]);
+    mfma_bf16(dU[1], aa[2], dOB[0]);
+    mfma_bf16(dU[0], aa[1], dOB[1]);
+    mfma_bf16(dU[1], aa[3], dOB[1]);
+    mfma_bf16(dU[2], aa[4], dOB[1]);
+    mfma_bf16(dU[3], aa[5], dOB[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    s16x8_t kq[2][NKT];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) kq[kt][rt] = lds_kmajor_perm(sQ + 16 * rt, L::LD, 32 * kt, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    // dS <- diag(e^{G_C}) dS + qg^T dO - W^T dU
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dS[rt][j] *= ee[rt][j];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], kq[kt][rt], dOB[kt]);
+    const s16x8_t dUnB[2] = {pack_acc_pair(-dU[0], -dU[1]), pack_acc_pair(-dU[2], -dU[3])};
+    s16x8_t km[2][NKT];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) km[kt][rt] = lds_kmajor_perm(sW + 16 * rt, L::LD, 32 * kt, lane);
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) *ub_slot(wave, s, kt) = __builtin_bit_cast(uint4, dUnB[kt]);
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], km[kt][rt], dUnB[kt]);
+    publish(s + 1);
+  }
+  __syncthreads();
+  if (p.dh0) {
+    float* db = p.dh0 + ((int64_t)n * H + h) * D * D + col0;
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt) store_acc_global<float>(db, D, dS[rt], 16 * rt, 0, D, lane);
+  }
 }
 
 template <int D>
@@ -2382,7 +2927,17 @@ int launch_state_bwd_rr_pc(const BwdParams& p, hipStream_t s) {
   const int N = p.geom.num_seqs;
   if (N <= 0) return 0;
   const bool narrow = (int64_t)N * p.H * (D / 64) < 256;
-  return narrow ? launch_state_bwd_rr_pc_as<D, 32>(p, s) : launch_state_bwd_rr_pc_as<D, 64>(p, s);
+  const bool split = narrow && state_pass_workgroups(p.geom, p.H, D / 32) <= kSplitChannelReverse;
+  auto kern = split    ? chunk_state_bwd_split_pc_kernel<D, 32>
+              : narrow ? chunk_state_bwd_rr_pc_kernel<D, 32>
+                       : chunk_state_bwd_rr_pc_kernel<D, 64>;
+  const int bytes = split    ? RrPcSplitBwdLayout<D, 32>::bytes
+                    : narrow ? RrPcBwdLayout<D, 32>::bytes
+                             : RrPcBwdLayout<D, 64>::bytes;
+  const int waves = split ? 4 + kSplitLoaders : (narrow ? 2 : 4) + kRrLoadersBwd;
+  if (int st = set_smem(kern, bytes)) return st;
+  hipLaunchKernelGGL(kern, doc_grid(N, p.H, D / (narrow ? 32 : 64)), dim3(64 * waves), bytes, s, p);
+  return launch_status("pkda_chunk_bwd(state)");
 }
 
 template <typename T, int D, int BV, typename OT, typename OK>

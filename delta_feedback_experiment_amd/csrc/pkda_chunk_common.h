@@ -949,4 +949,31 @@ __device__ __forceinline__ void mfma_bf16(f32x4& acc, const s16x8_t& a, const s1
                                                 0, 0, 0);
 }
 
+// ----------------------------------------------------------------------------
+// The state passes whose outputs have waves of their own (32 value columns a
+// workgroup, for calls that leave compute units idle).
+// ----------------------------------------------------------------------------
+constexpr int kSplitLoaders = 4;  // two groups of two waves
+
+// Whether a loader group sends its next loads in the step after the one in
+// which it staged a chunk (DEFER), not right behind the staging.  Staging takes
+// a group 2,450 cycles of a step and sending 2,020, so both in a row hold the
+// barrier up past the chain's 3,500; deferred, the loads are in flight for one
+// step instead of two, which covers their latency until most compute units
+// stream.  Measured, us: the form without output waves / split, not deferred /
+// split, deferred, at D = 128 and 32 chunks a row unless noted:
+//   workgroups             64                 128              192              224
+//   per head, forward      80.5 61.2 53.6     80.2 61.0 53.8   81.0 62.6 61.4   81.1 63.5 63.5
+//   per head, reverse      71.0 61.8 60.5     71.0 61.9 60.5   70.8 62.6 61.0   71.3 62.9 61.5
+//   per channel, forward   59.8 60.1 50.8     61.6 61.5 65.1   90.6 83.2 93.9   102.9 102.5 115
+//   per channel, reverse   56.8 56.0 45.5     57.7 57.8 54.7   60.0 60.1 61.0   61.1 63.2 64.6
+// 256 workgroups of 256 chunks, per head: forward 606 568 703, reverse 561 512
+// 642.  One prompt of 24 chunks, 32 workgroups, per channel: forward 46.4 47.8 37.4.
+// So per head the split form always, deferred to kDeferHead; per channel forward
+// the same to kDeferChannel; per channel reverse split (deferred) to
+// kSplitChannelReverse and the form without output waves past it, where the
+// output stage it has room for is worth more than the shorter chain.
+constexpr int kDeferHead = 192, kDeferChannel = 112, kSplitChannelReverse = 128;
+inline int64_t state_pass_workgroups(const ChunkGeom& g, int H, int slices) { return (int64_t)g.num_seqs * H * slices; }
+
 }  // namespace pkda

@@ -1449,6 +1449,341 @@ __global__ __launch_bounds__(64 * (BV / 16 + kRrLoaders)) void chunk_state_fwd_r
 }
 
 // ---------------------------------------------------------------------------
+// The same pass with the chunk's outputs on waves of their own, for calls whose
+// (document, head, 32 columns) workgroups leave compute units idle.  There the
+// serial chain S -> K S -> Y -> U -> S of each chunk is the time, and in the
+// form above one wave runs everything else between its links as well: Q S,
+// Aqk U, the gate factors of O, the checkpoint and the output rows.  Here
+// BV / 16 chain waves keep S and do only the chain; they leave the entering
+// state and U as B operands, lane for lane, in LDS, and BV / 16 output waves
+// take Q S from the first in the same step and Aqk U from the second in the
+// next one (Aqk's operands wait in registers), store the checkpoint and write
+// the U and O rows to the output stage.  Every value is formed by the same
+// operations in the same order as above.
+// ---------------------------------------------------------------------------
+// When a loader group sends its next loads.  Right after it staged a chunk
+// they are in flight for two steps, but the group then holds the barrier up
+// (staging 2,450 cycles, sending 2,020, against 3,500 of the chain); in the
+// following step, its idle one, they are in flight for one.  One step covers the
+// latency while other compute units leave the memory idle, not when all stream.
+template <int D, int BV>
+struct RrSplitLayout : RrFwdLayout<D, BV, true> {
+  using Base = RrFwdLayout<D, BV, true>;
+  static constexpr int NC = BV / 16;
+  static constexpr int SB = NC * (D / 32) * 1024;  // entering states as B operands, one 16-byte piece a lane
+  static constexpr int UB = NC * 2 * 1024;         // U as B operands
+  static constexpr int off_SB = 2 * Base::BUF;
+  static constexpr int off_UB = off_SB + 2 * SB;
+  static constexpr int off_Out = off_UB + 2 * UB;
+  static constexpr int bytes = off_Out + 2 * Base::OUT;
+  static_assert(bytes <= 160 * 1024, "LDS of one compute unit");
+};
+
+template <int D, int BV, bool PACK, bool DEFER>
+__global__ __launch_bounds__(64 * (2 * (BV / 16) + kSplitLoaders))
+__attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_state_fwd_split_kernel(FwdParams p) {
+  using L = RrSplitLayout<D, BV>;
+  using T = bf16_t;
+  constexpr int NC = BV / 16;           // chain waves, and as many output waves
+  constexpr int NKT = D / 16;           // 16-row tiles of the state slice
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const DocSlot ds = doc_slot(p.geom, p.H, D / BV);
+  const int n = ds.n, h = ds.h, v0 = ds.z * BV;
+  const int H = p.H;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int64_t gs = (int64_t)H * D;
+  int first, count, dstart, dlen;
+  doc_chunks(p.geom, n, first, count, dstart, dlen);
+  const int q4 = 4 * (lane >> 4), il = lane & 15;
+  auto sb_slot = [&](int w, int jc, int kk) {
+    return reinterpret_cast<uint4*>(smem + L::off_SB + (jc & 1) * L::SB + (w * (NKT / 2) + kk) * 1024) + lane;
+  };
+  auto ub_slot = [&](int w, int jc, int kt) {
+    return reinterpret_cast<uint4*>(smem + L::off_UB + (jc & 1) * L::UB + (w * 2 + kt) * 1024) + lane;
+  };
+
+  // Steps 0 .. count + 1, a barrier before each: the chain takes chunk jc in
+  // step jc, its rows reach the output stage by the end of step jc + 1 and
+  // global memory in step jc + 2.
+  if (wave >= 2 * NC) {
+    constexpr int NGT = 128;      // threads of one loader group
+    const int ltid = tid - 64 * 2 * NC;
+    const int lgroup = ltid / NGT;  // takes chunks jc with jc % 2 == lgroup
+    const int lt = ltid % NGT;
+    RegTile<NGT, C, D, T> rQ, rKW;
+    std::conditional_t<PACK, TriRegTile<NGT>, RegTile<NGT, C, C, T>> rA, rT;
+    RegTile<NGT, C, BV, T> rV;
+    float rg = 0.f, rb = 0.f;
+    if constexpr (PACK) {  // the stages' blocks above the diagonal: zero once
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        zero_upper_blocks<64 * kSplitLoaders>(ltid, reinterpret_cast<T*>(smem + b * L::BUF + L::off_A), L::LDC);
+        zero_upper_blocks<64 * kSplitLoaders>(ltid, reinterpret_cast<T*>(smem + b * L::BUF + L::off_T), L::LDC);
+      }
+    }
+    auto load = [&](int jc) {
+      const int cstart = dstart + jc * C;
+      const int clen = min(C, dlen - jc * C);
+      const int64_t row0 = (int64_t)cstart * H + h;
+      rQ.load_as(lt, static_cast<const T*>(p.q) + row0 * D, gs, clen);
+      rKW.load_as(lt, static_cast<const T*>(p.kw) + row0 * D, gs, clen);
+      if constexpr (PACK) {
+        const int64_t tri0 = ((int64_t)(first + jc) * H + h) * kTriElems;
+        rA.load_as(lt, static_cast<const T*>(p.aqk) + tri0);
+        rT.load_as(lt, static_cast<const T*>(p.akk) + tri0);
+      } else {
+        rA.load_as(lt, static_cast<const T*>(p.aqk) + row0 * C, (int64_t)H * C, clen);
+        rT.load_as(lt, static_cast<const T*>(p.akk) + row0 * C, (int64_t)H * C, clen);
+      }
+      rV.load_as(lt, static_cast<const T*>(p.v) + row0 * D + v0, gs, clen);
+      if (lt < C) {
+        const int64_t gi = (int64_t)(cstart + min(lt, clen - 1)) * H + h;
+        rg = p.gcum[gi];  // padded rows repeat the last gate
+        rb = lt < clen ? p.beta[gi] : 0.f;
+      }
+    };
+    auto stash = [&](int b) {
+      char* buf = smem + b * L::BUF;
+      rQ.store_as(lt, reinterpret_cast<T*>(buf + L::off_Q), L::LD);
+      rKW.store_as(lt, reinterpret_cast<T*>(buf + L::off_KW), L::LD);
+      rA.store_as(lt, reinterpret_cast<T*>(buf + L::off_A), L::LDC);
+      rT.store_as(lt, reinterpret_cast<T*>(buf + L::off_T), L::LDC);
+      rV.store_as(lt, reinterpret_cast<T*>(buf + L::off_V), L::LDV);
+      if (lt < C) {
+        reinterpret_cast<float*>(buf + L::off_G)[lt] = rg;
+        reinterpret_cast<float*>(buf + L::off_B)[lt] = rb;
+      }
+    };
+    // chunk jc's U and O rows from the output stage to global memory
+    auto flush = [&](int jc) {
+      constexpr int SEG = BV / 8;  // 16-byte pieces of a row
+      const T* so = reinterpret_cast<const T*>(smem + L::off_Out + (jc & 1) * L::OUT);
+      const int clen = min(C, dlen - jc * C);
+      const int64_t row0 = (int64_t)(dstart + jc * C) * H + h;
+      static_assert(2 * C * SEG % NGT == 0, "whole passes over the stage");
+#pragma unroll
+      for (int it = 0; it < 2 * C * SEG / NGT; ++it) {
+        const int i = lt + it * NGT;
+        const int which = i / (C * SEG);
+        const int r = (i - which * C * SEG) / SEG, sg = i % SEG;
+        if (r < clen) {
+          const uint4 x = *reinterpret_cast<const uint4*>(so + (which * C + r) * L::LDV + 8 * sg);
+          T* dst = static_cast<T*>(which ? p.o : p.u) + (row0 + (int64_t)r * H) * D + v0 + 8 * sg;
+          *reinterpret_cast<uint4*>(dst) = x;
+        }
+      }
+    };
+    if (lgroup < count) load(lgroup);
+    if (lgroup == 0 && count > 0) {
+      stash(0);
+      if (!DEFER && count > 2) load(2);
+    }
+    for (int jc = 0; jc < count + 2; ++jc) {
+      __syncthreads();
+      if (((jc + 1) & 1) == lgroup) {
+        if (jc + 1 < count) {
+          stash((jc + 1) & 1);
+          if (!DEFER && jc + 3 < count) load(jc + 3);
+        }
+      } else {
+        if (DEFER && jc + 2 < count) load(jc + 2);
+        if (jc >= 2) flush(jc - 2);
+      }
+    }
+    return;
+  }
+
+  if (wave >= NC) {  // output waves
+    const int w = wave - NC;          // the chain wave whose columns these are
+    const int col0 = v0 + 16 * w;
+    const float scale = p.scale;
+    f32x4 QS[4], og[4];  // Q S and the factors s e^G of its rows
+    s16x8_t aa[6];
+    for (int jc = 0; jc < count + 2; ++jc) {
+      __syncthreads();
+      if (jc >= 1 && jc <= count) {  // chunk jc - 1: U and O = diag(s e^G) Q S + Aqk U
+        const s16x8_t UB[2] = {__builtin_bit_cast(s16x8_t, *ub_slot(w, jc - 1, 0)),
+                               __builtin_bit_cast(s16x8_t, *ub_slot(w, jc - 1, 1))};
+        f32x4 AU[4];
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) {
+          AU[rb] = zero4();
+          mfma_bf16(AU[rb], aa[rb], UB[0]);
+        }
+        mfma_bf16(AU[2], aa[4], UB[1]);
+        mfma_bf16(AU[3], aa[5], UB[1]);
+        T* so = reinterpret_cast<T*>(smem + L::off_Out + ((jc - 1) & 1) * L::OUT) + 16 * w;
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) {
+          const uint4 u = __builtin_bit_cast(uint4, UB[rb / 2]);
+          store_packed_rows<true>(so, L::LDV, rb & 1 ? u.z : u.x, rb & 1 ? u.w : u.y, 16 * rb, 0, C, lane);
+          f32x4 o;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) o[j] = og[rb][j] * QS[rb][j] + AU[rb][j];
+          store_acc_global<T, true>(so + C * L::LDV, L::LDV, o, 16 * rb, 0, C, lane);
+        }
+      }
+      if (jc < count) {  // chunk jc: the checkpoint, Q S, Aqk's operands
+        const char* buf = smem + (jc & 1) * L::BUF;
+        const T* sQ = reinterpret_cast<const T*>(buf + L::off_Q);
+        const T* sA = reinterpret_cast<const T*>(buf + L::off_A);
+        const float* sG = reinterpret_cast<const float*>(buf + L::off_G);
+        s16x8_t SB[NKT / 2];
+#pragma unroll
+        for (int kk = 0; kk < NKT / 2; ++kk) SB[kk] = __builtin_bit_cast(s16x8_t, *sb_slot(w, jc, kk));
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) QS[rb] = zero4();
+        s16x8_t aq[NKT / 2][4];
+#pragma unroll
+        for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+          for (int rb = 0; rb < 4; ++rb) aq[kk][rb] = lds_a_perm(sQ + 16 * rb * L::LD, L::LD, 32 * kk, lane);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+          for (int rb = 0; rb < 4; ++rb) mfma_bf16(QS[rb], aq[kk][rb], SB[kk]);
+        if (p.h) {
+          T* hb = static_cast<T*>(p.h) + ((int64_t)(first + jc) * H + h) * D * D;
+#pragma unroll
+          for (int kk = 0; kk < NKT / 2; ++kk) {
+            const uint4 x = __builtin_bit_cast(uint4, SB[kk]);
+            store_packed_tile_nt(hb + tile_offset(D, 2 * kk, col0 / 16), x.x, x.y, lane);
+            store_packed_tile_nt(hb + tile_offset(D, 2 * kk + 1, col0 / 16), x.z, x.w, lane);
+          }
+        }
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) aa[rb] = lds_a_perm(sA + 16 * rb * L::LDC, L::LDC, 0, lane);
+        aa[4] = lds_a_perm(sA + 32 * L::LDC, L::LDC, 32, lane);
+        aa[5] = lds_a_perm(sA + 48 * L::LDC, L::LDC, 32, lane);
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) og[rb][j] = scale * exp_fast(sG[16 * rb + q4 + j]);
+      }
+    }
+    return;
+  }
+
+  const int col0 = v0 + 16 * wave;  // first column of this wave's block
+  const int col = col0 + il;
+  f32x4 S[NKT];
+  s16x8_t SB[NKT / 2];  // S as B operands
+#pragma unroll
+  for (int rt = 0; rt < NKT; ++rt)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      S[rt][j] = p.s0 ? p.s0[((state_row(p, n) * H + h) * D + 16 * rt + q4 + j) * D + col] : 0.f;
+  auto publish = [&](int jc) {  // the state entering chunk jc
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk) {
+      SB[kk] = pack_acc_pair(S[2 * kk], S[2 * kk + 1]);
+      *sb_slot(wave, jc, kk) = __builtin_bit_cast(uint4, SB[kk]);
+    }
+  };
+  publish(0);
+  for (int jc = 0; jc < count; ++jc) {
+    __syncthreads();
+    const char* buf = smem + (jc & 1) * L::BUF;
+    const T* sK = reinterpret_cast<const T*>(buf + L::off_KW);
+    const T* sT = reinterpret_cast<const T*>(buf + L::off_T);
+    const T* sV = reinterpret_cast<const T*>(buf + L::off_V);
+    const float* sG = reinterpret_cast<const float*>(buf + L::off_G);
+    const float* sB = reinterpret_cast<const float*>(buf + L::off_B);
+    // The LDS reads go out ahead of what waits for them, in this order; left
+    // to itself the scheduler puts each operand's read right before its MFMA
+    // and the chain pays the read's latency sixteen times.
+    s16x8_t ak[NKT / 2][4];
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) ak[kk][rb] = lds_a_perm(sK + 16 * rb * L::LD, L::LD, 32 * kk, lane);
+    s16x4_t vv[4];
+    float gg[4][4], bb[4][4];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) {
+      vv[rb] = lds_read_kmajor4(sV + 16 * wave, L::LDV, 16 * rb, lane);
+      lds4(sG + 16 * rb + q4, gg[rb]);
+      lds4(sB + 16 * rb + q4, bb[rb]);
+    }
+    const float gC = sG[C - 1];
+    s16x8_t at[6];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) at[rb] = lds_a_perm(sT + 16 * rb * L::LDC, L::LDC, 0, lane);
+    at[4] = lds_a_perm(sT + 32 * L::LDC, L::LDC, 32, lane);
+    at[5] = lds_a_perm(sT + 48 * L::LDC, L::LDC, 32, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 KS[4];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) KS[rb] = zero4();
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) mfma_bf16(KS[rb], ak[kk][rb], SB[kk]);
+    __builtin_amdgcn_sched_barrier(0);
+    s16x8_t km[2][NKT];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) km[kt][rt] = lds_kmajor_perm(sK + 16 * rt, L::LD, 32 * kt, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    // Y = diag(beta) (V - diag(e^G) K S) as B operands over the tokens
+    s16x8_t YB[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      f32x4 y[2];
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        const int rb = 2 * kt + hf;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          y[hf][j] = bb[rb][j] * (bf16_to_f32(static_cast<bf16_t>(vv[rb][j])) - exp_fast(gg[rb][j]) * KS[rb][j]);
+      }
+      YB[kt] = pack_acc_pair(y[0], y[1]);
+    }
+    // U = T Y   (T is lower triangular: row block rb needs k steps kt <= rb / 2)
+    f32x4 U[4];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) {
+      U[rb] = zero4();
+      mfma_bf16(U[rb], at[rb], YB[0]);
+    }
+    mfma_bf16(U[2], at[4], YB[1]);
+    mfma_bf16(U[3], at[5], YB[1]);
+    // S <- e^{G_C} S + KW^T diag(e^{G_C - G}) U
+    const float decay = exp_fast(gC);
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt) S[rt] = S[rt] * decay;
+    s16x8_t UgB[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      float fa[4], fb[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        fa[j] = exp_fast(gC - gg[2 * kt][j]);
+        fb[j] = exp_fast(gC - gg[2 * kt + 1][j]);
+      }
+      UgB[kt] = pack_acc_pair_scaled(U[2 * kt], fa, U[2 * kt + 1], fb);
+    }
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) mfma_bf16(S[rt], km[kt][rt], UgB[kt]);
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+      *ub_slot(wave, jc, kt) = __builtin_bit_cast(uint4, pack_acc_pair(U[2 * kt], U[2 * kt + 1]));
+    publish(jc + 1);
+  }
+  __syncthreads();
+  __syncthreads();
+  if (p.sT) {
+    float* sb = p.sT + (state_row(p, n) * H + h) * D * D + col0;
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt) store_acc_global<float>(sb, D, S[rt], 16 * rt, 0, D, lane);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // per-document state pass, BF16 with a per-channel gate: register-resident
 // form.  The structure of chunk_state_fwd_rr_kernel with the intra kernel's
 // W, u, qg = s e^G q and kg = e^{G_last - G} kw as inputs:
@@ -1686,6 +2021,240 @@ __global__ __launch_bounds__(64 * (BV / 16 + kRrLoaders)) void chunk_state_fwd_r
   }
 }
 
+// The per-channel form with its outputs on waves of their own
+// (chunk_state_fwd_split_kernel's division, for the same calls).  The stage
+// leaves no room for an output stage: the output waves store the rows.
+template <int D, int BV>
+struct RrPcSplitLayout : RrPcFwdLayout<D, BV> {
+  using Base = RrPcFwdLayout<D, BV>;
+  static constexpr int NC = BV / 16;
+  static constexpr int SB = NC * (D / 32) * 1024;
+  static constexpr int UB = NC * 2 * 1024;
+  static constexpr int off_SB = 2 * Base::BUF;
+  static constexpr int off_UB = off_SB + 2 * SB;
+  static constexpr int bytes = off_UB + 2 * UB;
+  static_assert(bytes <= 160 * 1024, "LDS of one compute unit");
+};
+
+template <int D, int BV, bool DEFER>
+__global__ __launch_bounds__(64 * (2 * (BV / 16) + kSplitLoaders))
+__attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_state_fwd_split_pc_kernel(FwdParams p) {
+  using L = RrPcSplitLayout<D, BV>;
+  using T = bf16_t;
+  constexpr int NC = BV / 16;   // chain waves, and as many output waves
+  constexpr int NKT = D / 16;   // 16-row tiles of the state slice
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const DocSlot ds = doc_slot(p.geom, p.H, D / BV);
+  const int n = ds.n, h = ds.h, v0 = ds.z * BV;
+  const int H = p.H;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int64_t gs = (int64_t)H * D;
+  int first, count, dstart, dlen;
+  doc_chunks(p.geom, n, first, count, dstart, dlen);
+  const int q4 = 4 * (lane >> 4), il = lane & 15;
+  auto sb_slot = [&](int w, int jc, int kk) {
+    return reinterpret_cast<uint4*>(smem + L::off_SB + (jc & 1) * L::SB + (w * (NKT / 2) + kk) * 1024) + lane;
+  };
+  auto ub_slot = [&](int w, int jc, int kt) {
+    return reinterpret_cast<uint4*>(smem + L::off_UB + (jc & 1) * L::UB + (w * 2 + kt) * 1024) + lane;
+  };
+
+  // steps 0 .. count, a barrier before each: the chain takes chunk jc in step
+  // jc, its rows leave in step jc + 1
+  if (wave >= 2 * NC) {
+    constexpr int NGT = 128;        // threads of one loader group
+    const int ltid = tid - 64 * 2 * NC;
+    const int lgroup = ltid / NGT;  // takes chunks jc with jc % 2 == lgroup
+    const int lt = ltid % NGT;
+    RegTile<NGT, C, D, T> rQ, rW, rK;
+    RegTile<NGT, C, C, T> rA;
+    RegTile<NGT, C, BV, T> rU;
+    float re = 0.f;
+    auto load = [&](int jc) {
+      const int cstart = dstart + jc * C;
+      const int clen = min(C, dlen - jc * C);
+      const int64_t row0 = (int64_t)cstart * H + h;
+      rQ.load_as(lt, static_cast<const T*>(p.qg) + row0 * D, gs, clen);
+      rW.load_as(lt, static_cast<const T*>(p.w) + row0 * D, gs, clen);
+      rK.load_as(lt, static_cast<const T*>(p.kg) + row0 * D, gs, clen);
+      rA.load_as(lt, static_cast<const T*>(p.aqk) + row0 * C, (int64_t)H * C, clen);
+      rU.load_as(lt, static_cast<const T*>(p.u) + row0 * D + v0, gs, clen);
+      if (lt < D) re = p.gcum[((int64_t)(cstart + clen - 1) * H + h) * D + lt];
+    };
+    auto stash = [&](int b) {
+      char* buf = smem + b * L::BUF;
+      rQ.store_as(lt, reinterpret_cast<T*>(buf + L::off_Q), L::LD);
+      rW.store_as(lt, reinterpret_cast<T*>(buf + L::off_W), L::LD);
+      rK.store_as(lt, reinterpret_cast<T*>(buf + L::off_KG), L::LD);
+      rA.store_as(lt, reinterpret_cast<T*>(buf + L::off_A), L::LDC);
+      rU.store_as(lt, reinterpret_cast<T*>(buf + L::off_U), L::LDV);
+      if (lt < D) reinterpret_cast<float*>(buf + L::off_E)[lt] = exp_fast(re);
+    };
+    static_assert(D <= NGT, "one loader thread per gate channel");
+    if (lgroup < count) load(lgroup);
+    if (lgroup == 0 && count > 0) {
+      stash(0);
+      if (!DEFER && count > 2) load(2);
+    }
+    for (int jc = 0; jc <= count; ++jc) {
+      __syncthreads();
+      if (((jc + 1) & 1) == lgroup) {
+        if (jc + 1 < count) {
+          stash((jc + 1) & 1);
+          if (!DEFER && jc + 3 < count) load(jc + 3);
+        }
+      } else if (DEFER && jc + 2 < count) {
+        load(jc + 2);
+      }
+    }
+    return;
+  }
+
+  if (wave >= NC) {  // output waves
+    const int w = wave - NC;          // the chain wave whose columns these are
+    const int col0 = v0 + 16 * w;
+    f32x4 QS[4];
+    s16x8_t aa[6];
+    for (int jc = 0; jc <= count; ++jc) {
+      __syncthreads();
+      if (jc >= 1) {  // chunk jc - 1: U and O = qg S + Aqk U
+        const s16x8_t UB[2] = {__builtin_bit_cast(s16x8_t, *ub_slot(w, jc - 1, 0)),
+                               __builtin_bit_cast(s16x8_t, *ub_slot(w, jc - 1, 1))};
+        f32x4 AU[4];
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) {
+          AU[rb] = zero4();
+          mfma_bf16(AU[rb], aa[rb], UB[0]);
+        }
+        mfma_bf16(AU[2], aa[4], UB[1]);
+        mfma_bf16(AU[3], aa[5], UB[1]);
+        const int clen = min(C, dlen - (jc - 1) * C);
+        const int64_t row0 = (int64_t)(dstart + (jc - 1) * C) * H + h;
+        T* u_out = static_cast<T*>(p.u) + row0 * D + col0;
+        T* o_out = static_cast<T*>(p.o) + row0 * D + col0;
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) {
+          const uint4 u = __builtin_bit_cast(uint4, UB[rb / 2]);
+          store_packed_rows(u_out, gs, rb & 1 ? u.z : u.x, rb & 1 ? u.w : u.y, 16 * rb, 0, clen, lane);
+          store_acc_global<T>(o_out, gs, QS[rb] + AU[rb], 16 * rb, 0, clen, lane);
+        }
+      }
+      if (jc < count) {  // chunk jc: the checkpoint, qg S, Aqk's operands
+        const char* buf = smem + (jc & 1) * L::BUF;
+        const T* sQ = reinterpret_cast<const T*>(buf + L::off_Q);
+        const T* sA = reinterpret_cast<const T*>(buf + L::off_A);
+        s16x8_t SB[NKT / 2];
+#pragma unroll
+        for (int kk = 0; kk < NKT / 2; ++kk) SB[kk] = __builtin_bit_cast(s16x8_t, *sb_slot(w, jc, kk));
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) QS[rb] = zero4();
+        s16x8_t aq[NKT / 2][4];
+#pragma unroll
+        for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+          for (int rb = 0; rb < 4; ++rb) aq[kk][rb] = lds_a_perm(sQ + 16 * rb * L::LD, L::LD, 32 * kk, lane);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+          for (int rb = 0; rb < 4; ++rb) mfma_bf16(QS[rb], aq[kk][rb], SB[kk]);
+        if (p.h) {
+          T* hb = static_cast<T*>(p.h) + ((int64_t)(first + jc) * H + h) * D * D;
+#pragma unroll
+          for (int kk = 0; kk < NKT / 2; ++kk) {
+            const uint4 x = __builtin_bit_cast(uint4, SB[kk]);
+            store_packed_tile_nt(hb + tile_offset(D, 2 * kk, col0 / 16), x.x, x.y, lane);
+            store_packed_tile_nt(hb + tile_offset(D, 2 * kk + 1, col0 / 16), x.z, x.w, lane);
+          }
+        }
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) aa[rb] = lds_a_perm(sA + 16 * rb * L::LDC, L::LDC, 0, lane);
+        aa[4] = lds_a_perm(sA + 32 * L::LDC, L::LDC, 32, lane);
+        aa[5] = lds_a_perm(sA + 48 * L::LDC, L::LDC, 32, lane);
+      }
+    }
+    return;
+  }
+
+  const int col0 = v0 + 16 * wave;  // first column of this wave's block
+  const int col = col0 + il;
+  f32x4 S[NKT];
+  s16x8_t SB[NKT / 2];  // S as B operands
+#pragma unroll
+  for (int rt = 0; rt < NKT; ++rt)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      S[rt][j] = p.s0 ? p.s0[((state_row(p, n) * H + h) * D + 16 * rt + q4 + j) * D + col] : 0.f;
+  auto publish = [&](int jc) {  // the state entering chunk jc
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk) {
+      SB[kk] = pack_acc_pair(S[2 * kk], S[2 * kk + 1]);
+      *sb_slot(wave, jc, kk) = __builtin_bit_cast(uint4, SB[kk]);
+    }
+  };
+  publish(0);
+  for (int jc = 0; jc < count; ++jc) {
+    __syncthreads();
+    const char* buf = smem + (jc & 1) * L::BUF;
+    const T* sW = reinterpret_cast<const T*>(buf + L::off_W);
+    const T* sK = reinterpret_cast<const T*>(buf + L::off_KG);
+    const T* sU = reinterpret_cast<const T*>(buf + L::off_U);
+    const float* sE = reinterpret_cast<const float*>(buf + L::off_E);
+    // the LDS reads ahead of what waits for them, as in the per-head form
+    s16x8_t aw[NKT / 2][4];
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) aw[kk][rb] = lds_a_perm(sW + 16 * rb * L::LD, L::LD, 32 * kk, lane);
+    s16x4_t uu[4];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) uu[rb] = lds_read_kmajor4(sU + 16 * wave, L::LDV, 16 * rb, lane);
+    float ee[NKT][4];
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt) lds4(sE + 16 * rt + q4, ee[rt]);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 WS[4];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) WS[rb] = zero4();
+#pragma unroll
+    for (int kk = 0; kk < NKT / 2; ++kk)
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) mfma_bf16(WS[rb], aw[kk][rb], SB[kk]);
+    __builtin_amdgcn_sched_barrier(0);
+    s16x8_t km[2][NKT];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) km[kt][rt] = lds_kmajor_perm(sK + 16 * rt, L::LD, 32 * kt, lane);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) S[rt][j] *= ee[rt][j];
+    // U = u - W S
+    f32x4 U[4];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) U[rb][j] = bf16_to_f32(static_cast<bf16_t>(uu[rb][j])) - WS[rb][j];
+    const s16x8_t UB[2] = {pack_acc_pair(U[0], U[1]), pack_acc_pair(U[2], U[3])};
+    // S <- diag(e^{G_C}) S + kg^T U
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rt = 0; rt < NKT; ++rt) mfma_bf16(S[rt], km[kt][rt], UB[kt]);
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) *ub_slot(wave, jc, kt) = __builtin_bit_cast(uint4, UB[kt]);
+    publish(jc + 1);
+  }
+  __syncthreads();
+  if (p.sT) {
+    float* sb = p.sT + (state_row(p, n) * H + h) * D * D + col0;
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt) store_acc_global<float>(sb, D, S[rt], 16 * rt, 0, D, lane);
+  }
+}
+
 template <typename K>
 int set_smem(K kernel, int bytes) {
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -1706,6 +2275,16 @@ int launch_state_fwd_rr_as(const FwdParams& p, hipStream_t s) {
   return launch_status("pkda_chunk_fwd(state)");
 }
 
+template <int D, bool PACK>
+int launch_state_fwd_split(const FwdParams& p, hipStream_t s) {
+  auto kern = state_pass_workgroups(p.geom, p.H, D / 32) <= kDeferHead ? chunk_state_fwd_split_kernel<D, 32, PACK, true>
+                                                                       : chunk_state_fwd_split_kernel<D, 32, PACK, false>;
+  constexpr int bytes = RrSplitLayout<D, 32>::bytes;
+  if (int st = set_smem(kern, bytes)) return st;
+  hipLaunchKernelGGL(kern, doc_grid(p.geom.num_seqs, p.H, D / 32), dim3(64 * (4 + kSplitLoaders)), bytes, s, p);
+  return launch_status("pkda_chunk_fwd(state)");
+}
+
 // Register-resident state pass: 64 value columns per workgroup, or 32 when
 // that leaves fewer workgroups than compute units.
 template <int D>
@@ -1714,20 +2293,10 @@ int launch_state_fwd_rr(const FwdParams& p, hipStream_t s) {
   if (N <= 0) return 0;
   const bool narrow = (int64_t)N * p.H * (D / 64) < 256;
   const bool alias = p.kw == p.k;
-  if (p.tri_packed) {  // kw = k (checked at the entry point)
-    return narrow ? launch_state_fwd_rr_as<D, 32, true, true>(p, s) : launch_state_fwd_rr_as<D, 64, true, true>(p, s);
-  }
-  if (narrow) return alias ? launch_state_fwd_rr_as<D, 32, true>(p, s) : launch_state_fwd_rr_as<D, 32, false>(p, s);
+  if (p.tri_packed)  // kw = k (checked at the entry point)
+    return narrow ? launch_state_fwd_split<D, true>(p, s) : launch_state_fwd_rr_as<D, 64, true, true>(p, s);
+  if (narrow) return alias ? launch_state_fwd_split<D, false>(p, s) : launch_state_fwd_rr_as<D, 32, false>(p, s);
   return alias ? launch_state_fwd_rr_as<D, 64, true>(p, s) : launch_state_fwd_rr_as<D, 64, false>(p, s);
-}
-
-template <int D, int BV>
-int launch_state_fwd_rr_pc_as(const FwdParams& p, hipStream_t s) {
-  auto kern = chunk_state_fwd_rr_pc_kernel<D, BV>;
-  constexpr int bytes = RrPcFwdLayout<D, BV>::bytes;
-  if (int st = set_smem(kern, bytes)) return st;
-  hipLaunchKernelGGL(kern, doc_grid(p.geom.num_seqs, p.H, D / BV), dim3(64 * (BV / 16 + kRrLoaders)), bytes, s, p);
-  return launch_status("pkda_chunk_fwd(state)");
 }
 
 template <int D>
@@ -1735,7 +2304,13 @@ int launch_state_fwd_rr_pc(const FwdParams& p, hipStream_t s) {
   const int N = p.geom.num_seqs;
   if (N <= 0) return 0;
   const bool narrow = (int64_t)N * p.H * (D / 64) < 256;
-  return narrow ? launch_state_fwd_rr_pc_as<D, 32>(p, s) : launch_state_fwd_rr_pc_as<D, 64>(p, s);
+  auto kern = !narrow                                                   ? chunk_state_fwd_rr_pc_kernel<D, 64>
+              : state_pass_workgroups(p.geom, p.H, D / 32) <= kDeferChannel ? chunk_state_fwd_split_pc_kernel<D, 32, true>
+                                                                        : chunk_state_fwd_split_pc_kernel<D, 32, false>;
+  const int bytes = narrow ? RrPcSplitLayout<D, 32>::bytes : RrPcFwdLayout<D, 64>::bytes;
+  if (int st = set_smem(kern, bytes)) return st;
+  hipLaunchKernelGGL(kern, doc_grid(N, p.H, D / (narrow ? 32 : 64)), dim3(64 * (4 + (narrow ? kSplitLoaders : kRrLoaders))), bytes, s, p);
+  return launch_status("pkda_chunk_fwd(state)");
 }
 
 template <typename T, int D, int BV>

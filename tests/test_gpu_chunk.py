@@ -775,3 +775,46 @@ def test_pkda_recurrence_overlap_same_bits(dev, lean, monkeypatch):
     for a, b in zip(step(), in_order):
         assert torch.equal(a, b)
     test_pkda_recurrence_graph_replays_match_eager(dev, lean)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("per_channel", [False, True])
+def test_state_pass_forms_agree(dev, D, per_channel):
+    """The state passes with 64 columns a workgroup (320 rows x heads), and
+    those whose outputs have waves of their own in each of their dispatches:
+    rows x heads 56 (at D = 128 224 workgroups: loads not deferred, the
+    per-channel reverse pass without output waves), 30 (120) and 14 (56: all
+    deferred).  Rows of 150 tokens (two whole chunks and a partial one) and of
+    one; initial and final states.  The forward forms every value by the same
+    operations, so outputs and states agree bit for bit; the reverse pass adds
+    Q^T dO before K^T Z, so gradients agree to a BF16 ulp's flips."""
+    from delta_feedback_experiment_amd import chunk_pkda
+
+    print(f"[gpu] state pass forms D={D} per_channel={per_channel}", flush=True)
+    gen = torch.Generator(device=dev).manual_seed(D + per_channel)
+
+    def rn(*s):
+        return torch.randn(*s, generator=gen, device=dev)
+
+    for T in (150, 1):
+        B, H = 20, 16
+        q, k = (torch.nn.functional.normalize(rn(B, T, H, D), dim=-1).to(torch.bfloat16) for _ in range(2))
+        v, do = rn(B, T, H, D).to(torch.bfloat16), rn(B, T, H, D).to(torch.bfloat16)
+        g = -torch.nn.functional.softplus(rn(B, T, H, D) if per_channel else rn(B, T, H))
+        beta, s0, dS = torch.sigmoid(rn(B, T, H)), 0.1 * rn(B, H, D, D), 0.1 * rn(B, H, D, D)
+
+        def step(rows, heads):
+            cut = [t[:rows, :, :heads].contiguous().requires_grad_() for t in (q, k, v, g, beta)]
+            cut.append(s0[:rows, :heads].contiguous().requires_grad_())
+            o, S, _ = chunk_pkda(*cut[:5], initial_state=cut[5], output_final_state=True)
+            gr = torch.autograd.grad([o, S], cut, [do[:rows, :, :heads], dS[:rows, :heads]])
+            return [o.detach(), *gr[:5]], [S.detach(), gr[5]]
+
+        wide = step(B, H)
+        for rows, heads in ((4, 14), (3, 10), (1, 14)):
+            tokens, states = step(rows, heads)
+            want = ([t[:rows, :, :heads] for t in wide[0]], [t[:rows, :heads] for t in wide[1]])
+            assert torch.equal(tokens[0], want[0][0]) and torch.equal(states[0], want[1][0]), (T, rows)
+            for name, a, b in zip(("dq", "dk", "dv", "dg", "dbeta", "dS0"), (*tokens[1:], states[1]),
+                                  (*want[0][1:], want[1][1])):
+                assert rel_l2(a.float(), b.float()) < 2 ** -9, (T, rows, name)

@@ -135,6 +135,24 @@ def gate_forward(plan: ChunkPlan, g: Tensor, kind: int, A_log: Tensor | None, dt
     return gcum
 
 
+def fuses_gate(kind: int, g: Tensor, k: Tensor, precond: bool) -> bool:
+    """Whether the preconditioner's local pass takes the gate along: a raw
+    per-channel gate in the key's dtype, BF16 (FP32 also wants the cumsum's
+    remainder, which the gate's own kernel forms), whose two channels a lane
+    come in one aligned load."""
+    return precond and kind == _lib.GATE_RAW_CHANNEL and g.dtype == k.dtype == torch.bfloat16 and not g.data_ptr() % 4
+
+
+def gate_or_fused(plan: ChunkPlan, kf: Tensor, gf: Tensor, kind: int, A_log: Tensor | None, dt_bias: Tensor | None,
+                  up_weight: Tensor | None, gcum_lo: Tensor | None, precond: bool) -> tuple[Tensor, tuple | None]:
+    """The gate's chunk cumsum by its own kernel, or its buffer and the ``gate``
+    argument with which ``precond_forward`` fills it (:func:`fuses_gate`)."""
+    if not fuses_gate(kind, gf, kf, precond):
+        return gate_forward(plan, gf, kind, A_log, dt_bias, up_weight, gcum_lo=gcum_lo), None
+    gcum = torch.empty(kf.shape, device=kf.device, dtype=torch.float32)
+    return gcum, (gf, A_log, dt_bias, gcum)
+
+
 def low_rank_rows(hidden: Tensor, num_tokens: int) -> Tensor:
     """The decay hidden ``[..., R]`` as ``[N_tok, R]`` rows the gate kernels
     read with 16-byte loads: a view when its rows are evenly strided and
@@ -365,12 +383,12 @@ class _ChunkPKDA(torch.autograd.Function):
         if wants_gcum_lo(kind, q.dtype):
             shp = (plan.num_tokens, plan.heads, plan.head_dim)
             gcum_lo = torch.empty(shp, device=q.device, dtype=torch.float32)
-        gcum = gate_forward(plan, _flat(g_used, plan), kind, A_log32, dt32, decay_up, gcum_lo=gcum_lo)
         precond = g_atk is not None
+        gcum, gate = gate_or_fused(plan, kf, _flat(g_used, plan), kind, A_log32, dt32, decay_up, gcum_lo, precond)
         needs_grad = any(ctx.needs_input_grad)
         if precond:
             pstate = pre.precond_forward(plan, kf, g_atk, beta_atk, log_atk_scale, x, eps, initial_A_state,
-                                         want_kw32=needs_grad and gcum.dim() == 3)
+                                         want_kw32=needs_grad and gcum.dim() == 3, gate=gate)
             kwf, A_T = pstate.kw, pstate.final_A
         else:
             pstate, kwf, A_T = None, kf, None

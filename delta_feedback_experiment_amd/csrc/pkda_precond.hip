@@ -69,6 +69,10 @@ struct PrecondParams {
   float* kw32;     // forward: kw also in FP32, or null
   bool narrow_grads;  // backward: dkw and dk in k's dtype (dk read only, dk_final written)
   float* chunk_decay;  // [num_chunks][H] exp(sum of the chunk's g_atk) from the local pass, or null
+  const void* gate_raw;  // forward: the raw gate in k's dtype for the local pass to sum, or null
+  const float* gate_A_log;
+  const float* gate_dt_bias;
+  float* gcum;
 };
 
 template <int D> struct PrecondThreads { static constexpr int v = D < 64 ? 64 : D; };
@@ -179,9 +183,20 @@ __device__ __forceinline__ float chunk_scan(const PrecondParams& p, float* buf, 
 // tokens whose k rows load before their chain runs; a short chunk
 // (FULL = false) clamps its loads to its last token and leaves the state
 // unchanged past it, so no load sits behind a branch.
-template <typename T, int D, bool APPLY, bool FULL>
+//
+// With GATE the local pass also walks the raw gate beside the key: its chunk
+// cumsum -exp(A_log) sum softplus(g + dt_bias), the operations of
+// gate_channel_fwd_kernel in their order.  Both are one round of loads per
+// group and a short chain, so the second rides on the first's latency and a
+// launch goes.  One prompt of 1,531 tokens, 8 heads: 15.2 us against 14.1 + 10.6
+// in two launches; 12,001 tokens, 16 heads 44 against 31 + 35; 32,768 tokens, 16
+// heads 102, 220 with the scan and the last pass, against 200 for the gate on a
+// second stream beside all three, whose fork and join cost more than the 20
+// (the training step 2,324 -> 2,315).  Groups of 8, 16 or 32 tokens: within 3 %
+// (32 takes 110 at the large size).
+template <typename T, int D, bool APPLY, bool FULL, bool GATE>
 __device__ __forceinline__ void precond_fwd_chunk(const PrecondParams& p, int j, int h, int start, int len) {
-  constexpr int G = 8, CH = PrecondChunk<D>::CH;
+  constexpr int G = APPLY ? 8 : 16, CH = PrecondChunk<D>::CH;
   using IO = ChanIO<T, CH>;
   using FIO = ChanIO<float, CH>;
   const int H = p.H, c0 = CH * threadIdx.x;
@@ -195,16 +210,27 @@ __device__ __forceinline__ void precond_fwd_chunk(const PrecondParams& p, int j,
   for (int q = 0; q < CH; ++q) a[q] = 0.f;
   if (APPLY) FIO::load(slot, a);
   const float center = APPLY ? p.center[h] : 0.f;
+  const T* __restrict__ raw = static_cast<const T*>(p.gate_raw);
+  float gate_scale = 0.f, bias[CH], gacc[CH];
+  if constexpr (GATE) {
+    gate_scale = -expf(p.gate_A_log[h]);
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+      bias[q] = p.gate_dt_bias[h * D + c0 + q];
+      gacc[q] = 0.f;
+    }
+  }
   float gs = 0.f;  // local pass: the chunk's g_atk summed in token order (masked rows add 0)
   auto tok = [&](int t) -> int64_t { return (int64_t)(start + (FULL ? t : min(t, len - 1))) * H + h; };
 #pragma unroll 1
   for (int g0 = 0; g0 < C; g0 += G) {
     // the group's k rows and its per-token gate values go out together
-    float kc[G][CH], lg[G], bg[G];
+    float kc[G][CH], xg[G][CH], lg[G], bg[G];
 #pragma unroll
     for (int u = 0; u < G; ++u) {
       const int64_t th = tok(g0 + u);
       IO::load(k + th * D + c0, kc[u]);
+      if constexpr (GATE) IO::load(raw + th * D + c0, xg[u]);
       lg[u] = g_atk[th];
       bg[u] = beta_atk[th];
     }
@@ -213,11 +239,16 @@ __device__ __forceinline__ void precond_fwd_chunk(const PrecondParams& p, int j,
       const int t = g0 + u;
       const int64_t th = tok(t);
       const float eg = exp_fast(lg[u]), bt = bg[u];
+      if constexpr (GATE) {
+#pragma unroll
+        for (int q = 0; q < CH; ++q) gacc[q] += gate_scale * softplus_sigmoid_fast(xg[u][q] + bias[q]).softplus;
+        if (FULL || t < len) FIO::store(p.gcum + th * D + c0, gacc);
+      }
       if (!APPLY) gs += (FULL || t < len) ? lg[u] : 0.f;
       float w[CH];
 #pragma unroll
       for (int q = 0; q < CH; ++q) {
-        const float an = eg * a[q] + bt * (kc[u][q] * kc[u][q]);
+        const float an = __builtin_fmaf(eg, a[q], bt * (kc[u][q] * kc[u][q]));  // chosen here: every form has the same bits
         a[q] = (FULL || t < len) ? an : a[q];
         if (APPLY) {
           const float r = log_fast(a[q] + p.eps) - center;
@@ -236,15 +267,15 @@ __device__ __forceinline__ void precond_fwd_chunk(const PrecondParams& p, int j,
   }
 }
 
-template <typename T, int D, bool APPLY>
+template <typename T, int D, bool APPLY, bool GATE>
 __global__ __launch_bounds__(PrecondChunk<D>::NT) void precond_fwd_chunk_kernel(PrecondParams p) {
   const ChunkHead ch = chunk_head<false>(p.H);
   if (threadIdx.x * PrecondChunk<D>::CH >= D) return;
   const ChunkInfo ci = chunk_info(p.geom, ch.cid);
   if (ci.len == C)
-    precond_fwd_chunk<T, D, APPLY, true>(p, ch.cid, ch.h, ci.start, C);
+    precond_fwd_chunk<T, D, APPLY, true, GATE>(p, ch.cid, ch.h, ci.start, C);
   else if (ci.len > 0)
-    precond_fwd_chunk<T, D, APPLY, false>(p, ch.cid, ch.h, ci.start, ci.len);
+    precond_fwd_chunk<T, D, APPLY, false, GATE>(p, ch.cid, ch.h, ci.start, ci.len);
 }
 
 // Forward launch 2: per (document, head), A entering every chunk and the
@@ -315,7 +346,7 @@ __device__ __forceinline__ void precond_bwd_chunk(const PrecondParams& p, int j,
     const float eg = exp_fast(lgv);
 #pragma unroll
     for (int q = 0; q < CH; ++q) {
-      const float an = eg * a[q] + bt * (kc[q] * kc[q]);
+      const float an = __builtin_fmaf(eg, a[q], bt * (kc[q] * kc[q]));  // the forward's bits
       a[q] = (FULL || t < len) ? an : a[q];
     }
   };
@@ -557,6 +588,10 @@ int precond_common(const pkda_precond_args* a, PrecondParams& p) {
   p.kw32 = a->kw32;
   p.narrow_grads = a->grad_dtype != PKDA_F32;
   p.chunk_decay = a->chunk_decay;
+  p.gate_raw = a->gate_raw;
+  p.gate_A_log = a->gate_A_log;
+  p.gate_dt_bias = a->gate_dt_bias;
+  p.gcum = a->gcum;
   PKDA_REQUIRE(!a->slot_idx || a->pool_size > 0, PKDA_EINVAL, "slot-indexed A states need pool_size > 0");
   return 0;
 }
@@ -582,9 +617,12 @@ int launch_precond(const PrecondParams& p, bool backward, hipStream_t s) {
     if (p.narrow_grads) launch_precond_bwd_chunks<T, D, T>(p, s);
     else launch_precond_bwd_chunks<T, D, float>(p, s);
   } else {
-    if (any) hipLaunchKernelGGL((precond_fwd_chunk_kernel<T, D, false>), chunks, dim3(NTC), 0, s, p);
+    if (any && p.gate_raw)
+      hipLaunchKernelGGL((precond_fwd_chunk_kernel<T, D, false, true>), chunks, dim3(NTC), 0, s, p);
+    else if (any)
+      hipLaunchKernelGGL((precond_fwd_chunk_kernel<T, D, false, false>), chunks, dim3(NTC), 0, s, p);
     hipLaunchKernelGGL((precond_fwd_scan_kernel<D>), docs, dim3(NT), 0, s, p);
-    if (any) hipLaunchKernelGGL((precond_fwd_chunk_kernel<T, D, true>), chunks, dim3(NTC), 0, s, p);
+    if (any) hipLaunchKernelGGL((precond_fwd_chunk_kernel<T, D, true, false>), chunks, dim3(NTC), 0, s, p);
   }
   return launch_status(backward ? "pkda_precond_bwd" : "pkda_precond_fwd");
 }
@@ -608,6 +646,8 @@ extern "C" int pkda_precond_fwd(const pkda_precond_args* a, void* stream) {
   if (int st = precond_common(a, p)) return st;
   if (a->num_seqs == 0) return 0;
   PKDA_REQUIRE(a->kw && a->a_chunk, PKDA_EINVAL, "preconditioner forward needs kw and a_chunk");
+  PKDA_REQUIRE(!a->gate_raw || (a->gate_A_log && a->gate_dt_bias && a->gcum), PKDA_EINVAL,
+               "the raw gate needs A_log, dt_bias and gcum");
   hipStream_t s = static_cast<hipStream_t>(stream);
   return a->dtype == PKDA_F32 ? dispatch_precond<float>(p, a->head_dim, false, s)
                               : dispatch_precond<bf16_t>(p, a->head_dim, false, s);

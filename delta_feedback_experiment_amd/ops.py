@@ -25,7 +25,7 @@ from torch import Tensor
 
 from . import _lib, _registry
 from .chunk import (CHUNK_SIZE, ChunkPlan, chunk_backward, chunk_forward, gate_backward, gate_forward,
-                    wants_gcum_lo)
+                    gate_or_fused, wants_gcum_lo)
 from .pkda import _f32, _on
 from . import precond as pre
 
@@ -118,18 +118,19 @@ _GATE_STREAMS: dict[int, torch.cuda.Stream] = {}
 
 
 OVERLAP_ELEMENTS = 3 << 24
-"""Elements of q from which the gate runs on its second stream.  The fork and
-the join cost the host 200 us a forward and backward, which a small call
-waits for, and the two kernels share the memory's bandwidth once they are
-large: 2 M elements (1,000 tokens of 16 heads) 700 us a step overlapped, 480
-in order; 8 M 720 and 480; 34 M 1,318 and 1,300; 67 M 2,315 and 2,333."""
+"""Elements of q from which the gate's backward runs on its second stream.  A
+fork and a join each way cost the host 200 us a step, which a small call waits
+for, and the kernels share the memory's bandwidth once they are large: 2 M
+elements (1,000 tokens of 16 heads) 700 us a step overlapped, 480 in order; 8 M
+720 and 480; 34 M 1,318 and 1,300; 67 M 2,315 and 2,333 (measured with the
+forward's gate overlapped as well; it now runs in the preconditioner's local
+pass)."""
 
 
 def _gate_stream(dev: torch.device) -> torch.cuda.Stream:
     """A second stream per device (default priority) for the per-channel
-    gate, which neither reads nor writes anything of the preconditioner's:
-    the two run side by side, joined before the first kernel that needs
-    both (the chunk forward; the end of the backward)."""
+    gate's backward, which neither reads nor writes anything of the
+    preconditioner's: the two run side by side, joined at the end."""
     i = dev.index if dev.index is not None else torch.cuda.current_device()
     s = _GATE_STREAMS.get(i)
     if s is None:
@@ -181,12 +182,9 @@ def _forward(q, k, v, g, g_atk, beta_atk, beta, A_log, dt_bias, log_atk_scale, s
         gf = gf.float()
     A32, dt32 = _f32(A_log), _f32(dt_bias)
     gcum_lo = _gcum_lo(plan, qf)
-    # the gate beside the preconditioner (both read only the inputs)
-    with _beside(qf) as own:
-        gcum = gate_forward(plan, gf, _lib.GATE_RAW_CHANNEL, A32, dt32, gcum_lo=gcum_lo)
+    gcum, gate = gate_or_fused(plan, kf, gf, _lib.GATE_RAW_CHANNEL, A32, dt32, None, gcum_lo, True)
     pstate = pre.precond_forward(plan, kf, g_atk, beta_atk, log_atk_scale, squash_x, squash_eps, None,
-                                 want_kw32=True)
-    own.join(gcum)
+                                 want_kw32=True, gate=gate)
     beta32 = _f32(beta).reshape(plan.num_tokens, plan.heads)
     o, _, fs = chunk_forward(plan, qf, kf, pstate.kw, vf, gcum, beta32, scale, None, False, save_states=save_all,
                              gcum_lo=gcum_lo)

@@ -38,7 +38,7 @@ def _flat2(t: Tensor, plan) -> Tensor:
 def precond_forward(plan, kf: Tensor, g_atk: Tensor, beta_atk: Tensor, center: Tensor, x: float, eps: float,
                     initial_A_state: Tensor | None, *, slot_idx: Tensor | None = None,
                     final_A: Tensor | None = None, want_kw32: bool = False,
-                    handoff: bool = True) -> PrecondState:
+                    handoff: bool = True, gate: tuple[Tensor, Tensor, Tensor, Tensor] | None = None) -> PrecondState:
     """Write keys for flat ``kf [N_tok, H, K]``; returns the scan's state.
 
     With ``slot_idx`` the A states are rows of a pool: ``initial_A_state``
@@ -47,10 +47,16 @@ def precond_forward(plan, kf: Tensor, g_atk: Tensor, beta_atk: Tensor, center: T
     ``want_kw32`` also returns the write keys in FP32 when ``kf`` is narrower
     (the chunk backward with per-channel gates sums its in-block pairs from
     them).  ``handoff=False`` passes no chunk-decay workspace: the document
-    scan then sums every chunk's g_atk itself (the same bits, more loads)."""
+    scan then sums every chunk's g_atk itself (the same bits, more loads).
+    ``gate``: the raw per-channel gate in ``kf``'s dtype, A_log and dt_bias
+    (FP32) and the buffer ``[N_tok, H, K]`` FP32 for its chunk cumsum, which the
+    local pass then forms beside its own (``gate_forward``'s bits)."""
     dev = kf.device
     H, K, N = plan.heads, plan.head_dim, plan.num_seqs
     ga, ba, cen = _flat2(g_atk, plan), _flat2(beta_atk, plan), _f32(center)
+    if gate is not None and (gate[0].dtype != kf.dtype or any(
+            tuple(t.shape) != tuple(kf.shape) or not t.is_contiguous() for t in (gate[0], gate[3]))):
+        raise ValueError("the raw gate and its cumsum must be contiguous of k's shape, the gate in k's dtype")
     if cen.shape != (H,):
         raise ValueError(f"log_atk_scale must be [{H}]")
     if slot_idx is not None:
@@ -73,6 +79,8 @@ def precond_forward(plan, kf: Tensor, g_atk: Tensor, beta_atk: Tensor, center: T
         slot_idx=_ptr(slot_idx), pool_size=final_A.shape[0] if slot_idx is not None else 0, kw32=_ptr(kw32),
         chunk_decay=_ptr(decay),
     )
+    if gate is not None:
+        args.gate_raw, args.gate_A_log, args.gate_dt_bias, args.gcum = map(_ptr, gate)
     _lib.call("pkda_precond_fwd", args, _stream(dev))
     return PrecondState(kw, a_chunk, final_A, a0, kw32)
 

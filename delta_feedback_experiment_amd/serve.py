@@ -34,7 +34,7 @@ import torch
 from torch import Tensor
 
 from . import _lib, _registry
-from .chunk import ChunkPlan, _flat, chunk_forward, gate_forward, validate_cu_seqlens, wants_gcum_lo
+from .chunk import ChunkPlan, _flat, chunk_forward, gate_or_fused, validate_cu_seqlens, wants_gcum_lo
 from .pkda import (_check_common, _dtype_code, _f32, _on, _ptr, _require_cuda, _require_device, _stream,
                    check_slot_indices, gate_form)
 
@@ -169,11 +169,12 @@ def prefill_op(
         gcum_lo = None
         if wants_gcum_lo(kind, q.dtype):  # as chunk_pkda takes it
             gcum_lo = torch.empty(plan.num_tokens, H, D, device=device, dtype=torch.float32)
-        gcum = gate_forward(plan, _flat(g_used, plan), kind, A_log32, dt32, gcum_lo=gcum_lo)
+        gcum, gate = gate_or_fused(plan, kf, _flat(g_used, plan), kind, A_log32, dt32, None, gcum_lo,
+                                   g_atk is not None)
         kwf = kf
         if g_atk is not None:
             pstate = pre.precond_forward(plan, kf, g_atk, beta_atk, log_atk_scale, x, eps,
-                                         a_pool if continue_state else None, slot_idx=idx, final_A=a_pool)
+                                         a_pool if continue_state else None, slot_idx=idx, final_A=a_pool, gate=gate)
             kwf = pstate.kw
         chunk_forward(plan, qf, kf, kwf, vf, gcum, beta32, float(scale),
                       state_pool if continue_state else None, True, False,

@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define PKDA_ABI_VERSION 13
+#define PKDA_ABI_VERSION 14
 #define PKDA_CHUNK 64
 
 enum pkda_dtype { PKDA_F32 = 0, PKDA_BF16 = 1 };
@@ -296,6 +296,13 @@ typedef struct pkda_precond_args {
                                     exp(sum of g_atk), written by the local chunk pass and read
                                     by the document scan (which otherwise sums every chunk's
                                     g_atk again); the same bits either way */
+  const void* gate_raw;          /* forward, optional: the raw per-channel gate [N_tok,H,K] in
+                                    dtype, activated and summed within each chunk by the local
+                                    chunk pass, in pkda_gate_fwd's place (PKDA_GATE_RAW_CHANNEL
+                                    without gcum_lo; the same bits) */
+  const float* gate_A_log;       /* [H] */
+  const float* gate_dt_bias;     /* [H*K] */
+  float* gcum;                   /* [N_tok,H,K], written when gate_raw != NULL */
 } pkda_precond_args;
 
 int pkda_precond_fwd(const pkda_precond_args* args, void* stream);

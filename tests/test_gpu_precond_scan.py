@@ -136,3 +136,38 @@ def test_slot_pool_in_place_scans(dev):
         assert torch.equal(a, b), name
     assert torch.equal(outs[0][0][[1, 3]], pool0[[1, 3]])  # rows of no document untouched
     assert torch.equal(outs[0][0][5], pool0[5])  # the empty document keeps its start A
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("B,T,cu", [(2, 150, None), (3, 1, None), (1, 400, [0, 17, 17, 100, 164, 300, 301, 301, 400])])
+def test_gate_in_the_local_pass_bitwise(dev, D, B, T, cu):
+    """The raw gate walked by the preconditioner's local pass against the
+    gate's own kernel: the chunk cumsum, the write keys, checkpoints and final
+    A bit for bit, over partial, one-token and empty chunks; and a gate whose
+    rows start at an odd element takes its own kernel."""
+    from delta_feedback_experiment_amd import _lib
+    from delta_feedback_experiment_amd import precond as pre
+    from delta_feedback_experiment_amd.chunk import ChunkPlan, fuses_gate, gate_forward
+
+    print(f"[gpu] gate in the local pass D={D} B={B} T={T}", flush=True)
+    H = 3
+    cu_t = None if cu is None else torch.tensor(cu, dtype=torch.int32, device=dev)
+    k, g_atk, beta_atk, center, *_ = (t.to(dev) for t in _inputs(B, T, H, D, torch.bfloat16, 1, D + T))
+    gen = torch.Generator().manual_seed(D)
+    g = torch.randn(B * T, H, D, generator=gen).to(dev, torch.bfloat16)
+    A_log, dt_bias = torch.rand(H, generator=gen).to(dev), torch.randn(H * D, generator=gen).to(dev)
+    plan = ChunkPlan.make(k, cu_t)
+    kf = k.reshape(B * T, H, D)
+    want = gate_forward(plan, g, _lib.GATE_RAW_CHANNEL, A_log, dt_bias)
+    gcum = torch.full_like(want, float("nan"))
+    one = pre.precond_forward(plan, kf, g_atk, beta_atk, center, 1.5, 1e-6, None, want_kw32=True)
+    two = pre.precond_forward(plan, kf, g_atk, beta_atk, center, 1.5, 1e-6, None, want_kw32=True,
+                              gate=(g, A_log, dt_bias, gcum))
+    torch.cuda.synchronize()
+    assert torch.equal(gcum, want)
+    for n in ("kw", "kw32", "final_A"):
+        assert torch.equal(getattr(one, n), getattr(two, n)), n
+    live = plan.num_chunks if cu is None else sum(-(-(b - a) // 64) for a, b in zip(cu, cu[1:]))
+    assert torch.equal(one.a_chunk[:live], two.a_chunk[:live])  # (packed: the launch bound's last slots stay unwritten)
+    odd = torch.empty(B * T * H * D + 1, device=dev, dtype=torch.bfloat16)[1:].reshape(B * T, H, D)
+    assert fuses_gate(_lib.GATE_RAW_CHANNEL, g, kf, True) and not fuses_gate(_lib.GATE_RAW_CHANNEL, odd, kf, True)

@@ -2127,9 +2127,10 @@ __global__ __launch_bounds__(64 * (BV / 16 + kRrLoadersBwd)) void chunk_state_bw
 // forward's chunk_state_fwd_split_kernel: BV / 16 chain waves keep dS and do the
 // chain dS -> KW dS -> dU -> Z -> dS; they leave the entering dS as B operands
 // and Z in FP32, lane for lane, in LDS, and BV / 16 output waves store the
-// checkpoint in the same step and form the dBv / dv rows in the next one.  Q^T
-// (s e^G dO), which waits for nothing of the chain, is added to the decayed dS
-// while Z forms.
+// checkpoint in the same step and form the dBv / dv rows in the next one.  The
+// first half of Q^T (s e^G dO), which waits for nothing of the chain, is added
+// to the decayed dS while Z forms.  Every value is formed by the same operations
+// in the same order as above.
 template <int D, int BV>
 struct RrSplitBwdLayout : RrBwdLayout<D, BV, true> {
   using Base = RrBwdLayout<D, BV, true>;
@@ -2419,9 +2420,7 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_state_bwd_split_kernel(Bwd
 #pragma unroll
     for (int rt = 0; rt < NKT; ++rt) dS[rt] = dS[rt] * decay;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], kq[kt][rt], dOgB[kt]);
+    for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], kq[0][rt], dOgB[0]);
     s16x8_t km[2][NKT];
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
@@ -2440,10 +2439,13 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_state_bwd_split_kernel(Bwd
     }
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) *z_slot(wave, s, rb) = Z[rb];
+    // (the order of the other forms: a call's gradients do not depend on which takes it)
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], km[0][rt], ZB[0]);
 #pragma unroll
-      for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], km[kt][rt], ZB[kt]);
+    for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], kq[1][rt], dOgB[1]);
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], km[1][rt], ZB[1]);
     publish(s + 1);
   }
   __syncthreads();
@@ -2897,9 +2899,7 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_state_bwd_split_pc_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j) dS[rt][j] *= ee[rt][j];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], kq[kt][rt], dOB[kt]);
+    for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], kq[0][rt], dOB[0]);
     const s16x8_t dUnB[2] = {pack_acc_pair(-dU[0], -dU[1]), pack_acc_pair(-dU[2], -dU[3])};
     s16x8_t km[2][NKT];
 #pragma unroll
@@ -2909,9 +2909,11 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_state_bwd_split_pc_kernel(
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) *ub_slot(wave, s, kt) = __builtin_bit_cast(uint4, dUnB[kt]);
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], km[0][rt], dUnB[0]);
 #pragma unroll
-      for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], km[kt][rt], dUnB[kt]);
+    for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], kq[1][rt], dOB[1]);
+#pragma unroll
+    for (int rt = 0; rt < NKT; ++rt) mfma_bf16(dS[rt], km[1][rt], dUnB[1]);
     publish(s + 1);
   }
   __syncthreads();

@@ -969,11 +969,29 @@ constexpr int kSplitLoaders = 4;  // two groups of two waves
 //   per channel, reverse   56.8 56.0 45.5     57.7 57.8 54.7   60.0 60.1 61.0   61.1 63.2 64.6
 // 256 workgroups of 256 chunks, per head: forward 606 568 703, reverse 561 512
 // 642.  One prompt of 24 chunks, 32 workgroups, per channel: forward 46.4 47.8 37.4.
-// So per head the split form always, deferred to kDeferHead; per channel forward
-// the same to kDeferChannel; per channel reverse split (deferred) to
-// kSplitChannelReverse and the form without output waves past it, where the
-// output stage it has room for is worth more than the shorter chain.
-constexpr int kDeferHead = 192, kDeferChannel = 112, kSplitChannelReverse = 128;
+// So per head the split form always, deferred to kDeferHead.
+//
+// Per channel the form without output waves is the better one past some count:
+// the output stage it has room for is worth more than the shorter chain once
+// the loads take their time.  Without output waves / split, 32 chunks a row:
+//   workgroups             80         96         112        128        160        192        256
+//   forward, D = 128       60.1 54.6  60.4 55.7  61.0 57.0  62.0 62.7  69.0 68.6  94.1 94.0  120 121
+//   forward, D = 64        41.0 34.5  41.5 34.8  42.6 36.0  43.0 38.9  56.0 53.0  76.7 79.2  91.0 91.4
+//   reverse, D = 128       54.8 48.5  54.2 55.0  55.6 59.1  56.3 60.9  62.8 63.1  71.3 71.3  100 99.3
+//   reverse, D = 64        34.9 29.3  35.2 36.9  39.6 40.6  41.2 42.8  43.8 42.6  49.0 48.5  64.6 63.8
+// Forward, 256 workgroups of 256 chunks 624 649; packed documents, 12,000 tokens
+// of 16 heads, 5 documents (320 workgroups) 189 196, 7 documents 164 169.
+// So forward split (deferred to kDeferChannel) to kSplitChannelForward, reverse
+// split, always deferred, to kSplitChannelReverse.
+//
+// All of these take 32 columns a workgroup, where 64 make fewer workgroups than
+// compute units.  A workgroup's LDS fills its compute unit, so 257 to 510 of
+// them run in two rounds, and the 64-column form, one round, would be faster for
+// rows of one length (per head, D = 128, 264 workgroups of 32 chunks: forward
+// 137 against 98, reverse 136 against 85) but slower for packed documents, whose
+// longest one is the time (5 documents of 12,000 tokens: 137 against 219, 138
+// against 189); the count does not tell them apart.
+constexpr int kDeferHead = 192, kDeferChannel = 112, kSplitChannelForward = 160, kSplitChannelReverse = 80;
 inline int64_t state_pass_workgroups(const ChunkGeom& g, int H, int slices) { return (int64_t)g.num_seqs * H * slices; }
 
 }  // namespace pkda

@@ -1471,11 +1471,6 @@ __global__ __launch_bounds__(64 * (BV / 16 + kRrLoaders)) void chunk_state_fwd_r
 // the U and O rows to the output stage.  Every value is formed by the same
 // operations in the same order as above.
 // ---------------------------------------------------------------------------
-// When a loader group sends its next loads.  Right after it staged a chunk
-// they are in flight for two steps, but the group then holds the barrier up
-// (staging 2,450 cycles, sending 2,020, against 3,500 of the chain); in the
-// following step, its idle one, they are in flight for one.  One step covers the
-// latency while other compute units leave the memory idle, not when all stream.
 template <int D, int BV>
 struct RrSplitLayout : RrFwdLayout<D, BV, true> {
   using Base = RrFwdLayout<D, BV, true>;
@@ -2314,12 +2309,18 @@ int launch_state_fwd_rr_pc(const FwdParams& p, hipStream_t s) {
   const int N = p.geom.num_seqs;
   if (N <= 0) return 0;
   const bool narrow = (int64_t)N * p.H * (D / 64) < 256;
-  auto kern = !narrow                                                   ? chunk_state_fwd_rr_pc_kernel<D, 64>
-              : state_pass_workgroups(p.geom, p.H, D / 32) <= kDeferChannel ? chunk_state_fwd_split_pc_kernel<D, 32, true>
-                                                                        : chunk_state_fwd_split_pc_kernel<D, 32, false>;
-  const int bytes = narrow ? RrPcSplitLayout<D, 32>::bytes : RrPcFwdLayout<D, 64>::bytes;
+  const int64_t workgroups = state_pass_workgroups(p.geom, p.H, D / 32);
+  const bool split = narrow && workgroups <= kSplitChannelForward;
+  auto kern = split && workgroups <= kDeferChannel ? chunk_state_fwd_split_pc_kernel<D, 32, true>
+              : split                              ? chunk_state_fwd_split_pc_kernel<D, 32, false>
+              : narrow                             ? chunk_state_fwd_rr_pc_kernel<D, 32>
+                                                   : chunk_state_fwd_rr_pc_kernel<D, 64>;
+  const int bytes = split    ? RrPcSplitLayout<D, 32>::bytes
+                    : narrow ? RrPcFwdLayout<D, 32>::bytes
+                             : RrPcFwdLayout<D, 64>::bytes;
+  const int waves = split ? 4 + kSplitLoaders : (narrow ? 2 : 4) + kRrLoaders;
   if (int st = set_smem(kern, bytes)) return st;
-  hipLaunchKernelGGL(kern, doc_grid(N, p.H, D / (narrow ? 32 : 64)), dim3(64 * (4 + (narrow ? kSplitLoaders : kRrLoaders))), bytes, s, p);
+  hipLaunchKernelGGL(kern, doc_grid(N, p.H, D / (narrow ? 32 : 64)), dim3(64 * waves), bytes, s, p);
   return launch_status("pkda_chunk_fwd(state)");
 }
 

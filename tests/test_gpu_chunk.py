@@ -783,7 +783,8 @@ def test_state_pass_forms_agree(dev, D, per_channel):
     """The state passes with 64 columns a workgroup (320 rows x heads) and the
     narrower ones in each of their dispatches.  Workgroups of 32 columns, 2 per
     row and head at D = 64 and 4 at D = 128: 360 and 448 (past one a compute
-    unit), 224 (loads not deferred), 112 and 120, 56 and 60 (all deferred).
+    unit), 280 and 140, 224 and 112, 120 and 60, 56 and 28 (with and without
+    output waves, loads deferred and not).
     Rows of one token, of two whole chunks and a partial one, of six whole
     chunks and of six and a partial one (a loader group sends its loads three
     chunks ahead); initial and final states.  All forms take every value by the
@@ -813,7 +814,7 @@ def test_state_pass_forms_agree(dev, D, per_channel):
             return [o.detach(), *gr[:5]], [S.detach(), gr[5]]
 
         wide = step(B, H)
-        for rows, heads in ((12, 15) if D == 64 else (8, 14), (8, 14), (4, 14), (3, 10), (1, 14)):
+        for rows, heads in ((12, 15) if D == 64 else (8, 14), (8, 14), (5, 14), (4, 14), (3, 10), (1, 14)):
             tokens, states = step(rows, heads)
             want = ([t[:rows, :, :heads] for t in wide[0]], [t[:rows, :heads] for t in wide[1]])
             for name, a, b in zip(("o", "dq", "dk", "dv", "dg", "dbeta", "S", "dS0"), (*tokens, *states),

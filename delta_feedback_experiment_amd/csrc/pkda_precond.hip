@@ -34,8 +34,8 @@
 //   3. per (chunk, head): the chunk again from its entering value, writing
 //      kw (forward) or the gradients (backward).
 // The forward's third launch and both backward chunk launches recompute A
-// inside the chunk from a_chunk with the same arithmetic, so the backward
-// sees exactly the A the forward squashed.  Channel sums (dg_atk, dbeta_atk,
+// inside the chunk from a_chunk with the same arithmetic (a_step's rounding
+// aside in BF16), so the backward sees the A the forward squashed.  Channel sums (dg_atk, dbeta_atk,
 // dcenter) reduce in a fixed order: lanes of a 16-lane row, then rows.
 #include <type_traits>
 
@@ -178,6 +178,17 @@ __device__ __forceinline__ float chunk_scan(const PrecondParams& p, float* buf, 
   return x;
 }
 
+// One token of A, e^g A + beta k^2, in one fused multiply-add, written out so
+// that every pass of a kind has the same bits.  Unrounded in it is the gain
+// beta k^2 (FP32, and the backward of either type) or the decayed A (the BF16
+// forward, whose write keys are rounded to eight bits).  With the decayed A the
+// FP32 write keys are 15 % further from 64 bits (unit keys, d = 64, 777 tokens,
+// log decays about -0.9).
+template <bool FUSE_GAIN>
+__device__ __forceinline__ float a_step(float eg, float a, float bt, float k) {
+  return FUSE_GAIN ? __builtin_fmaf(bt, k * k, eg * a) : __builtin_fmaf(eg, a, bt * (k * k));
+}
+
 // Forward launches 1 (APPLY = false: local end A from zero into a_chunk) and
 // 3 (APPLY: A from a_chunk, kw out).  The chunk runs in sub-blocks of 8
 // tokens whose k rows load before their chain runs; a short chunk
@@ -248,7 +259,7 @@ __device__ __forceinline__ void precond_fwd_chunk(const PrecondParams& p, int j,
       float w[CH];
 #pragma unroll
       for (int q = 0; q < CH; ++q) {
-        const float an = __builtin_fmaf(eg, a[q], bt * (kc[u][q] * kc[u][q]));  // chosen here: every form has the same bits
+        const float an = a_step<std::is_same<T, float>::value>(eg, a[q], bt, kc[u][q]);
         a[q] = (FULL || t < len) ? an : a[q];
         if (APPLY) {
           const float r = log_fast(a[q] + p.eps) - center;
@@ -340,13 +351,12 @@ __device__ __forceinline__ void precond_bwd_chunk(const PrecondParams& p, int j,
   if (APPLY && active) FIO::load(p.lam_chunk + row, lam);
   const float center = p.center[h], lx = p.log_x, eps = p.eps;
   auto tok = [&](int t) -> int64_t { return (int64_t)(start + (FULL ? t : min(t, len - 1))) * H + h; };
-  // one token of the forward's A recurrence, channel by channel (the same
-  // arithmetic as the forward pass, so the same values)
+  // one token of the forward's A recurrence, channel by channel
   auto step = [&](int t, float* a, const float* kc, float lgv, float bt) {
     const float eg = exp_fast(lgv);
 #pragma unroll
     for (int q = 0; q < CH; ++q) {
-      const float an = __builtin_fmaf(eg, a[q], bt * (kc[q] * kc[q]));  // the forward's bits
+      const float an = a_step<true>(eg, a[q], bt, kc[q]);
       a[q] = (FULL || t < len) ? an : a[q];
     }
   };

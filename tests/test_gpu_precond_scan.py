@@ -171,3 +171,28 @@ def test_gate_in_the_local_pass_bitwise(dev, D, B, T, cu):
     assert torch.equal(one.a_chunk[:live], two.a_chunk[:live])  # (packed: the launch bound's last slots stay unwritten)
     odd = torch.empty(B * T * H * D + 1, device=dev, dtype=torch.bfloat16)[1:].reshape(B * T, H, D)
     assert fuses_gate(_lib.GATE_RAW_CHANNEL, g, kf, True) and not fuses_gate(_lib.GATE_RAW_CHANNEL, odd, kf, True)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_step_rounding(dev, D, dtype):
+    """The A recurrence's one fused multiply-add: in FP32 the gain beta k^2 goes
+    into it unrounded (only k^2 and the decayed A are rounded), in the BF16
+    forward the decayed A.  With a decay of one both are plain to follow: the
+    final A of one chunk bit for bit, the fused sum taken in FP64 (whose own
+    rounding moves an FP32 result with a chance of 2^-29)."""
+    from delta_feedback_experiment_amd import precond as pre
+    from delta_feedback_experiment_amd.chunk import ChunkPlan
+
+    print(f"[gpu] A step rounding D={D} {dtype}", flush=True)
+    B, T, H = 2, 50, 3
+    k, _, beta_atk, center, *_ = _inputs(B, T, H, D, dtype, B, 11 + D)
+    plan = ChunkPlan.make(k.to(dev), None)
+    st = pre.precond_forward(plan, k.to(dev).reshape(B * T, H, D), torch.zeros(B, T, H, device=dev),
+                             beta_atk.to(dev), center.to(dev), 1.5, 1e-6, None)
+    torch.cuda.synchronize()
+    A = torch.zeros(B, H, D)
+    for t in range(T):
+        k2, b = k[:, t].float().square(), beta_atk[:, t, :, None]
+        A = (b.double() * k2.double() + A.double()).float() if dtype == torch.float32 else A + b * k2
+    assert torch.equal(st.final_A.cpu(), A)

@@ -15,10 +15,13 @@ struct ColumnSum {
   int blocks;  // workgroups that take it: ceil(n / COLS)
 };
 
-// A workgroup takes COLS adjacent columns: thread (slot, column) adds the
-// partials slot, slot + SLOTS, ... in order -- sixteen loads in flight, and
-// the COLS threads of a slot read adjacent words -- then a halving tree over
-// the slots in LDS.  Two sums share a launch; the second may be empty.
+// A workgroup takes COLS adjacent columns.  The partials of a column are summed
+// in 256 classes -- class c takes c, c + 256, ... in order -- and the classes in
+// a halving tree, so a chain is count / 256 additions long.  Thread (slot,
+// column) holds the classes slot, slot + SLOTS, ... in registers: their loads go
+// out together, and the COLS threads of a slot read adjacent words.  It takes the
+// tree down to one sum a slot, LDS the rest.  Two sums share a launch; the
+// second may be empty.
 //
 // With many columns the partials' bytes bound it, with few the loads'
 // latency, so the width follows n:
@@ -35,19 +38,35 @@ struct ColumnSum {
 // for the norm's dweight, 15.8 for the convolution's dw).
 template <int COLS, int THREADS>
 __global__ __launch_bounds__(THREADS) void column_sums_kernel(ColumnSum a, ColumnSum b) {
-  constexpr int SLOTS = THREADS / COLS;
+  constexpr int SLOTS = THREADS / COLS, CLASSES = 256, K = CLASSES / SLOTS;
   __shared__ float s[THREADS];
   const bool first = (int)blockIdx.x < a.blocks;
   const ColumnSum& j = first ? a : b;
   const int col = threadIdx.x % COLS, slot = threadIdx.x / COLS;
   const int i = (blockIdx.x - (first ? 0 : a.blocks)) * COLS + col;
-  float acc = 0.f;
+  float acc[K];
+#pragma unroll
+  for (int c = 0; c < K; ++c) acc[c] = 0.f;
   if (i < j.n) {
     const float* __restrict__ p = j.part + i;
-#pragma unroll 16
-    for (int q = slot; q < j.count; q += SLOTS) acc += p[(int64_t)q * j.stride];
+    int q = slot;
+#pragma unroll 2
+    for (; q - slot + CLASSES <= j.count; q += CLASSES)  // whole rounds
+#pragma unroll
+      for (int c = 0; c < K; ++c) acc[c] += p[(int64_t)(q + c * SLOTS) * j.stride];
+    if (q - slot < j.count) {  // the last round: rows past the end read the last one and add 0
+#pragma unroll
+      for (int c = 0; c < K; ++c) {
+        const float x = p[(int64_t)min(q + c * SLOTS, j.count - 1) * j.stride];
+        acc[c] += q + c * SLOTS < j.count ? x : 0.f;
+      }
+    }
   }
-  s[threadIdx.x] = acc;
+#pragma unroll
+  for (int off = K / 2; off > 0; off >>= 1)
+#pragma unroll
+    for (int c = 0; c < off; ++c) acc[c] += acc[c + off];
+  s[threadIdx.x] = acc[0];
   __syncthreads();
 #pragma unroll
   for (int off = SLOTS / 2; off > 0; off >>= 1) {

@@ -166,10 +166,31 @@ __device__ __forceinline__ float lane_group_sum(float v) {
 // The same over 32 lanes: the rows of 16 summed as above, then the two rows of
 // each half wave (v_permlane16_swap leaves rows 0, 0, 2, 2 of the value in one
 // register and rows 1, 1, 3, 3 in the other).
-__device__ __forceinline__ float lane_half_sum(float v) {
-  v = lane_group_sum<16>(v);
+__device__ __forceinline__ float half_wave_rows_sum(float v) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float lane_half_sum(float v) { return half_wave_rows_sum(lane_group_sum<16>(v)); }
+
+// Sum over N = 8, 16 or 32 lanes of the squares of four values each, as lanes of
+// eight would form it: lanes 2 i and 2 i + 1 make one chain (the second value's
+// square rounded by itself, the others fused onto it in turn), and the chains add
+// in pairs as above.
+template <int N>
+__device__ __forceinline__ float lane_pair_squares(const float (&x)[4]) {
+  static_assert(N == 8 || N == 16 || N == 32, "8, 16 or 32 lanes");
+  float v = __builtin_fmaf(x[0], x[0], x[1] * x[1]);
+  v = __builtin_fmaf(x[2], x[2], v);
+  v = __builtin_fmaf(x[3], x[3], v);
+  v = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xA0, 0xF, 0xF, false));  // quad [0,0,2,2]
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v = __builtin_fmaf(x[j], x[j], v);  // the odd lanes' is the chain
+  v = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xF5, 0xF, 0xF, false));  // quad [1,1,3,3]
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, false));
+  if constexpr (N >= 16) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, false));
+  if constexpr (N == 32) v = half_wave_rows_sum(v);
+  return v;
 }
 
 }  // namespace pkda

@@ -21,18 +21,20 @@
 // halo per tile) with fully coalesced loads, a group of four rows ahead of the
 // one computed; whole groups run without a row test, so the windows slide by
 // renaming and not by register moves.  The head's sum of squares is a DPP
-// reduction over the head_dim / 4 lanes that share the head.  The backward
+// reduction over the head_dim / 4 lanes that share the head; the forward's and
+// the token kernel's add as lanes of eight channels would, so that Q and K do not
+// depend on the split (five operations a row, 1 to 2 % of the forward).  The backward
 // recomputes a and y for its tile plus the W - 1 rows after it (the rows whose
 // gradient reaches the tile's x).  dw is summed per tile in registers and the
 // tiles in a fixed order by a second kernel: deterministic.
 //
-// Bounds: HBM, with the VALU close behind (85 operations a thread and row
+// Bounds: HBM, with the VALU close behind (90 operations a thread and row
 // forward, 125 backward).  B8 T4096, 3 x 1,024 channels, W = 4, BF16: forward
-// 83 us for 403 MB (4.9 TB/s, the card's copy rate 5.2), backward 146 for 604
-// MB and 25 of dw partials (4.3 TB/s, 112 VGPRs, four waves a SIMD).  Eight
+// 80 us for 403 MB (5.0 TB/s, the card's copy rate 5.2), backward 143 for 604
+// MB and 25 of dw partials (4.4 TB/s, 112 VGPRs, four waves a SIMD).  Eight
 // channels a thread, row tests and IEEE divisions in the sigmoids took 109
 // and 184 (227 VGPRs, two waves); eight channels in today's form 80 and 190,
-// but 15.4 us against 13.3 on 3 rows of 1,000 tokens.
+// but 15.4 us against 14 on 3 rows of 1,000 tokens.
 #include "pkda_common.h"
 #include "pkda_reduce.h"
 
@@ -52,9 +54,10 @@ constexpr int kFillWaves = 4096;  // four waves on every SIMD
 // Tokens of a workgroup's tile: the longest of long_tile, long_tile / 2 and
 // long_tile / 4 whose waves fill the chip, else the last.  A long tile reads
 // and recomputes fewer halo rows, a short one puts more waves on a small
-// call: 3 rows of 1,000 tokens, 3,072 channels, go 13.3 us forward (tile 8)
-// against 14.0 (tile 16), 21.8 backward (tile 16) against 26.8 (tile 32);
-// 8 rows of 4,096 take the long tiles, 83 and 146 us, 1 to 4 % faster than half.
+// call: one row of 200 tokens, 768 channels, goes 4.6 us forward (tile 8) against
+// 6.6 (tile 16), 10.0 backward (tile 16) against 16.0 (tile 32); 3 rows of 1,000,
+// 3,072 channels, 14 either way and 21 to 23 against 27; 8 rows of 4,096,
+// 6,144 channels, take the long tiles, 190 and 306 us, 3 % faster than half.
 inline int conv_tile(int B, int T, int C, int long_tile) {
   const int64_t waves = (C + 64 * kCh - 1) / (64 * kCh);
   int tile = long_tile;
@@ -243,17 +246,15 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_fwd_kernel(ConvParams p
   auto step = [&](int t, const Row& xr) {
     float xt[CH], y[CH];
     xr.unpack(xt);
-    float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       float a = wt[j][W - 1] * xt[j];
 #pragma unroll
       for (int w = 0; w < W - 1; ++w) a += wt[j][w] * hist[w][j];
       y[j] = a * sigmoid_fast(a);
-      ss += y[j] * y[j];
     }
     if (norm) {
-      const float r = rsqrtf(head_sum<G>(ss) + p.eps);
+      const float r = rsqrtf(lane_pair_squares<G>(y) + p.eps);
 #pragma unroll
       for (int j = 0; j < CH; ++j) y[j] *= r;
     }
@@ -491,17 +492,15 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_token_kernel(ConvParams
 #pragma unroll
     for (int w = 0; w < W - 1; ++w) hr[r][w].unpack(hist[w]);
     float y[CH];
-    float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       float a = wt[j][W - 1] * xt[j];
 #pragma unroll
       for (int w = 0; w < W - 1; ++w) a += wt[j][w] * hist[w][j];
       y[j] = a * sigmoid_fast(a);
-      ss += y[j] * y[j];
     }
     if (norm) {
-      const float rn = rsqrtf(head_sum<G>(ss) + p.eps);
+      const float rn = rsqrtf(lane_pair_squares<G>(y) + p.eps);
 #pragma unroll
       for (int j = 0; j < CH; ++j) y[j] *= rn;
     }

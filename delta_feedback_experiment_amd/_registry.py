@@ -18,7 +18,6 @@ from __future__ import annotations
 
 import torch
 from torch import Tensor, _C
-from torch.autograd.function import once_differentiable
 
 _LIBRARY = torch.library.Library("pkda_mi355x", "FRAGMENT")
 
@@ -43,7 +42,7 @@ def device_op(schema: str):
             return out
 
         _LIBRARY.impl(name, mutating if written else fn, "CUDA")
-        _autograd(op, name, None, None)
+        _autograd(op, name)
         return op
 
     return register
@@ -63,11 +62,14 @@ def register_autograd(op, backward, setup_context) -> None:
 _FORMULAS: dict = {}
 
 
-def _autograd(op, name: str, setup_context, backward) -> None:
+def _autograd(op, name: str) -> None:
+    returns = op._schema.returns
+    listed = bool(returns) and isinstance(returns[-1].type, _C.ListType)  # its tensors become outputs one by one
+
     def flat(out):
-        if isinstance(out, (tuple, list)) and out and isinstance(out[-1], list):
-            return (*out[:-1], *out[-1])
-        return out
+        if not listed:
+            return out
+        return (*out[:-1], *out[-1]) if len(returns) > 1 else tuple(out)
 
     class Operator(torch.autograd.Function):
         @staticmethod
@@ -79,20 +81,22 @@ def _autograd(op, name: str, setup_context, backward) -> None:
             return flat(out)
 
         @staticmethod
-        @once_differentiable
         def backward(ctx, *grads):
+            # under create_graph the formula's own operator, which has none, takes
+            # part in the graph and raises when a second derivative reaches it
             if op not in _FORMULAS:
                 raise RuntimeError(f"Trying to backward through {op} but no autograd formula was registered.")
             return (None, *_FORMULAS[op][1](ctx, *grads))
 
     Operator.__name__ = f"BackwardFor_pkda_mi355x_{name}"
-    returns = op._schema.returns
-    listed = len(returns) > 1 and isinstance(returns[-1].type, _C.ListType)
 
     def kernel(keyset, *args):
         if _C.is_grad_enabled() and _C._any_requires_grad(*args):
             out = Operator.apply(keyset, *args)
-            return (*out[:len(returns) - 1], list(out[len(returns) - 1:])) if listed else out
+            if not listed:
+                return out
+            last = list(out[len(returns) - 1:])
+            return (*out[:len(returns) - 1], last) if len(returns) > 1 else last
         with _C._AutoDispatchBelowAutograd():
             return op.redispatch(keyset & _C._after_autograd_keyset, *args)
 

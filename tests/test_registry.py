@@ -7,7 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from delta_feedback_experiment_amd import _registry, pkda_norm_gate, pkda_qkv_conv
+from delta_feedback_experiment_amd import _registry, pkda_controls, pkda_norm_gate, pkda_qkv_conv, pkda_recurrence
 from delta_feedback_experiment_amd.serve import qkv_conv_cached_op
 
 
@@ -24,15 +24,46 @@ def test_backward_without_a_formula_raises():
             q.sum().backward()
 
 
-@pytest.mark.parametrize("create_graph", [False, True])
-def test_second_derivative_raises(create_graph):
+def _norm_gate():
+    leaves = [_meta(5, 64, grad=True), _meta(5, 64, grad=True), _meta(64, grad=True)]
+    return leaves, pkda_norm_gate(*leaves, 1e-6)[0]
+
+
+def _conv():
+    leaves = [_meta(2, 5, 96, grad=True), _meta(96, 4, grad=True)]
+    return leaves, pkda_qkv_conv(*leaves, 32, 64, 1e-6)[0]
+
+
+def _recurrence():
+    token, head = (1, 5, 2, 64), (1, 5, 2)
+    leaves = [_meta(*s, grad=True) for s in (*[token] * 4, *[head] * 3, (2,), (128,), (2,))]
+    return leaves, pkda_recurrence(*leaves, 0.125, 1.5, 1e-6, False)[0]
+
+
+def _controls():
+    leaves = [_meta(2, 5, 2 * 64 + 3 * 2, grad=True), _meta(2, grad=True), _meta(2, grad=True)]
+    return leaves, pkda_controls(*leaves, 64, 2)[1]
+
+
+@pytest.mark.parametrize("make", [_norm_gate, _conv, _recurrence, _controls])
+def test_second_derivative_raises(make):
+    """Alone, and beside the first derivative, where a second one left out
+    would leave gradients that look whole."""
+    for penalty in (lambda y, dx: dx.square().sum(), lambda y, dx: y.sum() + dx.square().sum()):
+        leaves, y = make()
+        dx, = torch.autograd.grad(y.sum(), leaves[:1], create_graph=True)
+        assert dx.shape == leaves[0].shape
+        with pytest.raises(RuntimeError, match="no autograd formula"):
+            penalty(y, dx).backward()
+    leaves, y = make()
+    grads = torch.autograd.grad(y.sum(), leaves)
+    assert [g.shape for g in grads] == [t.shape for t in leaves] and not any(g.requires_grad for g in grads)
+
+
+def test_statistics_have_no_gradient():
     x, gate, w = _meta(5, 64, grad=True), _meta(5, 64, grad=True), _meta(64, grad=True)
     y, rstd = pkda_norm_gate(x, gate, w, 1e-6)
-    assert not rstd.requires_grad
-    dx, dgate, dw = torch.autograd.grad(y, (x, gate, w), torch.empty_like(y), create_graph=create_graph)
-    assert dx.shape == x.shape and dw.shape == w.shape
-    with pytest.raises(RuntimeError):
-        torch.autograd.grad(dx, x, torch.empty_like(dx))
+    assert y.requires_grad and not rstd.requires_grad
 
 
 def test_saved_tensor_hooks_see_the_inputs():

@@ -55,7 +55,7 @@ def _args(packed: Tensor, A_log_p: Tensor, dt_bias_p: Tensor, rank: int, heads: 
     return args, flat, A32, dt32, gate_width
 
 
-@_registry.device_op("pkda_controls_act(Tensor packed, Tensor A_log_p, Tensor dt_bias_p, int rank, int heads) "
+@_registry.device_op("pkda_controls_act(Tensor packed, Tensor A_log_p, Tensor dt_bias_p, SymInt rank, SymInt heads) "
                      "-> (Tensor, Tensor, Tensor)")
 def pkda_controls_act(packed: Tensor, A_log_p: Tensor, dt_bias_p: Tensor, rank: int,
                       heads: int) -> tuple[Tensor, Tensor, Tensor]:
@@ -79,7 +79,7 @@ def _pkda_controls_act_fake(packed, A_log_p, dt_bias_p, rank, heads):
 
 @_registry.device_op(
     "pkda_controls_backward(Tensor packed, Tensor A_log_p, Tensor dt_bias_p, Tensor? d_decay_hidden, Tensor? dbeta, "
-    "Tensor? dprecond_decay, Tensor? dprecond_beta, Tensor? d_gate_hidden, int rank, int heads) "
+    "Tensor? dprecond_decay, Tensor? dprecond_beta, Tensor? d_gate_hidden, SymInt rank, SymInt heads) "
     "-> (Tensor, Tensor, Tensor)")
 def pkda_controls_backward(packed: Tensor, A_log_p: Tensor, dt_bias_p: Tensor, d_decay_hidden: Tensor | None,
                            dbeta: Tensor | None, dprecond_decay: Tensor | None, dprecond_beta: Tensor | None,

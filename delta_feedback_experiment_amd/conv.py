@@ -34,7 +34,7 @@ def _args(x: Tensor, weight: Tensor, head_dim: int, norm_channels: int, eps: flo
     )
 
 
-@_registry.device_op("pkda_qkv_conv(Tensor x, Tensor weight, int head_dim, int norm_channels, float eps) "
+@_registry.device_op("pkda_qkv_conv(Tensor x, Tensor weight, SymInt head_dim, SymInt norm_channels, float eps) "
                      "-> (Tensor, Tensor, Tensor)")
 def pkda_qkv_conv(x: Tensor, weight: Tensor, head_dim: int, norm_channels: int,
                   eps: float) -> tuple[Tensor, Tensor, Tensor]:
@@ -56,8 +56,8 @@ def _pkda_qkv_conv_fake(x, weight, head_dim, norm_channels, eps):
     return tuple(x.new_empty(B, T, C // 3) for _ in range(3))
 
 
-@_registry.device_op("pkda_qkv_conv_backward(Tensor x, Tensor weight, Tensor dq, Tensor dk, Tensor dv, int head_dim, "
-                     "int norm_channels, float eps) -> (Tensor, Tensor)")
+@_registry.device_op("pkda_qkv_conv_backward(Tensor x, Tensor weight, Tensor dq, Tensor dk, Tensor dv, SymInt head_dim, "
+                     "SymInt norm_channels, float eps) -> (Tensor, Tensor)")
 def pkda_qkv_conv_backward(x: Tensor, weight: Tensor, dq: Tensor, dk: Tensor, dv: Tensor, head_dim: int,
                            norm_channels: int, eps: float) -> tuple[Tensor, Tensor]:
     """``(dx, dw)`` of :func:`pkda_qkv_conv` (fla_ops.py:181-215).  ``dw`` is a

@@ -290,9 +290,9 @@ def pkda_decode_step_(
 
 
 @_registry.device_op(
-    "decode_step_(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor(a!) state_pool, Tensor? slot_idx, "
-    "Tensor(b!)? a_pool, Tensor? g_atk, Tensor? beta_atk, Tensor? log_atk_scale, Tensor? A_log, Tensor? dt_bias, "
-    "bool use_gate_in_kernel, float scale, float x, float eps, Tensor(c!) o) -> ()")
+    "decode_step_(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor(a5!) state_pool, Tensor? slot_idx, "
+    "Tensor(a7!)? a_pool, Tensor? g_atk, Tensor? beta_atk, Tensor? log_atk_scale, Tensor? A_log, Tensor? dt_bias, "
+    "bool use_gate_in_kernel, float scale, float x, float eps, Tensor(a17!) o) -> ()")
 def decode_step_op(
     q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, state_pool: Tensor, slot_idx: Tensor | None,
     a_pool: Tensor | None, g_atk: Tensor | None, beta_atk: Tensor | None, log_atk_scale: Tensor | None,

@@ -139,10 +139,10 @@ def pkda_prefill_(
 
 
 @_registry.device_op(
-    "prefill_(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor(a!) state_pool, Tensor slot_idx, "
-    "Tensor(b!)? a_pool, bool continue_state, Tensor? cu_seqlens, Tensor? g_atk, Tensor? beta_atk, "
+    "prefill_(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor(a5!) state_pool, Tensor slot_idx, "
+    "Tensor(a7!)? a_pool, bool continue_state, Tensor? cu_seqlens, Tensor? g_atk, Tensor? beta_atk, "
     "Tensor? log_atk_scale, Tensor? A_log, Tensor? dt_bias, bool use_gate_in_kernel, float scale, float x, float eps, "
-    "Tensor(c!) o) -> ()")
+    "Tensor(a19!) o) -> ()")
 def prefill_op(
     q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, state_pool: Tensor, slot_idx: Tensor,
     a_pool: Tensor | None, continue_state: bool, cu_seqlens: Tensor | None, g_atk: Tensor | None,
@@ -227,7 +227,7 @@ def pkda_qkv_conv_cached_(
 
 
 @_registry.device_op(
-    "qkv_conv_cached_(Tensor x, Tensor weight, int head_dim, int norm_channels, float eps, Tensor(a!) conv_pool, "
+    "qkv_conv_cached_(Tensor x, Tensor weight, SymInt head_dim, SymInt norm_channels, float eps, Tensor(a5!) conv_pool, "
     "Tensor? slot_idx, bool continue_state) -> (Tensor, Tensor, Tensor)")
 def qkv_conv_cached_op(
     x: Tensor, weight: Tensor, head_dim: int, norm_channels: int, eps: float, conv_pool: Tensor,

@@ -75,6 +75,31 @@ def test_saved_tensor_hooks_see_the_inputs():
     torch.autograd.grad((q, k, v), (x, w), [torch.empty_like(t) for t in (q, k, v)])
 
 
+class _ConvOfAnyWidth(torch.nn.Module):
+    def forward(self, x, w):
+        return pkda_qkv_conv(x, w, 32, 2 * x.shape[2] // 3, 1e-6)
+
+
+def test_integers_may_be_symbolic():
+    """One graph for all widths under a dynamic compile, an export with a
+    dynamic width that runs at another one, and the same for every integer
+    argument of the other operators."""
+    graphs = []
+    run = torch.compile(_ConvOfAnyWidth(), backend=lambda g, _: graphs.append(g) or g.forward, dynamic=True,
+                        fullgraph=True)
+    for heads in (2, 3, 5):
+        assert run(_meta(2, 5, 96 * heads), _meta(96 * heads, 4))[0].shape == (2, 5, 32 * heads)
+    assert len(graphs) == 1
+    heads = torch.export.Dim("heads", min=2, max=64)
+    program = torch.export.export(_ConvOfAnyWidth(), (_meta(2, 5, 384), _meta(384, 4)),
+                                  dynamic_shapes=({2: 96 * heads}, {0: 96 * heads}))
+    assert program.module()(_meta(2, 5, 576), _meta(576, 4))[0].shape == (2, 5, 192)
+    ops = torch.ops.pkda_mi355x
+    for op in (ops.pkda_qkv_conv, ops.pkda_qkv_conv_backward, ops.pkda_controls_act, ops.pkda_controls_backward,
+               ops.qkv_conv_cached_):
+        assert " int " not in str(op.default._schema) and "SymInt" in str(op.default._schema)
+
+
 def test_cpu_tensors_are_refused():
     x = torch.zeros(5, 64)
     with pytest.raises(NotImplementedError, match="CPU"):

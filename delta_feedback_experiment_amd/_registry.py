@@ -9,8 +9,8 @@ schema defaults filled in, alias and disabled-kernel checks around the
 kernel) took about half of the 33 us of each operator of a decode token, and
 more for the training operator, whose outputs hold a list.
 
-The dispatcher's own order is kept: autograd, then tracing modes and
-functionalization, then the device kernel, so fake tensors, ``torch.compile``,
+The dispatcher's own order is kept: autograd, version counters, then tracing
+modes and functionalization, then the device kernel, so fake tensors, ``torch.compile``,
 saved-tensor hooks and the refusal of CPU tensors work as for any operator.
 """
 
@@ -22,30 +22,43 @@ from torch import Tensor, _C
 _LIBRARY = torch.library.Library("pkda_mi355x", "FRAGMENT")
 
 
+_WRITTEN: dict = {}  # operator -> positions of the arguments it writes
+
+
 def device_op(schema: str):
     """Decorator: register ``fn`` as the device kernel of ``schema`` (``name(args)
     -> returns``) and return the operator.  Arguments the schema marks as
-    written have their version counters raised after the kernel's launches."""
+    written have their version counters raised, whichever kernel runs."""
 
     def register(fn):
         name = schema.split("(", 1)[0]
         _LIBRARY.define(schema, tags=(torch.Tag.pt2_compliant_tag,))
         op = getattr(torch.ops.pkda_mi355x, name).default
-        written = [i for i, a in enumerate(op._schema.arguments) if a.alias_info is not None and a.alias_info.is_write]
-
-        def mutating(*args):
-            out = fn(*args)
-            for i in written:
-                t = args[i]
-                if t is not None and not t.is_inference():
-                    torch.autograd.graph.increment_version(t)
-            return out
-
-        _LIBRARY.impl(name, mutating if written else fn, "CUDA")
+        _WRITTEN[op] = [i for i, a in enumerate(op._schema.arguments)
+                        if a.alias_info is not None and a.alias_info.is_write]
+        _LIBRARY.impl(name, fn, "CUDA")
+        if _WRITTEN[op]:
+            _versions(op, name)
         _autograd(op, name)
         return op
 
     return register
+
+
+def _raise_versions(op, args) -> None:
+    for i in _WRITTEN[op]:
+        t = args[i]
+        if t is not None and not t.is_inference():
+            torch.autograd.graph.increment_version(t)
+
+
+def _versions(op, name: str) -> None:
+    def kernel(keyset, *args):
+        _raise_versions(op, args)
+        with _C._AutoDispatchBelowADInplaceOrView():
+            return op.redispatch(keyset & _C._after_ADInplaceOrView_keyset, *args)
+
+    _LIBRARY.impl(name, kernel, "ADInplaceOrView", with_keyset=True)
 
 
 def register_fake(op, fn) -> None:
@@ -104,10 +117,11 @@ def _autograd(op, name: str) -> None:
 
 
 def call(op, *args):
-    """``op(*args)``, past the autograd key when nothing asks for gradients:
-    the same dispatch below it, without the round trip through the autograd
-    kernel above.  (Dynamo traces the plain call.)"""
+    """``op(*args)``, past the autograd and version keys when nothing asks for
+    gradients: the same dispatch below them, without the round trips through
+    the kernels above.  (Dynamo traces the plain call.)"""
     if torch.compiler.is_compiling() or (_C.is_grad_enabled() and _C._any_requires_grad(*args)):
         return op(*args)
-    with _C._AutoDispatchBelowAutograd():
+    _raise_versions(op, args)
+    with _C._AutoDispatchBelowADInplaceOrView():
         return op(*args)

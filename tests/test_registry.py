@@ -7,7 +7,10 @@ from __future__ import annotations
 import pytest
 import torch
 
-from delta_feedback_experiment_amd import _registry, pkda_controls, pkda_norm_gate, pkda_qkv_conv, pkda_recurrence
+from torch._subclasses.fake_tensor import FakeTensorMode
+
+from delta_feedback_experiment_amd import (_registry, pkda_controls, pkda_norm_gate, pkda_qkv_conv,
+                                           pkda_qkv_conv_cached_, pkda_recurrence)
 from delta_feedback_experiment_amd.serve import qkv_conv_cached_op
 
 
@@ -73,6 +76,43 @@ def test_saved_tensor_hooks_see_the_inputs():
         q, k, v = pkda_qkv_conv(x, w, 32, 64, 1e-6)
     assert packed == [(2, 5, 96), (96, 4)]
     torch.autograd.grad((q, k, v), (x, w), [torch.empty_like(t) for t in (q, k, v)])
+
+
+def _cached_calls(x, pool):
+    """The ways into one writing operator: its public function and itself."""
+    w = _meta(96, 4)
+    return (lambda: pkda_qkv_conv_cached_(x, w, 32, 64, 1e-6, pool),
+            lambda: qkv_conv_cached_op(x, w, 32, 64, 1e-6, pool, None, True))
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("inference", [False, True])
+def test_written_tensors_change_version_without_a_device(grad, inference):
+    """Once per call, whatever kernel stands in for the device's."""
+    pool = _meta(4, 3, 96)
+    for call in _cached_calls(_meta(2, 1, 96, grad=grad), pool):
+        before = pool._version
+        with torch.inference_mode(inference):
+            call()
+        assert pool._version == before + 1
+    with torch.inference_mode():  # tensors that count no versions
+        for call in _cached_calls(_meta(2, 1, 96), _meta(4, 3, 96)):
+            call()
+    with FakeTensorMode():
+        pool = torch.empty(4, 3, 96, device="meta")
+        before = pool._version
+        qkv_conv_cached_op(torch.empty(2, 1, 96, device="meta"), torch.empty(96, 4, device="meta"), 32, 64, 1e-6,
+                           pool, None, True)
+        assert pool._version == before + 1
+
+
+def test_saved_tensor_written_before_backward_raises():
+    for i in range(2):
+        pool = _meta(4, 3, 96)
+        y = (pool * _meta(4, 3, 96, grad=True)).sum()
+        _cached_calls(_meta(2, 1, 96), pool)[i]()
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            y.backward()
 
 
 class _ConvOfAnyWidth(torch.nn.Module):

@@ -16,30 +16,42 @@ saved-tensor hooks and the refusal of CPU tensors work as for any operator.
 
 from __future__ import annotations
 
+from functools import partial
+
 import torch
-from torch import Tensor, _C
+from torch import _C
 
-_LIBRARY = torch.library.Library("pkda_mi355x", "FRAGMENT")
-
+_LIBRARIES: dict[str, torch.library.Library] = globals().get("_LIBRARIES", {})  # one an operator, kept over a reload
 
 _WRITTEN: dict = {}  # operator -> positions of the arguments it writes
 
 
 def device_op(schema: str):
     """Decorator: register ``fn`` as the device kernel of ``schema`` (``name(args)
-    -> returns``) and return the operator.  Arguments the schema marks as
-    written have their version counters raised, whichever kernel runs."""
+    -> returns``) and return the operator, with ``fn``'s docstring and
+    ``custom_op``'s ways to add to it (``register_kernel`` for another device,
+    ``register_vmap``, ...).  Arguments the schema marks as written have their
+    version counters raised, whichever kernel runs.  A name defined again (its
+    module reloaded) replaces the operator."""
 
     def register(fn):
         name = schema.split("(", 1)[0]
-        _LIBRARY.define(schema, tags=(torch.Tag.pt2_compliant_tag,))
+        if name in _LIBRARIES:
+            _LIBRARIES.pop(name)._destroy()
+        lib = _LIBRARIES[name] = torch.library.Library("pkda_mi355x", "FRAGMENT")
+        lib.define(schema, tags=(torch.Tag.pt2_compliant_tag,))
         op = getattr(torch.ops.pkda_mi355x, name).default
         _WRITTEN[op] = [i for i, a in enumerate(op._schema.arguments)
                         if a.alias_info is not None and a.alias_info.is_write]
-        _LIBRARY.impl(name, fn, "CUDA")
+        lib.impl(name, fn, "CUDA")
         if _WRITTEN[op]:
-            _versions(op, name)
-        _autograd(op, name)
+            _versions(op, name, lib)
+        _autograd(op, name, lib)
+        op.__doc__ = fn.__doc__
+        for way in ("register_kernel", "register_vmap", "register_torch_dispatch"):
+            setattr(op, way, partial(getattr(torch.library, way), op, lib=lib))
+        op.register_fake = partial(torch.library.register_fake, op, lib=lib, allow_override=True)
+        op.register_autograd = lambda backward, *, setup_context=None: register_autograd(op, backward, setup_context)
         return op
 
     return register
@@ -52,30 +64,30 @@ def _raise_versions(op, args) -> None:
             torch.autograd.graph.increment_version(t)
 
 
-def _versions(op, name: str) -> None:
+def _versions(op, name: str, lib) -> None:
     def kernel(keyset, *args):
         _raise_versions(op, args)
         with _C._AutoDispatchBelowADInplaceOrView():
             return op.redispatch(keyset & _C._after_ADInplaceOrView_keyset, *args)
 
-    _LIBRARY.impl(name, kernel, "ADInplaceOrView", with_keyset=True)
+    lib.impl(name, kernel, "ADInplaceOrView", with_keyset=True)
 
 
 def register_fake(op, fn) -> None:
-    torch.library.register_fake(op.name(), fn, lib=_LIBRARY)
+    torch.library.register_fake(op.name(), fn, lib=_LIBRARIES[op._schema.name.split("::")[1]])
 
 
 def register_autograd(op, backward, setup_context) -> None:
     """Give ``op`` a backward formula, ``backward(ctx, *output_grads)`` and
     ``setup_context(ctx, inputs, output)`` as ``torch.library.register_autograd``
     takes them (a list output's gradients come one by one, after the others)."""
-    _FORMULAS[op] = (setup_context, backward)
+    _FORMULAS[op] = (setup_context or (lambda ctx, inputs, output: None), backward)
 
 
 _FORMULAS: dict = {}
 
 
-def _autograd(op, name: str) -> None:
+def _autograd(op, name: str, lib) -> None:
     returns = op._schema.returns
     listed = bool(returns) and isinstance(returns[-1].type, _C.ListType)  # its tensors become outputs one by one
 
@@ -84,28 +96,26 @@ def _autograd(op, name: str) -> None:
             return out
         return (*out[:-1], *out[-1]) if len(returns) > 1 else tuple(out)
 
-    class Operator(torch.autograd.Function):
-        @staticmethod
-        def forward(ctx, keyset, *args):
-            with _C._AutoDispatchBelowAutograd():
-                out = op.redispatch(keyset & _C._after_autograd_keyset, *args)
-            if op in _FORMULAS:
-                _FORMULAS[op][0](ctx, args, out)
-            return flat(out)
+    def forward(ctx, keyset, *args):
+        with _C._AutoDispatchBelowAutograd():
+            out = op.redispatch(keyset & _C._after_autograd_keyset, *args)
+        if op in _FORMULAS:
+            _FORMULAS[op][0](ctx, args, out)
+        return flat(out)
 
-        @staticmethod
-        def backward(ctx, *grads):
-            # under create_graph the formula's own operator, which has none, takes
-            # part in the graph and raises when a second derivative reaches it
-            if op not in _FORMULAS:
-                raise RuntimeError(f"Trying to backward through {op} but no autograd formula was registered.")
-            return (None, *_FORMULAS[op][1](ctx, *grads))
+    def backward(ctx, *grads):
+        # under create_graph the formula's own operator, which has none, takes
+        # part in the graph and raises when a second derivative reaches it
+        if op not in _FORMULAS:
+            raise RuntimeError(f"Trying to backward through {op} but no autograd formula was registered.")
+        return (None, *_FORMULAS[op][1](ctx, *grads))
 
-    Operator.__name__ = f"BackwardFor_pkda_mi355x_{name}"
+    function = type(f"pkda_mi355x_{name}", (torch.autograd.Function,),
+                    {"forward": staticmethod(forward), "backward": staticmethod(backward)})
 
     def kernel(keyset, *args):
         if _C.is_grad_enabled() and _C._any_requires_grad(*args):
-            out = Operator.apply(keyset, *args)
+            out = function.apply(keyset, *args)
             if not listed:
                 return out
             last = list(out[len(returns) - 1:])
@@ -113,7 +123,7 @@ def _autograd(op, name: str) -> None:
         with _C._AutoDispatchBelowAutograd():
             return op.redispatch(keyset & _C._after_autograd_keyset, *args)
 
-    _LIBRARY.impl(name, kernel, "Autograd", with_keyset=True)
+    lib.impl(name, kernel, "Autograd", with_keyset=True)
 
 
 def call(op, *args):

@@ -1,17 +1,21 @@
 """The operators' registration: what a backward through an operator without a
-formula, a second derivative and a CPU tensor raise, and the version counters
-of what an operator writes."""
+formula, a second derivative and a CPU tensor raise, the version counters of
+what an operator writes, symbolic sizes, and what can be added to one."""
 
 from __future__ import annotations
 
+import subprocess
+import sys
+
 import pytest
 import torch
-
 from torch._subclasses.fake_tensor import FakeTensorMode
 
 from delta_feedback_experiment_amd import (_registry, pkda_controls, pkda_norm_gate, pkda_qkv_conv,
                                            pkda_qkv_conv_cached_, pkda_recurrence)
 from delta_feedback_experiment_amd.serve import qkv_conv_cached_op
+
+from conftest import ROOT
 
 
 def _meta(*shape, grad=False):
@@ -144,6 +148,50 @@ def test_cpu_tensors_are_refused():
     x = torch.zeros(5, 64)
     with pytest.raises(NotImplementedError, match="CPU"):
         pkda_norm_gate(x, x, torch.ones(64), 1e-6)
+
+
+def test_operators_can_be_added_to_and_defined_again():
+    """custom_op's ways to add to an operator, its docstring, and a module that
+    defines it a second time."""
+
+    def define(factor):
+        @_registry.device_op("registry_test(Tensor x, float by) -> Tensor")
+        def registry_test(x, by):
+            """Scaled."""
+            raise AssertionError("no device here")
+
+        _registry.register_fake(registry_test, lambda x, by: torch.empty_like(x))
+        registry_test.register_kernel("cpu", lambda x, by: factor * by * x)
+        return registry_test
+
+    x = torch.randn(3, 4, requires_grad=True)
+    for factor in (2.0, 3.0):
+        op = define(factor)
+        assert op.__doc__ == "Scaled."
+        assert torch.equal(op(x, by=5.0), factor * 5.0 * x)
+        with pytest.raises(RuntimeError, match="no autograd formula"):
+            op(x, 5.0).sum().backward()
+        op.register_autograd(lambda ctx, dy: (factor * 5.0 * dy, None))
+        assert torch.equal(torch.autograd.grad(op(x, 5.0).sum(), x)[0], torch.full_like(x, factor * 5.0))
+        op.register_vmap(lambda info, in_dims, x, by: (op(x, by) + 1, in_dims[0]))
+        assert torch.equal(torch.vmap(lambda r: op(r, 5.0))(x.detach()), factor * 5.0 * x.detach() + 1)
+        assert op(_meta(3, 4), 5.0).shape == (3, 4)
+    assert pkda_norm_gate.__doc__.startswith("Fused RMSNorm")
+
+
+def test_operator_modules_reload():
+    program = """
+import importlib, torch
+from delta_feedback_experiment_amd import _registry, controls, conv, norm_gate, ops, pkda, serve
+for module in (_registry, pkda, controls, conv, norm_gate, ops, serve):
+    importlib.reload(module)
+meta = lambda *s: torch.empty(*s, device="meta", requires_grad=True)
+y, _ = norm_gate.pkda_norm_gate(meta(5, 64), meta(5, 64), meta(64), 1e-6)
+y.sum().backward()
+q, _, _ = serve.pkda_qkv_conv_cached_(meta(2, 1, 96), meta(96, 4), 32, 64, 1e-6, torch.empty(4, 3, 96, device="meta"))
+assert y.shape == (5, 64) and q.shape == (2, 1, 32)
+"""
+    subprocess.run([sys.executable, "-c", program], check=True, cwd=ROOT)
 
 
 @pytest.mark.gpu

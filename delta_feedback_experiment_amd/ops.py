@@ -117,14 +117,14 @@ def _check_inputs(q, k, v, g, g_atk, beta_atk, beta, A_log, dt_bias, log_atk_sca
 _GATE_STREAMS: dict[int, torch.cuda.Stream] = {}
 
 
-OVERLAP_ELEMENTS = 3 << 24
-"""Elements of q from which the gate's backward runs on its second stream.  A
-fork and a join each way cost the host 200 us a step, which a small call waits
-for, and the kernels share the memory's bandwidth once they are large: 2 M
-elements (1,000 tokens of 16 heads) 700 us a step overlapped, 480 in order; 8 M
-720 and 480; 34 M 1,318 and 1,300; 67 M 2,315 and 2,333 (measured with the
-forward's gate overlapped as well; it now runs in the preconditioner's local
-pass)."""
+OVERLAP_ELEMENTS = 1 << 26
+"""Elements of q from which the gate's backward runs on its second stream.  The
+fork and the join cost the host 50 to 120 us a step, which a small call waits
+for, and the two share the memory's bandwidth once they are large, so there is
+little to win.  A step in order and overlapped, us, 16 heads of 128 channels in
+BF16: 2 M elements 530 and 650; 8 M 530 and 583; 34 M 1,296 and 1,307; 50 M 1,995
+and 2,005; 67 M 2,322 and 2,318; 134 M 4,570 and 4,547 (32 heads of 64 channels
+67 M 2,859 and 2,853, in FP32 4,926 and 4,918)."""
 
 
 def _gate_stream(dev: torch.device) -> torch.cuda.Stream:

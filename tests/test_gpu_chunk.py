@@ -660,13 +660,13 @@ def test_pkda_recurrence_op_matches_oracle(dev, lean, seed):
 
 @pytest.mark.parametrize("lean", [False, True])
 def test_pkda_recurrence_graph_replays_match_eager(dev, lean):
-    """The production op runs the per-channel gate on a second stream beside
-    the preconditioner and joins it, in the forward and in the backward.
-    Captured in a HIP graph (after warm-up on a side stream, as torch's
-    capture requires) the fork and the join become graph dependencies: each
-    of three replays, with eager steps and synchronisations between them,
-    gives the eager call's output and ten gradients bit for bit, and so does
-    every eager step in between."""
+    """The production op captured in a HIP graph (after warm-up on a side
+    stream, as torch's capture requires): each of three replays, with eager
+    steps and synchronisations between them, gives the eager call's output and
+    ten gradients bit for bit, and so does every eager step in between.  At
+    this size everything runs on the caller's stream;
+    test_pkda_recurrence_overlap_same_bits runs the same with the gate's
+    backward on a second one, whose fork and join become graph edges."""
     from delta_feedback_experiment_amd import pkda_recurrence
 
     print(f"[gpu] pkda_recurrence graph replays lean={lean}", flush=True)
@@ -753,8 +753,8 @@ def test_production_key_gradient_handoff(dev):
 
 @pytest.mark.parametrize("lean", [False, True])
 def test_pkda_recurrence_overlap_same_bits(dev, lean, monkeypatch):
-    """The gate on its second stream (large calls) and on the caller's (small
-    ones): the same output and gradients bit for bit, and the overlapped form
+    """The gate's backward on its second stream (large calls) and on the caller's
+    (small ones): the same output and gradients bit for bit, and the overlapped form
     captured and replayed as the graph test above does for the other."""
     from delta_feedback_experiment_amd import ops
 

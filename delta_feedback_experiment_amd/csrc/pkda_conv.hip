@@ -48,7 +48,6 @@ constexpr int kCh = 4;          // channels of a thread
 constexpr int kGroup = 4;       // token rows loaded together
 constexpr int kTileFwd = 32;    // longest tiles, tokens
 constexpr int kTileBwd = 64;
-constexpr int kTokRows = 1;     // decode tokens of a thread
 constexpr int kFillWaves = 4096;  // four waves on every SIMD
 
 // Tokens of a workgroup's tile: the longest of long_tile, long_tile / 2 and
@@ -448,13 +447,13 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_bwd_kernel(ConvParams p
 
 // ---------------------------------------------------------------------------
 // decode tokens: rows of one token, each continuing its slot's history.  A
-// thread owns 4 channels of kTokRows rows: it loads its weights once, and
-// every row's W - 1 history rows and new projection row before computing;
-// out = the normalised silu(conv), and the slot's history shifts by one row
-// in place (each thread reads its channels' rows before writing them).  Bound
-// by the latency of one round of loads, so a row a thread: 256 rows of 3 x
-// 4,096 channels 10.3 us, 4 of 3 x 1,024 3.2 (two rows a thread 11.3 and 4.2;
-// eight rows of eight channels, the earlier form, 16.3 and 5.5).
+// thread owns 4 channels of one row: it loads its weights, W - 1 history rows
+// and new projection row before computing; out = the normalised silu(conv),
+// and the slot's history shifts by one row in place (each thread reads its
+// channels' rows before writing them).  Bound by the latency of one round of
+// loads, so a row a thread: 256 rows of 3 x 4,096 channels 10.8 us, 4 of 3 x
+// 1,024 3.3 (two rows a thread 11.3 and 4.2; eight rows of eight channels, the
+// earlier form, 15.8 and 5.5).
 // ---------------------------------------------------------------------------
 template <typename T, int W, int D>
 __global__ __launch_bounds__(kConvThreads) void qkv_conv_token_kernel(ConvParams p) {
@@ -464,61 +463,49 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_token_kernel(ConvParams
   const bool norm = c0 < p.norm_channels;
   float wt[CH][W];
   load_weights<CH, W>(p, c0, wt);
-  const int b0 = blockIdx.x * kTokRows;
-  const int nb = min(kTokRows, p.B - b0);
-  RawRow<T, CH> hr[kTokRows][W - 1], xr[kTokRows];
+  const int b = blockIdx.x;
+  const int64_t sb = p.slot ? p.slot[b] : b;
+  RawRow<T, CH> hr[W - 1], xr;
+  xr.load(static_cast<const T*>(p.x) + (int64_t)b * p.C + c0);
 #pragma unroll
-  for (int r = 0; r < kTokRows; ++r) {
-    if (r >= nb) break;
-    const int b = b0 + r;
-    const int64_t sb = p.slot ? p.slot[b] : b;
-    xr[r].load(static_cast<const T*>(p.x) + (int64_t)b * p.C + c0);
-#pragma unroll
-    for (int w = 0; w < W - 1; ++w) {
-      if (p.hist_in) {
-        hr[r][w].load(static_cast<const T*>(p.hist_in) + (sb * (W - 1) + w) * p.C + c0);
-      } else {
-        hr[r][w].zero();
-      }
+  for (int w = 0; w < W - 1; ++w) {
+    if (p.hist_in) {
+      hr[w].load(static_cast<const T*>(p.hist_in) + (sb * (W - 1) + w) * p.C + c0);
+    } else {
+      hr[w].zero();
     }
   }
+  float xt[CH], hist[W - 1][CH];
+  xr.unpack(xt);
 #pragma unroll
-  for (int r = 0; r < kTokRows; ++r) {
-    if (r >= nb) break;
-    const int b = b0 + r;
-    const int64_t sb = p.slot ? p.slot[b] : b;
-    float xt[CH], hist[W - 1][CH];
-    xr[r].unpack(xt);
+  for (int w = 0; w < W - 1; ++w) hr[w].unpack(hist[w]);
+  float y[CH];
 #pragma unroll
-    for (int w = 0; w < W - 1; ++w) hr[r][w].unpack(hist[w]);
-    float y[CH];
+  for (int j = 0; j < CH; ++j) {
+    float a = wt[j][W - 1] * xt[j];
 #pragma unroll
-    for (int j = 0; j < CH; ++j) {
-      float a = wt[j][W - 1] * xt[j];
+    for (int w = 0; w < W - 1; ++w) a += wt[j][w] * hist[w][j];
+    y[j] = a * sigmoid_fast(a);
+  }
+  if (norm) {
+    const float rn = rsqrtf(lane_pair_squares<G>(y) + p.eps);
 #pragma unroll
-      for (int w = 0; w < W - 1; ++w) a += wt[j][w] * hist[w][j];
-      y[j] = a * sigmoid_fast(a);
-    }
-    if (norm) {
-      const float rn = rsqrtf(lane_pair_squares<G>(y) + p.eps);
+    for (int j = 0; j < CH; ++j) y[j] *= rn;
+  }
+  int off;
+  T* out = slab_ptr<T>(p.q, p.k, p.v, p.P, c0, (int64_t)b, off) + off;
+  store_row<T, CH>(out, y);
+  if (p.hist_out) {
+    T* ho = static_cast<T*>(p.hist_out) + sb * (W - 1) * p.C + c0;
 #pragma unroll
-      for (int j = 0; j < CH; ++j) y[j] *= rn;
-    }
-    int off;
-    T* out = slab_ptr<T>(p.q, p.k, p.v, p.P, c0, (int64_t)b, off) + off;
-    store_row<T, CH>(out, y);
-    if (p.hist_out) {
-      T* ho = static_cast<T*>(p.hist_out) + sb * (W - 1) * p.C + c0;
-#pragma unroll
-      for (int w = 0; w + 1 < W - 1; ++w) store_row<T, CH>(ho + (int64_t)w * p.C, hist[w + 1]);
-      store_row<T, CH>(ho + (int64_t)(W - 2) * p.C, xt);
-    }
+    for (int w = 0; w + 1 < W - 1; ++w) store_row<T, CH>(ho + (int64_t)w * p.C, hist[w + 1]);
+    store_row<T, CH>(ho + (int64_t)(W - 2) * p.C, xt);
   }
 }
 
 // ---------------------------------------------------------------------------
 // cached rows longer than one forward tile: the history left for the next
-// call, the last W - 1 rows of history ++ x.  One thread per 8 channels of
+// call, the last W - 1 rows of history ++ x.  One thread per 4 channels of
 // one row reads every row it needs before writing any, so history_out may
 // alias history_in; it runs after the forward kernel (whose first tile of a
 // row reads history_in) on the same stream.
@@ -555,8 +542,7 @@ int launch_conv(const ConvParams& p, bool backward, hipStream_t s) {
   if (!backward) {
     if constexpr (W > 1) {
       if (p.T == 1 && (p.hist_in || p.hist_out)) {  // decode tokens
-        hipLaunchKernelGGL((qkv_conv_token_kernel<T, W, D>), dim3((p.B + kTokRows - 1) / kTokRows, cblocks),
-                           dim3(kConvThreads), 0, s, p);
+        hipLaunchKernelGGL((qkv_conv_token_kernel<T, W, D>), dim3(p.B, cblocks), dim3(kConvThreads), 0, s, p);
         return launch_status("pkda_qkv_conv_fwd(token)");
       }
     }

@@ -212,7 +212,7 @@ __global__ __launch_bounds__(NT) void gate_channel_fwd_kernel(GateParams p) {
 // ---- gate backward -------------------------------------------------------------
 // dglog[t] = sum_{s >= t in chunk} dgcum[s]; raw form also
 // dg = dglog * (-exp(A_log)) * sigmoid(g + dt_bias), dA_log += dglog * glog,
-// ddt_bias += dg.  Per-chunk partials, reduced by gate_reduce_kernel.
+// ddt_bias += dg.  Per-chunk partials, summed by column_sums_kernel.
 __global__ __launch_bounds__(64) void gate_bwd_kernel(GateParams p) {
   const int H = p.heads;
   const ChunkHead wg = chunk_head<true>(H);

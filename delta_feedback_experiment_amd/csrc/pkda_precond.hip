@@ -190,12 +190,12 @@ __device__ __forceinline__ float a_step(float eg, float a, float bt, float k) {
 }
 
 // Forward launches 1 (APPLY = false: local end A from zero into a_chunk) and
-// 3 (APPLY: A from a_chunk, kw out).  The chunk runs in sub-blocks of 8
-// tokens whose k rows load before their chain runs; a short chunk
-// (FULL = false) clamps its loads to its last token and leaves the state
-// unchanged past it, so no load sits behind a branch.
+// 3 (APPLY: A from a_chunk, kw out).  The chunk runs in groups of G tokens
+// whose k rows load before their chain runs; a short chunk (FULL = false)
+// clamps its loads to its last token and leaves the state unchanged past it,
+// so no load sits behind a branch.
 //
-// With GATE the local pass also walks the raw gate beside the key: its chunk
+// With GATE (BF16) the local pass also walks the raw gate beside the key: its chunk
 // cumsum -exp(A_log) sum softplus(g + dt_bias), the operations of
 // gate_channel_fwd_kernel in their order.  Both are one round of loads per
 // group and a short chain, so the second rides on the first's latency and a
@@ -203,8 +203,8 @@ __device__ __forceinline__ float a_step(float eg, float a, float bt, float k) {
 // in two launches; 12,001 tokens, 16 heads 44 against 31 + 35; 32,768 tokens, 16
 // heads 102, 220 with the scan and the last pass, against 200 for the gate on a
 // second stream beside all three, whose fork and join cost more than the 20
-// (the training step 2,324 -> 2,315).  Groups of 8, 16 or 32 tokens: within 3 %
-// (32 takes 110 at the large size).
+// (the training step 2,324 -> 2,315).  Groups of 8 and 16 tokens are within 3 %,
+// groups of 32 take 110 at the large size.
 template <typename T, int D, bool APPLY, bool FULL, bool GATE>
 __device__ __forceinline__ void precond_fwd_chunk(const PrecondParams& p, int j, int h, int start, int len) {
   constexpr int G = APPLY ? 8 : 16, CH = PrecondChunk<D>::CH;
@@ -627,10 +627,12 @@ int launch_precond(const PrecondParams& p, bool backward, hipStream_t s) {
     if (p.narrow_grads) launch_precond_bwd_chunks<T, D, T>(p, s);
     else launch_precond_bwd_chunks<T, D, float>(p, s);
   } else {
-    if (any && p.gate_raw)
-      hipLaunchKernelGGL((precond_fwd_chunk_kernel<T, D, false, true>), chunks, dim3(NTC), 0, s, p);
-    else if (any)
-      hipLaunchKernelGGL((precond_fwd_chunk_kernel<T, D, false, false>), chunks, dim3(NTC), 0, s, p);
+    if (any) {
+      auto local = precond_fwd_chunk_kernel<T, D, false, false>;
+      if constexpr (std::is_same<T, bf16_t>::value)
+        if (p.gate_raw) local = precond_fwd_chunk_kernel<T, D, false, true>;
+      hipLaunchKernelGGL(local, chunks, dim3(NTC), 0, s, p);
+    }
     hipLaunchKernelGGL((precond_fwd_scan_kernel<D>), docs, dim3(NT), 0, s, p);
     if (any) hipLaunchKernelGGL((precond_fwd_chunk_kernel<T, D, true, false>), chunks, dim3(NTC), 0, s, p);
   }
@@ -656,6 +658,7 @@ extern "C" int pkda_precond_fwd(const pkda_precond_args* a, void* stream) {
   if (int st = precond_common(a, p)) return st;
   if (a->num_seqs == 0) return 0;
   PKDA_REQUIRE(a->kw && a->a_chunk, PKDA_EINVAL, "preconditioner forward needs kw and a_chunk");
+  PKDA_REQUIRE(!a->gate_raw || a->dtype == PKDA_BF16, PKDA_EUNSUPPORTED, "the raw gate is summed for BF16 keys");
   PKDA_REQUIRE(!a->gate_raw || (a->gate_A_log && a->gate_dt_bias && a->gcum), PKDA_EINVAL,
                "the raw gate needs A_log, dt_bias and gcum");
   hipStream_t s = static_cast<hipStream_t>(stream);

@@ -48,7 +48,7 @@ def precond_forward(plan, kf: Tensor, g_atk: Tensor, beta_atk: Tensor, center: T
     (the chunk backward with per-channel gates sums its in-block pairs from
     them).  ``handoff=False`` passes no chunk-decay workspace: the document
     scan then sums every chunk's g_atk itself (the same bits, more loads).
-    ``gate``: the raw per-channel gate in ``kf``'s dtype, A_log and dt_bias
+    ``gate`` (BF16): the raw per-channel gate in ``kf``'s dtype, A_log and dt_bias
     (FP32) and the buffer ``[N_tok, H, K]`` FP32 for its chunk cumsum, which the
     local pass then forms beside its own (``gate_forward``'s bits)."""
     dev = kf.device

@@ -296,8 +296,8 @@ typedef struct pkda_precond_args {
                                     exp(sum of g_atk), written by the local chunk pass and read
                                     by the document scan (which otherwise sums every chunk's
                                     g_atk again); the same bits either way */
-  const void* gate_raw;          /* forward, optional: the raw per-channel gate [N_tok,H,K] in
-                                    dtype, activated and summed within each chunk by the local
+  const void* gate_raw;          /* forward, BF16, optional: the raw per-channel gate [N_tok,H,K],
+                                    BF16 and 4-byte aligned, activated and summed within each chunk by the local
                                     chunk pass, in pkda_gate_fwd's place (PKDA_GATE_RAW_CHANNEL
                                     without gcum_lo; the same bits) */
   const float* gate_A_log;       /* [H] */

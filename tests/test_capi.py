@@ -105,3 +105,15 @@ def test_packed_triangular_refused_outside_its_configuration():
         args = _lib.ChunkBwdArgs(dtype=dtype, **geo, kw=kw, tri_packed=1, **fake, **grads)
         with pytest.raises(ValueError, match="tri_packed"):
             _lib.call("pkda_chunk_bwd", args, 0)
+
+
+def test_raw_gate_refused_outside_bf16():
+    """The preconditioner's local pass sums the raw gate for BF16 keys (FP32
+    also wants the cumsum's remainder); refused before any HIP call."""
+    from delta_feedback_experiment_amd import _lib
+
+    args = _lib.PrecondArgs(dtype=_lib.PKDA_F32, num_seqs=1, seqlen=64, heads=1, head_dim=64, num_chunks=1,
+                            squash_x=1.5, k=16, g_atk=32, beta_atk=48, center=64, kw=80, a_chunk=96,
+                            gate_raw=112, gate_A_log=128, gate_dt_bias=144, gcum=160)
+    with pytest.raises(ValueError, match="raw gate"):
+        _lib.call("pkda_precond_fwd", args, 0)

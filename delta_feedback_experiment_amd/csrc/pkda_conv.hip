@@ -30,8 +30,8 @@
 //
 // Bounds: HBM, with the VALU close behind (90 operations a thread and row
 // forward, 125 backward).  B8 T4096, 3 x 1,024 channels, W = 4, BF16: forward
-// 80 us for 403 MB (5.0 TB/s, the card's copy rate 5.2), backward 143 for 604
-// MB and 25 of dw partials (4.4 TB/s, 112 VGPRs, four waves a SIMD).  Eight
+// 79 us for 403 MB (5.1 TB/s, the card's copy rate 5.2), backward 141 for 604
+// MB and 25 of dw partials (4.5 TB/s, 112 VGPRs, four waves a SIMD).  Eight
 // channels a thread, row tests and IEEE divisions in the sigmoids took 109
 // and 184 (227 VGPRs, two waves); eight channels in today's form 80 and 190,
 // but 15.4 us against 14 on 3 rows of 1,000 tokens.
@@ -43,7 +43,11 @@
 namespace pkda {
 namespace {
 
-constexpr int kConvThreads = 128;
+// A workgroup's piece of a row is 2 KB of BF16 and 4 KB of FP32 with 256 threads,
+// contiguous; half of that costs FP32 6 to 10 % (8 x 4,096 rows of 3,072 channels,
+// forward 169 us against 154, backward 284 against 264; 8 x 4,000 rows 162
+// against 150 and 296 against 266), BF16 up to 1 %.
+constexpr int kConvThreads = 256;
 constexpr int kCh = 4;          // channels of a thread
 constexpr int kGroup = 4;       // token rows loaded together
 constexpr int kTileFwd = 32;    // longest tiles, tokens

@@ -203,11 +203,12 @@ __device__ __forceinline__ float a_step(float eg, float a, float bt, float k) {
 // in two launches; 12,001 tokens, 16 heads 44 against 31 + 35; 32,768 tokens, 16
 // heads 102, 220 with the scan and the last pass, against 200 for the gate on a
 // second stream beside all three, whose fork and join cost more than the 20
-// (the training step 2,324 -> 2,315).  Groups of 8 and 16 tokens are within 3 %,
-// groups of 32 take 110 at the large size.
+// (the training step 2,324 -> 2,315).  With the gate, groups of 8 and 16 tokens are
+// within 3 %, groups of 32 take 110 at the large size; without it groups of 16 cost
+// small calls up to 10 % (BF16, 3 rows of 1,000 tokens, 8 heads 9.1 us against 10.2).
 template <typename T, int D, bool APPLY, bool FULL, bool GATE>
 __device__ __forceinline__ void precond_fwd_chunk(const PrecondParams& p, int j, int h, int start, int len) {
-  constexpr int G = APPLY ? 8 : 16, CH = PrecondChunk<D>::CH;
+  constexpr int G = GATE ? 16 : 8, CH = PrecondChunk<D>::CH;
   using IO = ChanIO<T, CH>;
   using FIO = ChanIO<float, CH>;
   const int H = p.H, c0 = CH * threadIdx.x;

@@ -2459,8 +2459,8 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_state_bwd_split_kernel(Bwd
 
 template <int D, bool PACK>
 int launch_state_bwd_split(const BwdParams& p, hipStream_t s) {
-  auto kern = state_pass_workgroups(p.geom, p.H, D / 32) <= kDeferHead ? chunk_state_bwd_split_kernel<D, 32, PACK, true>
-                                                                       : chunk_state_bwd_split_kernel<D, 32, PACK, false>;
+  auto kern = defer_head_reverse(p.geom, p.H, D) ? chunk_state_bwd_split_kernel<D, 32, PACK, true>
+                                                 : chunk_state_bwd_split_kernel<D, 32, PACK, false>;
   constexpr int bytes = RrSplitBwdLayout<D, 32>::bytes;
   if (int st = set_smem(kern, bytes)) return st;
   hipLaunchKernelGGL(kern, doc_grid(p.geom.num_seqs, p.H, D / 32), dim3(64 * (4 + kSplitLoaders)), bytes, s, p);
@@ -2929,7 +2929,7 @@ int launch_state_bwd_rr_pc(const BwdParams& p, hipStream_t s) {
   const int N = p.geom.num_seqs;
   if (N <= 0) return 0;
   const bool narrow = (int64_t)N * p.H * (D / 64) < 256;
-  const bool split = narrow && state_pass_workgroups(p.geom, p.H, D / 32) <= kSplitChannelReverse;
+  const bool split = narrow && split_channel_reverse(p.geom, p.H, D);
   auto kern = split    ? chunk_state_bwd_split_pc_kernel<D, 32>
               : narrow ? chunk_state_bwd_rr_pc_kernel<D, 32>
                        : chunk_state_bwd_rr_pc_kernel<D, 64>;

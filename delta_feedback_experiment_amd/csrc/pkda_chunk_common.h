@@ -959,30 +959,32 @@ constexpr int kSplitLoaders = 4;  // two groups of two waves
 // which it staged a chunk (DEFER), not right behind the staging.  Staging takes
 // a group 2,450 cycles of a step and sending 2,020, so both in a row hold the
 // barrier up past the chain's 3,500; deferred, the loads are in flight for one
-// step instead of two, which covers their latency until most compute units
-// stream.  Measured, us: the form without output waves / split, not deferred /
-// split, deferred, at D = 128 and 32 chunks a row unless noted:
-//   workgroups             64                 128              192              224
-//   per head, forward      80.5 61.2 53.6     80.2 61.0 53.8   81.0 62.6 61.4   81.1 63.5 63.5
-//   per head, reverse      71.0 61.8 60.5     71.0 61.9 60.5   70.8 62.6 61.0   71.3 62.9 61.5
-//   per channel, forward   59.8 60.1 50.8     61.6 61.5 65.1   90.6 83.2 93.9   102.9 102.5 115
-//   per channel, reverse   56.8 56.0 45.5     57.7 57.8 54.7   60.0 60.1 61.0   61.1 63.2 64.6
-// 256 workgroups of 256 chunks, per head: forward 606 568 703, reverse 561 512
-// 642.  One prompt of 24 chunks, 32 workgroups, per channel: forward 46.4 47.8 37.4.
-// So per head the split form always, deferred to kDeferHead.
-//
-// Per channel the form without output waves is the better one past some count:
-// the output stage it has room for is worth more than the shorter chain once
-// the loads take their time.  Without output waves / split, 32 chunks a row:
-//   workgroups             80         96         112        128        160        192        256
-//   forward, D = 128       60.1 54.6  60.4 55.7  61.0 57.0  62.0 62.7  69.0 68.6  94.1 94.0  120 121
-//   forward, D = 64        41.0 34.5  41.5 34.8  42.6 36.0  43.0 38.9  56.0 53.0  76.7 79.2  91.0 91.4
-//   reverse, D = 128       54.8 48.5  54.2 55.0  55.6 59.1  56.3 60.9  62.8 63.1  71.3 71.3  100 99.3
-//   reverse, D = 64        34.9 29.3  35.2 36.9  39.6 40.6  41.2 42.8  43.8 42.6  49.0 48.5  64.6 63.8
-// Forward, 256 workgroups of 256 chunks 624 649; packed documents, 12,000 tokens
-// of 16 heads, 5 documents (320 workgroups) 189 196, 7 documents 164 169.
-// So forward split (deferred to kDeferChannel) to kSplitChannelForward, reverse
-// split, always deferred, to kSplitChannelReverse.
+// step instead of two.  That covers their latency while the rows, which the
+// intra kernel has just written, are in the memory's cache or few workgroups
+// read, so what decides is the call's elements (tokens x heads x channels, Mi =
+// 2^20) more than its workgroups.  Measured, us: without output waves / split, not
+// deferred / split, deferred (per channel always: not deferred it nowhere beat
+// the better of the two by more than 2 %).
+//   D = 128, workgroups x tokens a row   64 x 2,048    160 x 2,048    256 x 2,048    96 x 8,192     128 x 8,192
+//   elements                             4 Mi          10 Mi          16 Mi          24 Mi          32 Mi
+//   per head, forward                    81 60 53      80 60 54       83 69 72       303 223 213    303 236 259
+//   per head, reverse                    71 62 59      70 62 60       73 65 63       266 227 220    268 229 248
+//   per channel, forward                 60 52         66 60          104 118        287 355        289 364
+//   per channel, reverse                 55 45         56 57          63 68          213 238        225 262
+//   D = 128, long rows                   32 x 16,384   64 x 16,384    128 x 16,384   64 x 49,152
+//   elements                             16 Mi         32 Mi          64 Mi          96 Mi
+//   per head, forward                    597 439 385   599 447 459    600 498 610    1810 1370 1593
+//   per head, reverse                    525 446 433   529 447 456    528 455 536    1590 1345 1447
+//   per channel, forward                 443 502       502 642        557 707        1451 1883
+//   per channel, reverse                 399 370       427 472        461 551        1329 1553
+//   D = 64                               64 x 2,048    160 x 2,048    256 x 2,048    48 x 8,192     64 x 16,384
+//   elements                             4 Mi          10 Mi          16 Mi          12 Mi          32 Mi
+//   per head, forward                    65 42 43      66 42 45       68 60 61       249 151 175    492 357 449
+//   per head, reverse                    57 47 44      59 47 45       60 50 55       217 171 161    430 339 399
+//   per channel, forward                 41 38         43 42          89 96          153 161        473 527
+//   per channel, reverse                 35 30         43 46          49 56          135 145        313 358
+// Short rows (256 to 1,024 tokens, up to 448 workgroups) as their elements say: 12
+// rows of 1,024, 4 heads, per channel at D = 128, 6 Mi: forward 35 31, reverse 33 33.
 //
 // All of these take 32 columns a workgroup, where 64 make fewer workgroups than
 // compute units.  A workgroup's LDS fills its compute unit, so 257 to 510 of
@@ -991,7 +993,21 @@ constexpr int kSplitLoaders = 4;  // two groups of two waves
 // 137 against 98, reverse 136 against 85) but slower for packed documents, whose
 // longest one is the time (5 documents of 12,000 tokens: 137 against 219, 138
 // against 189); the count does not tell them apart.
-constexpr int kDeferHead = 192, kDeferChannel = 112, kSplitChannelForward = 160, kSplitChannelReverse = 80;
-inline int64_t state_pass_workgroups(const ChunkGeom& g, int H, int slices) { return (int64_t)g.num_seqs * H * slices; }
+inline int64_t state_pass_workgroups(const ChunkGeom& g, int H, int D) { return (int64_t)g.num_seqs * H * (D / 32); }
+inline int64_t state_pass_mi(const ChunkGeom& g, int H, int D) {  // rounded up
+  return ((int64_t)g.num_chunks * C * H * D + (1 << 20) - 1) >> 20;
+}
+// Per head: always split.
+inline bool defer_head_forward(const ChunkGeom& g, int H, int D) {
+  const int64_t mi = state_pass_mi(g, H, D);
+  return D == 128 && (mi <= 8 || (mi <= 24 && state_pass_workgroups(g, H, D) <= 160));
+}
+inline bool defer_head_reverse(const ChunkGeom& g, int H, int D) { return state_pass_mi(g, H, D) <= (D == 128 ? 24 : 12); }
+// Per channel: split and deferred, or neither (past this the output stage that the
+// form without output waves has room for is worth more than the shorter chain).
+inline bool split_channel_forward(const ChunkGeom& g, int H, int D) { return state_pass_mi(g, H, D) <= 8; }
+inline bool split_channel_reverse(const ChunkGeom& g, int H, int D) {
+  return state_pass_mi(g, H, D) <= (D == 128 && state_pass_workgroups(g, H, D) <= 64 ? 16 : 6);
+}
 
 }  // namespace pkda

@@ -2041,7 +2041,7 @@ struct RrPcSplitLayout : RrPcFwdLayout<D, BV> {
   static_assert(bytes <= 160 * 1024, "LDS of one compute unit");
 };
 
-template <int D, int BV, bool DEFER>
+template <int D, int BV>
 __global__ __launch_bounds__(64 * (2 * (BV / 16) + kSplitLoaders))
 __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_state_fwd_split_pc_kernel(FwdParams p) {
   using L = RrPcSplitLayout<D, BV>;
@@ -2099,16 +2099,12 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_state_fwd_split_pc_kernel(
     if (lgroup < count) load(lgroup);
     if (lgroup == 0 && count > 0) {
       stash(0);
-      if (!DEFER && count > 2) load(2);
     }
-    for (int jc = 0; jc <= count; ++jc) {
+    for (int jc = 0; jc <= count; ++jc) {  // the loads deferred (pkda_chunk_common.h)
       __syncthreads();
       if (((jc + 1) & 1) == lgroup) {
-        if (jc + 1 < count) {
-          stash((jc + 1) & 1);
-          if (!DEFER && jc + 3 < count) load(jc + 3);
-        }
-      } else if (DEFER && jc + 2 < count) {
+        if (jc + 1 < count) stash((jc + 1) & 1);
+      } else if (jc + 2 < count) {
         load(jc + 2);
       }
     }
@@ -2282,8 +2278,9 @@ int launch_state_fwd_rr_as(const FwdParams& p, hipStream_t s) {
 
 template <int D, bool PACK>
 int launch_state_fwd_split(const FwdParams& p, hipStream_t s) {
-  auto kern = state_pass_workgroups(p.geom, p.H, D / 32) <= kDeferHead ? chunk_state_fwd_split_kernel<D, 32, PACK, true>
-                                                                       : chunk_state_fwd_split_kernel<D, 32, PACK, false>;
+  auto kern = chunk_state_fwd_split_kernel<D, 32, PACK, false>;
+  if constexpr (D == 128)
+    if (defer_head_forward(p.geom, p.H, D)) kern = chunk_state_fwd_split_kernel<D, 32, PACK, true>;
   constexpr int bytes = RrSplitLayout<D, 32>::bytes;
   if (int st = set_smem(kern, bytes)) return st;
   hipLaunchKernelGGL(kern, doc_grid(p.geom.num_seqs, p.H, D / 32), dim3(64 * (4 + kSplitLoaders)), bytes, s, p);
@@ -2309,12 +2306,10 @@ int launch_state_fwd_rr_pc(const FwdParams& p, hipStream_t s) {
   const int N = p.geom.num_seqs;
   if (N <= 0) return 0;
   const bool narrow = (int64_t)N * p.H * (D / 64) < 256;
-  const int64_t workgroups = state_pass_workgroups(p.geom, p.H, D / 32);
-  const bool split = narrow && workgroups <= kSplitChannelForward;
-  auto kern = split && workgroups <= kDeferChannel ? chunk_state_fwd_split_pc_kernel<D, 32, true>
-              : split                              ? chunk_state_fwd_split_pc_kernel<D, 32, false>
-              : narrow                             ? chunk_state_fwd_rr_pc_kernel<D, 32>
-                                                   : chunk_state_fwd_rr_pc_kernel<D, 64>;
+  const bool split = narrow && split_channel_forward(p.geom, p.H, D);
+  auto kern = split    ? chunk_state_fwd_split_pc_kernel<D, 32>
+              : narrow ? chunk_state_fwd_rr_pc_kernel<D, 32>
+                       : chunk_state_fwd_rr_pc_kernel<D, 64>;
   const int bytes = split    ? RrPcSplitLayout<D, 32>::bytes
                     : narrow ? RrPcFwdLayout<D, 32>::bytes
                              : RrPcFwdLayout<D, 64>::bytes;

@@ -781,13 +781,13 @@ def test_pkda_recurrence_overlap_same_bits(dev, lean, monkeypatch):
 @pytest.mark.parametrize("per_channel", [False, True])
 def test_state_pass_forms_agree(dev, D, per_channel):
     """The state passes with 64 columns a workgroup (320 rows x heads) and the
-    narrower ones in each of their dispatches.  Workgroups of 32 columns, 2 per
-    row and head at D = 64 and 4 at D = 128: 360 and 448 (past one a compute
-    unit), 280 and 140, 224 and 112, 120 and 60, 56 and 28 (with and without
-    output waves, loads deferred and not).
-    Rows of one token, of two whole chunks and a partial one, of six whole
-    chunks and of six and a partial one (a loader group sends its loads three
-    chunks ahead); initial and final states.  All forms take every value by the
+    narrower ones in each of their dispatches, which go by a call's elements
+    and workgroups of 32 columns (2 per row and head at D = 64, 4 at D = 128):
+    with and without output waves, loads deferred and not, up to 448
+    workgroups, past one a compute unit.  Rows of one token, of two whole
+    chunks and a partial one, of six whole chunks and of six and a partial one
+    (a loader group sends its loads three chunks ahead), and rows long enough
+    for the forms of the largest calls.  All forms take every value by the
     same operations in the same order, so outputs, states and gradients agree
     bit for bit: what a row and head gets does not depend on what else is in
     the call."""
@@ -799,7 +799,8 @@ def test_state_pass_forms_agree(dev, D, per_channel):
     def rn(*s):
         return torch.randn(*s, generator=gen, device=dev)
 
-    for T in (1, 150, 384, 400):
+    many = (12, 15) if D == 64 else (8, 14)
+    for T in (1, 150, 384, 400, 1170 if D == 64 else 1850):
         B, H = 20, 16
         q, k = (torch.nn.functional.normalize(rn(B, T, H, D), dim=-1).to(torch.bfloat16) for _ in range(2))
         v, do = rn(B, T, H, D).to(torch.bfloat16), rn(B, T, H, D).to(torch.bfloat16)
@@ -814,7 +815,7 @@ def test_state_pass_forms_agree(dev, D, per_channel):
             return [o.detach(), *gr[:5]], [S.detach(), gr[5]]
 
         wide = step(B, H)
-        for rows, heads in ((12, 15) if D == 64 else (8, 14), (8, 14), (5, 14), (4, 14), (3, 10), (1, 14)):
+        for rows, heads in (many,) if T > 400 else (many, (8, 14), (5, 14), (4, 14), (3, 10), (1, 14)):
             tokens, states = step(rows, heads)
             want = ([t[:rows, :, :heads] for t in wide[0]], [t[:rows, :heads] for t in wide[1]])
             for name, a, b in zip(("o", "dq", "dk", "dv", "dg", "dbeta", "S", "dS0"), (*tokens, *states),

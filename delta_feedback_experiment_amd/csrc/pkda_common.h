@@ -61,8 +61,9 @@ __device__ __forceinline__ float log_fast(float x) { return __builtin_amdgcn_log
 // a / b as a * (1 / b) on the hardware reciprocal (v_rcp_f32, 1 ulp).
 __device__ __forceinline__ float div_fast(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
 
-// 1 / d for d >= 1: the hardware reciprocal and one Newton step, within an ulp
-// as a division is, in five operations instead of eleven.  Infinity and NaN
+// 1 / d for d >= 1: the hardware reciprocal and one Newton step, the division's
+// result but for 3 of the 2^23 mantissas (32 where the reciprocal is an ulp
+// high), in five operations instead of eleven.  Infinity and NaN
 // (and d past 2^126, whose reciprocal is not a normal number) keep the
 // hardware's own result, 0 or NaN, which the step would turn into NaN.
 __device__ __forceinline__ float recip_from_one(float d) {

@@ -30,9 +30,9 @@
 //
 // Bounds: HBM, with the VALU close behind (90 operations a thread and row
 // forward, 125 backward).  B8 T4096, 3 x 1,024 channels, W = 4, BF16: forward
-// 79 us for 403 MB (5.1 TB/s, the card's copy rate 5.2), backward 141 for 604
-// MB and 25 of dw partials (4.5 TB/s, 112 VGPRs, four waves a SIMD).  Eight
-// channels a thread, row tests and IEEE divisions in the sigmoids took 109
+// 82 us for 403 MB (4.9 TB/s, the card's copy rate 5.2), backward 144 for 604
+// MB and 25 of dw partials (4.4 TB/s, 112 VGPRs, four waves a SIMD).  Eight
+// channels a thread, row tests and IEEE divisions in the sigmoids took 105
 // and 184 (227 VGPRs, two waves); eight channels in today's form 80 and 190,
 // but 15.4 us against 14 on 3 rows of 1,000 tokens.
 #include "pkda_common.h"
@@ -455,9 +455,9 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_bwd_kernel(ConvParams p
 // and new projection row before computing; out = the normalised silu(conv),
 // and the slot's history shifts by one row in place (each thread reads its
 // channels' rows before writing them).  Bound by the latency of one round of
-// loads, so a row a thread: 256 rows of 3 x 4,096 channels 10.8 us, 4 of 3 x
-// 1,024 3.3 (two rows a thread 11.3 and 4.2; eight rows of eight channels, the
-// earlier form, 15.8 and 5.5).
+// loads, so a row a thread: 256 rows of 3 x 4,096 channels, histories among 512
+// slots, 12 us, 4 of 3 x 1,024 3.3 (two rows a thread 10 and 30 % more; eight
+// rows of eight channels, the earlier form, 18 and 5.5).
 // ---------------------------------------------------------------------------
 template <typename T, int W, int D>
 __global__ __launch_bounds__(kConvThreads) void qkv_conv_token_kernel(ConvParams p) {

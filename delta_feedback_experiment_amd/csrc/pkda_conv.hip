@@ -451,8 +451,9 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_bwd_kernel(ConvParams p
 
 // ---------------------------------------------------------------------------
 // decode tokens: rows of one token, each continuing its slot's history.  A
-// thread owns 4 channels of one row: it loads its weights, W - 1 history rows
-// and new projection row before computing; out = the normalised silu(conv),
+// thread owns 4 channels of one row: it loads its W - 1 history rows, new
+// projection row and (last: the rows' loads wait for the slot) weights before
+// computing; out = the normalised silu(conv),
 // and the slot's history shifts by one row in place (each thread reads its
 // channels' rows before writing them).  Bound by the latency of one round of
 // loads, so a row a thread: 256 rows of 3 x 4,096 channels, histories among 512
@@ -465,8 +466,6 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_token_kernel(ConvParams
   const int c0 = (blockIdx.y * kConvThreads + threadIdx.x) * CH;
   if (c0 >= p.C) return;
   const bool norm = c0 < p.norm_channels;
-  float wt[CH][W];
-  load_weights<CH, W>(p, c0, wt);
   const int b = blockIdx.x;
   const int64_t sb = p.slot ? p.slot[b] : b;
   RawRow<T, CH> hr[W - 1], xr;
@@ -479,6 +478,8 @@ __global__ __launch_bounds__(kConvThreads) void qkv_conv_token_kernel(ConvParams
       hr[w].zero();
     }
   }
+  float wt[CH][W];
+  load_weights<CH, W>(p, c0, wt);
   float xt[CH], hist[W - 1][CH];
   xr.unpack(xt);
 #pragma unroll

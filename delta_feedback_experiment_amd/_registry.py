@@ -21,9 +21,10 @@ from functools import partial
 import torch
 from torch import _C
 
-_LIBRARIES: dict[str, torch.library.Library] = globals().get("_LIBRARIES", {})  # one an operator, kept over a reload
-
-_WRITTEN: dict = {}  # operator -> positions of the arguments it writes
+# kept over a reload of this module, which leaves the operators standing
+_LIBRARIES: dict[str, torch.library.Library] = globals().get("_LIBRARIES", {})  # one an operator
+_WRITTEN: dict = globals().get("_WRITTEN", {})  # operator -> positions of the arguments it writes
+_FORMULAS: dict = globals().get("_FORMULAS", {})  # operator -> its setup_context and backward
 
 
 def device_op(schema: str):
@@ -82,9 +83,6 @@ def register_autograd(op, backward, setup_context) -> None:
     ``setup_context(ctx, inputs, output)`` as ``torch.library.register_autograd``
     takes them (a list output's gradients come one by one, after the others)."""
     _FORMULAS[op] = (setup_context or (lambda ctx, inputs, output: None), backward)
-
-
-_FORMULAS: dict = {}
 
 
 def _autograd(op, name: str, lib) -> None:

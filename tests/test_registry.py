@@ -183,13 +183,15 @@ def test_operator_modules_reload():
     program = """
 import importlib, torch
 from delta_feedback_experiment_amd import _registry, controls, conv, norm_gate, ops, pkda, serve
-for module in (_registry, pkda, controls, conv, norm_gate, ops, serve):
-    importlib.reload(module)
 meta = lambda *s: torch.empty(*s, device="meta", requires_grad=True)
-y, _ = norm_gate.pkda_norm_gate(meta(5, 64), meta(5, 64), meta(64), 1e-6)
-y.sum().backward()
-q, _, _ = serve.pkda_qkv_conv_cached_(meta(2, 1, 96), meta(96, 4), 32, 64, 1e-6, torch.empty(4, 3, 96, device="meta"))
-assert y.shape == (5, 64) and q.shape == (2, 1, 32)
+for modules in ((_registry,), (pkda, controls, conv, norm_gate, ops, serve), (_registry, norm_gate, serve)):
+    for module in modules:
+        importlib.reload(module)
+    y, _ = norm_gate.pkda_norm_gate(meta(5, 64), meta(5, 64), meta(64), 1e-6)
+    y.sum().backward()
+    pool = torch.empty(4, 3, 96, device="meta")
+    q, _, _ = serve.pkda_qkv_conv_cached_(meta(2, 1, 96), meta(96, 4), 32, 64, 1e-6, pool)
+    assert y.shape == (5, 64) and q.shape == (2, 1, 32) and pool._version == 1
 """
     subprocess.run([sys.executable, "-c", program], check=True, cwd=ROOT)
 
